@@ -112,7 +112,6 @@ inline int pair_lu_fast_ppb(int n, int nx, int nr) {
   if (n <= 4 && nx <= 4 && nr <= 4) return kWave / 8;
   if (n <= 8 && nx <= 8 && nr <= 8) return kWave / 16;
   if (n <= 16 && nx <= 8 && nr <= 8) return kWave / 32;
-  if (n <= 32 && nx <= 8 && nr <= 8) return 1;
   return 0;
 }
 template <typename TS, typename TW>
