@@ -15,46 +15,14 @@
 // solution vector, solves, and scatters (x_0, x_N, q, xb) back (the
 // reference's swap of x[0:n] with x[(N-1)n:Nn], cc:1392-1423, is the same
 // gather/scatter written in place).
-#include "bcr_launch.hh"
-#include "bcr_wave.hh"
+#include "bcr_last_body.hh"
 
 namespace bcr {
 
 
 template <typename TW, typename TA>
-__device__ __forceinline__ void assemble_last_body(AssembleArgs<TW, TA> const& a) {
-  const int n = a.n, Nr = a.Nr, Nc = a.Nc, qr = a.qr, qx = a.qx, nr = a.nr, nx = a.nx;
-  const int tid = threadIdx.x, nth = blockDim.x;
-  const size_t rn = size_t(nr) * n;
-  for (int i = tid; i < Nr * Nc; i += nth) {
-    const int r = i % Nr, c = i / Nr;
-    double v = 0;
-    if (r < n) {
-      if (c < n) v = double(a.D0[r + c * n]);
-      else if (c < 2 * n) v = double(a.E0[r + (c - n) * n]);
-      else if (c >= 2 * n + qx) v = double(a.B0[r + (c - 2 * n - qx) * n]);
-    } else if (r < 2 * n + qr) {
-      v = double(a.H[(r - n) + size_t(c) * (n + qr)]);
-    } else {
-      const int rr = r - 2 * n - qr;
-      if (c < n) {
-        v = double(a.C[rr + c * nr]);
-      } else if (c < 2 * n) {
-        const size_t off = size_t(a.N) * rn + rr + (c - n) * nr;
-        v = double(a.C[off]) + double(a.Cpend[off]) + double(a.Cpend[size_t(a.N + 1) * rn + off]);
-      } else if (c < 2 * n + qx) {
-        v = double(a.Cq[rr + (c - 2 * n) * nr]);
-      } else {
-        v = a.Feff[rr + (c - 2 * n - qx) * nr];
-      }
-    }
-    a.Hm[i] = v;
-  }
-}
-
-template <typename TW, typename TA>
 __global__ void __launch_bounds__(256) assemble_last_kernel(AssembleArgs<TW, TA> a) {
-  assemble_last_body<TW, TA>(a);
+  assemble_last_body<TW, TA>(a, blockIdx.x * 256 + threadIdx.x, gridDim.x * 256);
 }
 
 // LU with partial pivoting (dgetf2 order: first max, whole-row swaps,
@@ -270,7 +238,7 @@ __global__ void __launch_bounds__(1024) last_solve_kernel(LastSolveArgs<TX> a) {
 // ---- batched: one workgroup per system ------------------------------------
 template <typename TW, typename TA>
 __global__ void __launch_bounds__(256) assemble_last_batched(const AssembleArgs<TW, TA>* args) {
-  assemble_last_body<TW, TA>(args[blockIdx.x]);
+  assemble_last_body<TW, TA>(args[blockIdx.x], threadIdx.x, blockDim.x);
 }
 
 template <bool IN_LDS>
@@ -285,102 +253,18 @@ __global__ void __launch_bounds__(1024) last_solve_batched(const LastSolveArgs<T
   last_solve_body<TX, A_LDS>(args[blockIdx.x]);
 }
 
-// The LU solve of a square last block for one right-hand side, one
-// wavefront per system: lane l holds rows l + 64 k (k < RPL) of y, the row
-// interchanges are composed into a source row per lane (no serial swaps),
-// and the two substitutions walk the columns of the factors from HBM/L2
-// eight at a time with y[c] broadcast by v_readlane, without a workgroup
-// barrier.  Same arithmetic per element as last_solve_body's LU path.
+// one wavefront per system (see last_solve_lu_wave_body)
 template <typename TX, int RPL>
 __global__ void __launch_bounds__(64) last_solve_lu_wave_batched(const LastSolveArgs<TX>* args) {
   const LastSolveArgs<TX>& a = args[blockIdx.x];
   if (skipped(a.skip)) return;
-  constexpr int CH = 8;
-  const int lane = threadIdx.x;
-  const int n = a.n, Nc = a.Nc, ld = a.Nr;
-  const double* A = a.Hm;
-  const size_t xN = size_t(a.N) * n, xC = size_t(a.N + 1) * n + a.qr;
-  TX* const x = a.x;
-  // the source row of each row after the interchanges c = 0 .. Nc-1
-  // (1-based ipiv), found by undoing them from the last
-  int pos[RPL];
-#pragma unroll
-  for (int k = 0; k < RPL; ++k) pos[k] = lane + 64 * k;
-  for (int c = Nc - 1; c >= 0; --c) {
-    const int pv = a.P[c] - 1;
-#pragma unroll
-    for (int k = 0; k < RPL; ++k) pos[k] = pos[k] == c ? pv : pos[k] == pv ? c : pos[k];
-  }
-  double y[RPL], dinv[RPL];
-#pragma unroll
-  for (int k = 0; k < RPL; ++k) {
-    const int r = lane + 64 * k, s = r < Nc ? pos[k] : 0;
-    const size_t row = s < n ? size_t(s) : s < 2 * n + a.qr ? xN + (s - n) : xC + (s - 2 * n - a.qr);
-    y[k] = r < Nc ? double(x[row]) : 0.0;
-    dinv[k] = r < Nc ? 1.0 / A[r + size_t(r) * ld] : 1.0;
-  }
-  // y <- L^{-1} y (unit lower), column c of L below the diagonal
-#pragma unroll
-  for (int kc = 0; kc < RPL; ++kc) {
-    const int cend = min(64 * kc + 64, Nc);
-    for (int c0 = 64 * kc; c0 < cend; c0 += CH) {
-      double l[CH][RPL];
-#pragma unroll
-      for (int i = 0; i < CH; ++i)
-#pragma unroll
-        for (int k = 0; k < RPL; ++k) {
-          const int c = min(c0 + i, Nc - 1), r = lane + 64 * k;
-          l[i][k] = A[(r < Nc ? r : 0) + size_t(c) * ld];
-        }
-#pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        const int c = c0 + i;
-        if (c < cend) {
-          const double yc = wave::rl(y[kc], c - 64 * kc);
-#pragma unroll
-          for (int k = 0; k < RPL; ++k) {
-            const int r = lane + 64 * k;
-            if (r > c && r < Nc) y[k] -= l[i][k] * yc;
-          }
-        }
-      }
-    }
-  }
-  // y <- U^{-1} y, bottom up: y_c = y_c / u_cc, then the rows above
-#pragma unroll
-  for (int kc = RPL - 1; kc >= 0; --kc) {
-    const int cbeg = 64 * kc;
-    for (int c1 = min(64 * kc + 63, Nc - 1); c1 >= cbeg; c1 -= CH) {
-      double u[CH][RPL];
-#pragma unroll
-      for (int i = 0; i < CH; ++i)
-#pragma unroll
-        for (int k = 0; k < RPL; ++k) {
-          const int c = max(c1 - i, 0), r = lane + 64 * k;
-          u[i][k] = A[(r < Nc ? r : 0) + size_t(c) * ld];
-        }
-#pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        const int c = c1 - i;
-        if (c >= cbeg) {
-          const double xc = wave::rl(y[kc] * dinv[kc], c - 64 * kc);
-#pragma unroll
-          for (int k = 0; k < RPL; ++k) {
-            const int r = lane + 64 * k;
-            y[k] = r < c ? y[k] - u[i][k] * xc : r == c ? xc : y[k];
-          }
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < RPL; ++k) {
-    const int r = lane + 64 * k;
-    if (r < Nc) {
-      const size_t row = r < n ? size_t(r) : r < 2 * n ? xN + (r - n) : size_t(a.N + 1) * n + (r - 2 * n);
-      x[row] = TX(y[k]);
-    }
-  }
+  last_solve_lu_wave_body<TX, RPL>(a, a.x, threadIdx.x);
+}
+
+// one system, one wavefront per right-hand side
+template <typename TX, int RPL>
+__global__ void __launch_bounds__(64) last_solve_lu_wave(LastSolveArgs<TX> a) {
+  last_solve_lu_wave_body<TX, RPL>(a, a.x + size_t(blockIdx.x) * a.ldx, threadIdx.x);
 }
 
 template <typename TW, typename TA>
@@ -389,141 +273,21 @@ hipError_t launch_assemble_last_batched(const AssembleArgs<TW, TA>* args, int ns
   return hipGetLastError();
 }
 
-// The same factorization (Nc <= 64 RPL) by one workgroup of NWV wavefronts
-// per system with the block in registers: wavefront w holds columns
-// [CW w, CW w + CW) of every row (lane l: rows l + 64 k).  Rows stay in
-// their lanes with their current positions tracked (the pivot row takes
-// position c, the row there the pivot's old place); the wavefront owning
-// column c searches it (largest |a|, ties to the smaller position, as
-// lu_last_body's scan) and publishes the multipliers through LDS, and every
-// wavefront applies the rank-1 update to its columns after c.  The rows are
-// stored back in their final positions with the 1-based ipiv, so the result
-// and its arithmetic per element are lu_last_body's.
 template <int RPL, int NWV>
 __global__ void __launch_bounds__(64 * NWV) lu_last_regs_batched(const LastSolveArgs<double>* args,
                                                                  int32_t* const* status) {
-  using V16d = double __attribute__((ext_vector_type(16)));
-  constexpr int CW = 64 * RPL / NWV, CB = CW / 16;   // columns and 16-column blocks per wavefront
-  static_assert(CW * NWV == 64 * RPL && CW % 16 == 0, "the waves cover the columns in 16-column blocks");
-  __shared__ double lbuf[2][64 * RPL];
-  __shared__ int pbuf[2][2];
+  __shared__ LastLuLds<RPL> sm;
   const LastSolveArgs<double>& a = args[blockIdx.x];
-  const int Nc = a.Nc;
-  double* const Hm = const_cast<double*>(a.Hm);
-  int32_t* const ipiv = const_cast<int32_t*>(a.P);
-  int32_t* const st = status[blockIdx.x];
-  const int lane = threadIdx.x & 63;
   const int w = NWV == 1 ? 0 : __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  V16d V[RPL][CB];
-  int pos[RPL];
-#pragma unroll
-  for (int k = 0; k < RPL; ++k) {
-    const int r = lane + 64 * k;
-    pos[k] = r;
-#pragma unroll
-    for (int jj = 0; jj < CW; ++jj) {
-      const int gj = CW * w + jj;
-      V[k][jj / 16][jj % 16] = r < Nc && gj < Nc ? Hm[r + size_t(gj) * Nc] : 0.0;
-    }
-  }
-  // column blocks of 16 (unrolled: the owning wavefront and its block are
-  // compile-time per block), steps inside a block rolled (the column read
-  // through a uniform register index)
-#pragma unroll
-  for (int gb = 0; gb < 4 * RPL; ++gb) {
-    const int o = 16 * gb / CW, lb = (16 * gb % CW) / 16;
-    const int cend = min(16 * gb + 16, Nc);
-    for (int c = 16 * gb; c < cend; ++c) {
-      const int cc = c - 16 * gb;
-      double lk[RPL];
-      int who = 0, ps = 0, P = 0;
-      if (w == o) {
-        double x[RPL];
-        bool cb = false;
-        unsigned hb = 0, lbits = 0;
-        int pb = 0, kb = 0;
-#pragma unroll
-        for (int k = 0; k < RPL; ++k) {
-          x[k] = V[k][lb][cc];
-          unsigned h, l;
-          wave::abs_key(x[k], h, l);
-          if (x[k] != x[k]) h = l = 0;   // a NaN is never preferred
-          const bool cand = pos[k] >= c && lane + 64 * k < Nc;
-          const bool better = cand && (!cb || h > hb || (h == hb && (l > lbits || (l == lbits && pos[k] < pb))));
-          if (better) {
-            cb = true;
-            hb = h;
-            lbits = l;
-            pb = pos[k];
-            kb = k;
-          }
-        }
-        bool zero;
-        who = wave::argmax_pos<true>(cb, hb, lbits, pb, lane, zero);
-        P = __builtin_amdgcn_readlane(pb, who);
-        ps = __builtin_amdgcn_readlane(kb, who);
-        double xs = x[0];
-#pragma unroll
-        for (int k = 1; k < RPL; ++k) xs = kb == k ? x[k] : xs;
-        const double pv = wave::rl(xs, who);
-        if (lane == 0) {
-          if (zero) atomicOr(st, 2);
-          ipiv[c] = P + 1;
-        }
-        const double rinv = pv != 0.0 ? 1.0 / pv : 0.0;
-#pragma unroll
-        for (int k = 0; k < RPL; ++k) {
-          const int np = pos[k] == c ? P : pos[k] == P ? c : pos[k];
-          const bool below = np > c && lane + 64 * k < Nc;
-          const double m = x[k] * rinv;
-          lk[k] = below ? m : 0.0;
-          V[k][lb][cc] = below ? m : x[k];
-          if constexpr (NWV > 1) lbuf[c & 1][lane + 64 * k] = lk[k];
-        }
-        if (NWV > 1 && lane == 0) {
-          pbuf[c & 1][0] = who | (ps << 8);
-          pbuf[c & 1][1] = P;
-        }
-      }
-      if constexpr (NWV > 1) {
-        __syncthreads();
-        if (w != o) {
-          const int q = __builtin_amdgcn_readfirstlane(pbuf[c & 1][0]);
-          who = q & 255;
-          ps = q >> 8;
-          P = __builtin_amdgcn_readfirstlane(pbuf[c & 1][1]);
-#pragma unroll
-          for (int k = 0; k < RPL; ++k) lk[k] = lbuf[c & 1][lane + 64 * k];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < RPL; ++k) pos[k] = pos[k] == c ? P : pos[k] == P ? c : pos[k];
-      // this wavefront's columns after c: A[r][j] -= l_r * A[c][j]
-      if (CW * w + CW - 1 > c) {
-#pragma unroll
-        for (int jj = 0; jj < CW; ++jj) {
-          if (CW * w + jj > c) {
-            double v = V[0][jj / 16][jj % 16];
-#pragma unroll
-            for (int k = 1; k < RPL; ++k) v = ps == k ? V[k][jj / 16][jj % 16] : v;
-            const double u = wave::rl(v, who);
-#pragma unroll
-            for (int k = 0; k < RPL; ++k) V[k][jj / 16][jj % 16] -= lk[k] * u;
-          }
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < RPL; ++k) {
-    if (lane + 64 * k < Nc) {
-#pragma unroll
-      for (int jj = 0; jj < CW; ++jj) {
-        const int gj = CW * w + jj;
-        if (gj < Nc) Hm[pos[k] + size_t(gj) * Nc] = V[k][jj / 16][jj % 16];
-      }
-    }
-  }
+  lu_last_regs_body<RPL, NWV, (RPL < 3)>(const_cast<double*>(a.Hm), a.Nc, const_cast<int32_t*>(a.P), status[blockIdx.x], w,
+                              threadIdx.x & 63, sm);
+}
+
+template <int RPL, int NWV>
+__global__ void __launch_bounds__(64 * NWV) lu_last_regs(double* Hm, int Nc, int32_t* ipiv, int32_t* status) {
+  __shared__ LastLuLds<RPL> sm;
+  lu_last_regs_body<RPL, NWV, false>(Hm, Nc, ipiv, status, __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)),
+                              threadIdx.x & 63, sm);
 }
 
 // args[s].Hm / .P (ipiv) / .Nc describe the square last block of system s;
@@ -532,6 +296,10 @@ hipError_t launch_lu_last_batched(const LastSolveArgs<double>* args, int32_t* co
                                   size_t lds_limit, hipStream_t st) {
   if (Ncmax <= 64) {
     hipLaunchKernelGGL((lu_last_regs_batched<1, 1>), dim3(nsys), dim3(64), 0, st, args, status);
+    return hipGetLastError();
+  }
+  if (Ncmax > 128 && Ncmax <= 192) {
+    hipLaunchKernelGGL((lu_last_regs_batched<3, 12>), dim3(nsys), dim3(768), 0, st, args, status);
     return hipGetLastError();
   }
   if (Ncmax <= 128) {
@@ -581,11 +349,18 @@ template bool launch_last_solve_lu_wave_batched<double>(const LastSolveArgs<doub
 
 template <typename TW, typename TA>
 hipError_t launch_assemble_last(AssembleArgs<TW, TA> const& a, hipStream_t st) {
-  hipLaunchKernelGGL((assemble_last_kernel<TW, TA>), dim3(1), dim3(256), 0, st, a);
+  const int blocks = (a.Nr * a.Nc + 255) / 256;   // one element per thread
+  hipLaunchKernelGGL((assemble_last_kernel<TW, TA>), dim3(blocks < 1 ? 1 : blocks), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
 hipError_t launch_lu_last(double* Hm, int Nc, int32_t* ipiv, int32_t* status, size_t lds_limit, hipStream_t st) {
+  if (Nc <= 192) {   // in registers, 16 columns per wavefront
+    if (Nc <= 64) hipLaunchKernelGGL((lu_last_regs<1, 4>), dim3(1), dim3(256), 0, st, Hm, Nc, ipiv, status);
+    else if (Nc <= 128) hipLaunchKernelGGL((lu_last_regs<2, 8>), dim3(1), dim3(512), 0, st, Hm, Nc, ipiv, status);
+    else hipLaunchKernelGGL((lu_last_regs<3, 12>), dim3(1), dim3(768), 0, st, Hm, Nc, ipiv, status);
+    return hipGetLastError();
+  }
   const size_t bytes = size_t(Nc) * Nc * sizeof(double);
   if (bytes <= lds_limit)
     hipLaunchKernelGGL((lu_last_kernel<true>), dim3(1), dim3(1024), bytes, st, Hm, Nc, ipiv, status);
@@ -596,6 +371,13 @@ hipError_t launch_lu_last(double* Hm, int Nc, int32_t* ipiv, int32_t* status, si
 
 template <typename TX>
 hipError_t launch_last_solve(LastSolveArgs<TX> const& a, size_t lds_limit, hipStream_t st) {
+  // LU, square, no second solver behind it: one wavefront per right-hand side
+  if (a.method == kLastLU && a.status == nullptr && a.Nr == a.Nc && a.Nc <= 256) {
+    if (a.Nc <= 64) hipLaunchKernelGGL((last_solve_lu_wave<TX, 1>), dim3(a.nrhs), dim3(64), 0, st, a);
+    else if (a.Nc <= 128) hipLaunchKernelGGL((last_solve_lu_wave<TX, 2>), dim3(a.nrhs), dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((last_solve_lu_wave<TX, 4>), dim3(a.nrhs), dim3(64), 0, st, a);
+    return hipGetLastError();
+  }
   const int R = a.Nr > a.Nc ? a.Nr : a.Nc;
   const size_t xbytes = (size_t(R) + a.Nc) * 16 * sizeof(double);
   const size_t bytes = size_t(a.Nr) * a.Nc * sizeof(double) + xbytes;
