@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "bcr_launch.hh"
+#include "bcr_small.hh"
 
 namespace bcr {
 
@@ -259,10 +260,7 @@ void Engine<TA, TW>::build_schedule() {
       l.L = L; l.npairs = (N + L - 1) / (2 * L); l.slot = lg & 1; l.first = L == 1;
       sched_.push_back(l);
     }
-    // blocks the first level does not touch: row N-1 when N is odd, C_N
-    if (N > 1 && N % 2 == 1) { copy_rows_.push_back(N - 1); copy_cols_.push_back(N - 1); }
-    copy_cols_.push_back(N);
-    return;
+    return;   // the blocks the first level does not touch: launch_prep_single
   }
   used_P_ = P;
   iblock_.assign(size_t(2 * P), 0);
@@ -409,45 +407,67 @@ void Engine<TA, TW>::factorize_async() {
   // and 16 border rows
   if (n > 64 || nr > 16) throw HipError("factorize: block size n <= 64 and nr <= 16 are supported");
   stats_ = FactorStats{};
-  hip_check(launch_convert<int32_t, int32_t>(nullptr, status_.p, 4, st_), "status");
-  // pending border contributions accumulate per factorization
-  timed(kReduce, [&] { hip_check(launch_convert<TW, TW>(nullptr, Cpend_.p, int64_t(Cpend_.count), st_), "zero pending"); });
-  // rows and border blocks the first launch does not read from A (row N-1
-  // when N is odd and C_N in pure cyclic reduction; the range ends too when
-  // partitioned) go to the working arrays as they are
-  for (int r : copy_rows_) {
-    const size_t k = size_t(r);
-    hip_check(launch_convert<TA, TW>(pD_ + k * nn, wD_.p + k * nn, int64_t(nn), st_), "copy D");
-    hip_check(launch_convert<TA, TW>(pE_ + k * nn, wE_.p + k * nn, int64_t(nn), st_), "copy E");
-    hip_check(launch_convert<TA, TW>(pB_ + k * bn, wB_.p + k * bn, int64_t(bn), st_), "copy B");
-  }
-  for (int c : copy_cols_) {
-    const size_t k = size_t(c);
-    hip_check(launch_convert<TA, TW>(pC_ + k * rn, wC_.p + k * rn, int64_t(rn), st_), "copy C");
+  AssembleArgs<TW, TA> as{};
+  as.N = N; as.n = n; as.qr = d_.qr; as.qx = d_.qx; as.nr = nr; as.nx = nx; as.Nr = d_.Nr(); as.Nc = d_.Nc();
+  as.D0 = wD_.p; as.E0 = wE_.p; as.B0 = wB_.p; as.C = wC_.p; as.Cpend = Cpend_.p;
+  as.H = pH_; as.Cq = pCq_; as.Feff = Feff_.p; as.Hm = Hm_.p;
+  const bool pure = used_P_ == 1;   // pure cyclic reduction
+  SingleArgs<TA, TW> sa{};
+  sa.f.N = N; sa.f.n = n; sa.f.nr = nr; sa.f.nx = nx;
+  sa.f.D = wD_.p; sa.f.E = wE_.p; sa.f.B = wB_.p; sa.f.C = wC_.p;
+  sa.f.sD = wD_.p; sa.f.sE = wE_.p; sa.f.sB = wB_.p; sa.f.sC = wC_.p;
+  sa.f.Tm = Tm_.p; sa.f.perm = perm_.p; sa.f.Cpend = Cpend_.p; sa.f.Fpart = Fpart_.p; sa.f.status = status_.p;
+  sa.pD = pD_; sa.pE = pE_; sa.pB = pB_; sa.pC = pC_; sa.pF = pF_;
+  sa.npend = 2 * (int64_t(N) + 1) * nr * n;
+  sa.as = as; sa.Feff = Feff_.p; sa.ipiv = ipiv_.p;
+  // the levels from Ls on in one workgroup (bcr_small.hip), the last block
+  // with them; separate launches while every phase is timed
+  const bool small = pure && method_ == kLU && pair_variant_ == 0 && !timing_ && n <= 16 && nx <= 8 && nr <= 8;
+  const int Ls = small ? small_factor_level(N, n, sizeof(TW), sizeof(TA) == sizeof(TW)) : N;
+  const bool small_asm = small && int64_t(N - 1) * nr * nx <= kSmallSum;
+  const bool small_last = small_asm && last_method_ == kLastLU && !last2_ && d_.Nc() <= 64;
+  sa.L0 = Ls;
+  sa.last = small_last ? kSmallAssemble | kSmallFactor : small_asm ? kSmallAssemble : 0;
+  sa.prep = small && Ls == 1 && (Ls < N || small_asm) ? 1 : 0;
+  if (pure) {
+    if (!sa.prep) timed(kReduce, [&] { hip_check(launch_prep_single(sa, st_), "factorize start"); });
+  } else {
+    hip_check(launch_convert<int32_t, int32_t>(nullptr, status_.p, 4, st_), "status");
+    // pending border contributions accumulate per factorization
+    timed(kReduce, [&] { hip_check(launch_convert<TW, TW>(nullptr, Cpend_.p, int64_t(Cpend_.count), st_), "zero pending"); });
+    // rows and border blocks the first launch does not read from A (the range
+    // ends too) go to the working arrays as they are
+    for (int r : copy_rows_) {
+      const size_t k = size_t(r);
+      hip_check(launch_convert<TA, TW>(pD_ + k * nn, wD_.p + k * nn, int64_t(nn), st_), "copy D");
+      hip_check(launch_convert<TA, TW>(pE_ + k * nn, wE_.p + k * nn, int64_t(nn), st_), "copy E");
+      hip_check(launch_convert<TA, TW>(pB_ + k * bn, wB_.p + k * bn, int64_t(bn), st_), "copy B");
+    }
+    for (int c : copy_cols_) {
+      const size_t k = size_t(c);
+      hip_check(launch_convert<TA, TW>(pC_ + k * rn, wC_.p + k * rn, int64_t(rn), st_), "copy C");
+    }
   }
   for (Level const& l : sched_) {
-    timed(kPair, [&] { level_factor(l); });
+    if (!small || l.L < Ls) timed(kPair, [&] { level_factor(l); });
     ++stats_.levels;
+  }
+  if (small && (Ls < N || small_asm)) {
+    hipError_t e = hipSuccess;
+    if (!launch_small_factor(sa, st_, &e)) throw HipError("factorize: no small-system kernel");
+    hip_check(e, "small factor");
+    stats_.fast_path = 1;
+    if (small_last) return;
   }
   // F_eff = F + sum_j Fpart[j]  (cc:823-829 / 1146-1154)
   const int mF = nr * nx;
-  if (mF > 0)
+  if (mF > 0 && !small_asm)
     timed(kReduce, [&] {
       hip_check(launch_convert<TA, double>(pF_, Feff_.p, mF, st_), "F");
       if (N > 1)
         hip_check(launch_reduce<TW, double>(Fpart_.p, 1, N - 1, mF, tmpw_.p, max_chunks_, Feff_.p, mF, mF, st_),
                   "reduce F");
     });
-  AssembleArgs<TW, TA> as{};
-  as.N = N; as.n = n; as.qr = d_.qr; as.qx = d_.qx; as.nr = nr; as.nx = nx; as.Nr = d_.Nr(); as.Nc = d_.Nc();
-  as.D0 = wD_.p; as.E0 = wE_.p; as.B0 = wB_.p; as.C = wC_.p; as.Cpend = Cpend_.p;
-  as.H = pH_; as.Cq = pCq_; as.Feff = Feff_.p; as.Hm = Hm_.p;
-  if (N == 1) {  // no reduction level: row 0 and C_0 come straight from A
-    hip_check(launch_convert<TA, TW>(pD_, wD_.p, int64_t(nn), st_), "copy D0");
-    hip_check(launch_convert<TA, TW>(pE_, wE_.p, int64_t(nn), st_), "copy E0");
-    hip_check(launch_convert<TA, TW>(pB_, wB_.p, int64_t(bn), st_), "copy B0");
-    hip_check(launch_convert<TA, TW>(pC_, wC_.p, int64_t(rn), st_), "copy C0");
-  }
   const bool svd_first = last_method_ >= kLastSVD;
   if (svd_first || last2_) {
     const int k = std::min(d_.Nr(), d_.Nc()), rows = std::max(d_.Nr(), d_.Nc());
@@ -463,7 +483,7 @@ void Engine<TA, TW>::factorize_async() {
   sv.Nr = d_.Nr(); sv.Nc = d_.Nc(); sv.W = svdW_.p; sv.Vj = svdVj_.p; sv.U = svdU_.p; sv.V = svdV_.p;
   sv.S = svdS_.p; sv.rank = svd_rank_.p; sv.status = status_.p;
   timed(kLast, [&] {
-    hip_check(launch_assemble_last(as, st_), "assemble last");
+    if (!small_asm) hip_check(launch_assemble_last(as, st_), "assemble last");
     if (svd_first) {
       sv.A = Hm_.p;
       sv.conditional = 0;
@@ -521,7 +541,30 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
     tmp = reinterpret_cast<TX*>(tmpw_.p);
   }
   a.Xpart = Xpart;
+  LastSolveArgs<TX> ls{};
+  ls.N = N; ls.n = n; ls.qr = d_.qr; ls.qx = d_.qx; ls.nr = nr; ls.nx = d_.nx; ls.Nr = d_.Nr(); ls.Nc = d_.Nc();
+  ls.method = std::min(last_method_, int(kLastSVD)); ls.nrhs = nrhs; ls.Hm = Hm_.p; ls.P = ipiv_.p;
+  ls.Q = jpiv_.p; ls.tau = tau_.p; ls.x = x; ls.ldx = ldx;
+  ls.status = last2_ ? status_.p : nullptr;
+  ls.U = svdU_.p; ls.V = svdV_.p; ls.S = svdS_.p; ls.rank = svd_rank_.p;
+  // the levels from Ls on in one workgroup (bcr_small.hip), with the xb sum
+  // and the last solve between its two sweeps where they fit one too
+  const bool small = used_P_ == 1 && method_ == kLU && sweep_fast_ && !timing_ && n <= 16;
+  const int Ls = small ? small_solve_level(N, n) : N;
+  SmallSolveArgs<TW, TX> ss{};
+  ss.s = a;
+  ss.L0 = Ls;
+  ss.last = ls;
+  const bool small_xb = small && m <= 512 && int64_t(N - 1) * int64_t(m) <= kSmallSum;
+  const bool small_last = small_xb && ls.method == kLastLU && !last2_ && ls.Nr == ls.Nc && ls.Nc <= 64;
+  auto run_small = [&](int phases) {
+    ss.phases = phases;
+    hipError_t e = hipSuccess;
+    if (!launch_small_solve(ss, st_, &e)) throw HipError("solve: no small-system kernel");
+    hip_check(e, "small solve");
+  };
   for (Level const& l : sched_) {
+    if (small && l.L >= Ls) break;
     a.L = l.L;
     a.npairs = l.npairs;
     a.pairs = l.off >= 0 ? pairtab_.p + l.off : nullptr;
@@ -533,22 +576,21 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
       else hip_check(launch_forward(method_, a, st_), "forward");
     });
   }
-  if (N > 1 && m > 0)
+  if (small_last) run_small(kSmallFwd | kSmallXb | kSmallLast | kSmallBwd);
+  else if (small && Ls < N) run_small(kSmallFwd | (small_xb ? kSmallXb : 0));
+  const bool xb_done = small_last || (small_xb && Ls < N);
+  if (!xb_done && N > 1 && m > 0)
     timed(kReduce, [&] {
       hip_check(launch_reduce<TX, TX>(Xpart, 1, N - 1, int(m), tmp, max_chunks_, x + size_t(N + 1) * n + d_.qr, nr,
                                       ldx, st_),
                 "reduce xb");
     });
-  timed(kLast, [&] {
-    LastSolveArgs<TX> ls{};
-    ls.N = N; ls.n = n; ls.qr = d_.qr; ls.qx = d_.qx; ls.nr = nr; ls.nx = d_.nx; ls.Nr = d_.Nr(); ls.Nc = d_.Nc();
-    ls.method = std::min(last_method_, int(kLastSVD)); ls.nrhs = nrhs; ls.Hm = Hm_.p; ls.P = ipiv_.p;
-    ls.Q = jpiv_.p; ls.tau = tau_.p; ls.x = x; ls.ldx = ldx;
-    ls.status = last2_ ? status_.p : nullptr;
-    ls.U = svdU_.p; ls.V = svdV_.p; ls.S = svdS_.p; ls.rank = svd_rank_.p;
-    hip_check(launch_last_solve<TX>(ls, lds_limit_, st_), "last solve");
-  });
+  if (!small_last) {
+    timed(kLast, [&] { hip_check(launch_last_solve<TX>(ls, lds_limit_, st_), "last solve"); });
+    if (small && Ls < N) run_small(kSmallBwd);
+  }
   for (auto it = sched_.rbegin(); it != sched_.rend(); ++it) {
+    if (small && it->L >= Ls) continue;
     a.L = it->L;
     a.npairs = it->npairs;
     a.pairs = it->off >= 0 ? pairtab_.p + it->off : nullptr;
