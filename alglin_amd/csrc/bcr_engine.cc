@@ -17,6 +17,23 @@ template <typename TS, typename TW>
 bool launch_mfma(FactorArgs<TS, TW> const& a, hipStream_t st, hipError_t* e) {
   return launch_pair_lu_mfma(a, st, e);
 }
+
+// Several right-hand sides: whether a level's sweep goes through the matrix
+// cores (bcr_sweep_mfma.hip), one wave per pair and 16 columns whatever their
+// number.  Solve times, this against the other sweeps (FP64, one MI355X):
+//   n <= 8     several pairs share a wave elsewhere: only for levels of few
+//              pairs (n = 8: N = 31250, 16 columns 318 / 586 us; N = 468750,
+//              2 columns 1621 / 938 us)
+//   n <= 32    always (n = 32, N = 29296: 2 columns 570 / 789, 16 columns
+//              749 / 2001 us; n = 10, N = 300000: 2 columns 1161 / 1243 us)
+//   n > 32     from five columns on (n = 48, N = 13020: 4 columns 1198 / 888,
+//              6 columns 1211 / 1400 us), below that at levels of few pairs
+//              (N = 43: 2 columns 222 / 263 us; N = 868: 500 / 439 us)
+bool sweep_mfma(int n, int nrhs, int npairs) {
+  if (n <= 8) return nrhs > 4 && npairs <= 4096;
+  if (n <= 32) return nrhs >= 2;
+  return nrhs > 4 || (nrhs >= 2 && npairs <= 64);
+}
 }  // namespace
 
 void hip_check(hipError_t e, char const* what) {
@@ -549,7 +566,7 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
   ls.U = svdU_.p; ls.V = svdV_.p; ls.S = svdS_.p; ls.rank = svd_rank_.p;
   // the levels from Ls on in one workgroup (bcr_small.hip), with the xb sum
   // and the last solve between its two sweeps where they fit one too
-  const bool small = used_P_ == 1 && method_ == kLU && sweep_fast_ && !timing_ && n <= 16;
+  const bool small = used_P_ == 1 && method_ == kLU && sweep_fast_ && !timing_ && n <= 16 && nrhs <= 4;
   const int Ls = small ? small_solve_level(N, n) : N;
   SmallSolveArgs<TW, TX> ss{};
   ss.s = a;
@@ -571,7 +588,7 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
     timed(kForward, [&] {
       hipError_t e = hipSuccess;
       if (method_ == kLU && sweep_fast_ &&
-          (launch_sweep_lu_fast(true, a, st_, &e) || launch_sweep_lu_stream(true, a, st_, &e)))
+          ((sweep_mfma(n, nrhs, a.npairs) && launch_sweep_lu_mfma(true, a, st_, &e)) || launch_sweep_lu_fast(true, a, st_, &e) || launch_sweep_lu_stream(true, a, st_, &e)))
         hip_check(e, "forward_fast");
       else hip_check(launch_forward(method_, a, st_), "forward");
     });
@@ -600,7 +617,7 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
       // QRP adds the pair's column exchanges (the streamed sweep's exch)
       a.exch = method_ == kQRP ? 1 : 0;
       if ((method_ == kLU || method_ == kQR) && sweep_fast_ &&
-          (launch_sweep_lu_fast(false, a, st_, &e) || launch_sweep_lu_stream(false, a, st_, &e)))
+          ((sweep_mfma(n, nrhs, a.npairs) && launch_sweep_lu_mfma(false, a, st_, &e)) || launch_sweep_lu_fast(false, a, st_, &e) || launch_sweep_lu_stream(false, a, st_, &e)))
         hip_check(e, "backward_fast");
       else if (method_ == kQRP && sweep_fast_ && launch_sweep_lu_stream(false, a, st_, &e))
         hip_check(e, "backward_stream");

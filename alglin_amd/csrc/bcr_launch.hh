@@ -46,6 +46,9 @@ hipError_t launch_backward(int method, SolveArgs<TW, TX> const& a, hipStream_t s
 // streamed LU sweeps, one wavefront per pair (n <= 64)
 template <typename TW, typename TX>
 bool launch_sweep_lu_stream(bool forward, SolveArgs<TW, TX> const& a, hipStream_t st, hipError_t* err);
+// matrix-core LU sweeps, several right-hand sides (n <= 64, nr <= 16)
+template <typename TW, typename TX>
+bool launch_sweep_lu_mfma(bool forward, SolveArgs<TW, TX> const& a, hipStream_t st, hipError_t* err);
 // wave-synchronous LU sweeps (n <= 32); false when the shape is not covered
 template <typename TW, typename TX>
 bool launch_sweep_lu_fast(bool forward, SolveArgs<TW, TX> const& a, hipStream_t st, hipError_t* err);
