@@ -14,8 +14,8 @@
 namespace bcr {
 namespace {
 
-// the matrix-core pair of the 16 < n <= 32 and 32 < n <= 48 LU classes
-// (FP64 factors: n <= 48; FP32 factors also up to 64): the default (variant
+// the matrix-core pair of the 16 < n <= 32 and 32 < n <= 64 LU classes
+// (nr <= 8, nx <= 16): the default (variant
 // 0) and variant 5; variant 4 keeps the rank-1 kernels (two-wave split,
 // column-split)
 template <typename TS, typename TW, typename L>

@@ -12,7 +12,7 @@
 namespace bcr {
 
 namespace {
-// the matrix-core pair (FP32 factors n <= 64, FP64 factors n <= 48)
+// the matrix-core pair (n <= 64)
 template <typename TS, typename TW>
 bool launch_mfma(FactorArgs<TS, TW> const& a, hipStream_t st, hipError_t* e) {
   return launch_pair_lu_mfma(a, st, e);
@@ -372,7 +372,7 @@ void Engine<TA, TW>::level_factor(Level const& l) {
     (void)sizeof(A);
     hipError_t e = hipSuccess;
     // variants: 0 default (16 < n: the matrix-core pair where it applies,
-    // FP32 factors n <= 64, FP64 factors n <= 48; else wave-per-row kernels
+    // n <= 64; else wave-per-row kernels
     // for n <= 32, column-split waves up to n = 64, register tiles beyond), 3
     // register tiles only, 4 column-split waves only, 5 the matrix-core pair
     // where it applies

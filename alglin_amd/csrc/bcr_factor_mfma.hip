@@ -1,43 +1,50 @@
-// Pair elimination, LU, FP32 factors n <= 64 and FP64 factors n <= 48: the getrf + applyT split of
-// the reference pair step (buildT BABD_BorderedCR.cc:856, applyT cc:917-982,
-// the border update cc:1107-1154), with the right-hand columns on the matrix
-// cores.  The augmented panel is the one of bcr_factor_generic.hip: R = 2n +
-// nr rows [row jp; row j; border], columns [T = col j | col jp | col jpp | xb].
-// Two launches per level, so that the latency-bound pivot steps run with
-// many pairs per CU (A needs 2 KB of LDS) and only B holds the LDS a GEMM
-// needs.
+// Pair elimination, LU, n <= 64: the getrf + applyT split of the reference
+// pair step (buildT BABD_BorderedCR.cc:856, applyT cc:917-982, the border
+// update cc:1107-1154), with the right-hand columns on the matrix cores.  The
+// augmented panel is the one of bcr_factor_generic.hip: R = 2n + nr rows
+// [row jp; row j; border], columns [T = col j | col jp | col jpp | xb].
+// Two launches per level, so that the pivot steps of a panel and the products
+// each run with the registers and LDS they need.
 //
-//  A. pair_lu_t: the T panel [E_jp; D_j; C_j] (R x n), one wave per pair,
-//     in registers: rows over lanes (row lane + 64 s, s < 2), columns in
-//     two (n <= 32) or three 16-wide register vectors; LAPACK partial pivoting among the first 2n
-//     rows (first maximum), multiplier a * (1/pivot), fma updates -- the
-//     arithmetic of the other LU kernels, so T, the pivots and C_j U^-1
-//     agree with them bit for bit.  The step loop is rolled within each
-//     16-column block (column c read and written through a uniform register
-//     index; FP32: in groups of four steps, each updating its block's
-//     columns from the group's first on).  Rows do not move; each row is
-//     stored at its final position (T, C_j U^-1, perm), and the positions
-//     themselves go to the unused tail of T (one byte per row).
+//  A. pair_lu_t: the T panel [E_jp; D_j; C_j] (R x n), one wave per pair, in
+//     registers: rows over lanes (row lane + 64 s), columns in 16-wide
+//     register vectors; LAPACK partial pivoting among the first 2n rows (first
+//     maximum), multiplier a * (1/pivot), fma updates -- the arithmetic of the
+//     other LU kernels, so T, the pivots and C_j U^-1 agree with them bit for
+//     bit.  The step loop is rolled within each 16-column block (column c
+//     read and written through a uniform register index, in groups of four
+//     steps that update the block's columns from the group's first on).  In
+//     FP64 the trailing blocks take a block's 16 steps at once on the matrix
+//     cores (trailing_update); in FP32 each step updates them (a lane read
+//     and two FMAs per column: the way through LDS costs as much).  VALU
+//     issue bounds it: N = 100000, n = 32 FP64, first level 909 -> 750 us
+//     with the blocked update (loads and stores alone are 0.4 ms).  Rows do
+//     not move; each row is stored at its final position (T, C_j U^-1, perm),
+//     and the positions themselves go to the unused tail of T (one byte per
+//     row).
 //  B. pair_rhs_mfma: the right-hand part X = [col jp | col jpp | xb], two
-//     waves per pair.  The row positions come from A's bytes; LDS gets
-//     -L11 below its 16 x 16 diagonal blocks, the inverses of those unit
-//     lower blocks on them (forward substitution, one column per lane), and
-//     -[L21; C_j U^-1].  X goes in 16-column tiles, each inside one of the
-//     three column blocks, its sources loaded one tile ahead and staged in
-//     LDS with the rows at their final positions; then
+//     waves per pair, 16-column tiles, each inside one of the three column
+//     blocks.  -L11 below its diagonal blocks, the inverses of those unit
+//     lower blocks (forward substitution in LDS, one column per lane) and
+//     -[L21; C_j U^-1] are A operands held in registers for all tiles of a
+//     wave; a tile is one contiguous run of its source block, loaded one tile
+//     ahead and staged in LDS with the rows at their final positions; then
 //        U12_kb  = inv(L_kk) (X_kb - sum_{m<kb} L_km U12_m)
 //                                           -> pivot rows: D_j', E_j', B_j'
 //        X_rest' = X_rest - [L21; C_j U^-1] U12
 //                                           -> reduced rows D_jp', E_jp', B_jp'
 //     on v_mfma_f32_16x16x4f32 (FP32 factors) or v_mfma_f64_16x16x4f64 (FP64
-//     factors).  The sum over k runs as 16-wide blocks, lane group
-//     g = lane / 16 taking k = 16 kb + kro(g, i) in the i-th MFMA of a block
-//     (kro: the row the result layout puts in value i of group g, 4 g + i in
-//     FP32, g + 4 i in FP64): in FP32 every LDS operand is one 16-byte read
-//     per lane per four MFMAs, and in both a block of U12 in the accumulator
-//     layout is the next products' B operand as it stands.  The border rows
-//     (C_jp', pending C_jpp, F partial) leave through LDS in one coalesced
-//     pass per tile.
+//     factors), the results leaving through the tile's place in LDS as whole
+//     runs.  The sum over k runs as 16-wide blocks, lane group g = lane / 16
+//     taking k = 16 kb + kro(g, i) in the i-th MFMA of a block (kro: the row
+//     the result layout puts in value i of group g, 4 g + i in FP32, g + 4 i
+//     in FP64), so a block of U12 in the accumulator layout is the next
+//     products' B operand as it stands.  Memory latency bounds it, so all
+//     loads of a tile are issued before the stores of the one before (a wait
+//     for loads behind stores waits for those: 1.62 -> 1.27 ms at N = 100000,
+//     n = 32 FP64, first level), the operands live in registers instead of
+//     LDS (more pairs per CU), and stores are whole runs (1.41 ms with
+//     operands in LDS and stores by column; now 0.97 ms, 3.2 TB/s).
 // The right-hand results differ from the rank-1 kernels in rounding only
 // (other summation order, the inverted diagonal blocks).  A pivot whose
 // reciprocal overflows (a subnormal pivot) turns the finished T columns into
@@ -53,47 +60,6 @@ namespace {
 
 // the most border rows (nr) the matrix-core pair takes
 constexpr int kNrB = 8;
-
-// LDS geometry: NT top slots (pivot positions, NMAX a multiple of 16), NR
-// rest slots (reduced and border rows, n + nr <= RESTMAX)
-template <int NMAX, int RESTMAX, int RS>
-struct MfmaGeom {
-  static constexpr int NT = NMAX;
-  static constexpr int NR = (RESTMAX + 15) / 16 * 16;
-  static constexpr int LD = NT + 4;        // row stride of Ls
-  static constexpr int XLD = NT + NR + 4;  // column stride of a staged tile
-  static_assert(NT % 16 == 0, "NMAX must be a multiple of 16");
-  static_assert(NT + NR <= 64 * RS, "padding slots come from the lanes beyond row R");
-};
-
-// rows 16 kb + kro(g, i) (i < 4) of one column, those below lim: for FP32 one
-// 16-byte store when the 16-row block lies below lim (a uniform test),
-// single stores in the block lim cuts
-template <typename T>
-__device__ __forceinline__ void store_block(T* col, int kb, int g, V4<T> v, int lim) {
-  if constexpr (sizeof(T) == 4) {
-    const int r0 = 16 * kb + 4 * g;
-    if (16 * kb + 16 <= lim) {
-      __builtin_memcpy(col + r0, &v, 4 * sizeof(T));   // element-aligned; the hardware takes it
-    } else if (16 * kb < lim) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (r0 + i < lim) col[r0 + i] = v[i];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 16 * kb + kro<T>(g, i);
-      if (r < lim) col[r] = v[i];
-    }
-  }
-}
-
-// v when the mask is all ones, +0 when it is zero
-__device__ __forceinline__ float mask_bits(float v, int m) { return __int_as_float(__float_as_int(v) & m); }
-__device__ __forceinline__ double mask_bits(double v, int m) {
-  return __longlong_as_double(__double_as_longlong(v) & static_cast<long long>(m));
-}
 
 // lane `who`'s value of v when K > cc, else 0: a scalar select on the
 // v_readlane result (written out: the compiler would move the value to a
@@ -140,79 +106,136 @@ __device__ __forceinline__ void update_after(V16<TW>& v0, V16<TW>& v1, V16<TW>& 
   }
 }
 
-// X_rest' = X_rest - [L21; C_j U^-1] U12 over the first NRT 16-row tiles of
-// the rest rows (the minus sign is in Ls); the tiles' independent
-// accumulators alternate on the matrix core.  Reduced rows go to drest,
-// border rows back to their staging slots.
-template <int NB, int NRT, int NT, int LD, int XLD, typename TW>
-__device__ __forceinline__ void rest_tiles(const V4<TW> (&u)[NB], const TW* Ls, TW* xt, int cl, int g, int n, int nr,
-                                           bool colok, TW* drest) {
-  V4<TW> acc[NRT];
-#pragma unroll
-  for (int rt = 0; rt < NRT; ++rt) acc[rt] = ld4(xt + cl * XLD + NT + rt * 16, g);
-#pragma unroll
-  for (int kb = 0; kb < NB; ++kb) {
-    V4<TW> av[NRT];
-#pragma unroll
-    for (int rt = 0; rt < NRT; ++rt)
-      av[rt] = ld4(Ls + (NT + rt * 16 + cl) * LD + kb * 16, g);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int rt = 0; rt < NRT; ++rt) acc[rt] = mfma1(av[rt][i], u[kb][i], acc[rt]);
-  }
-  // rest position q = 16 rt + kro(g, i): reduced row q (< n), else border row q - n
-  if (colok) {
-#pragma unroll
-    for (int rt = 0; rt < NRT; ++rt) store_block(drest, rt, g, acc[rt], n);
-  }
-#pragma unroll
-  for (int rt = 0; rt < NRT; ++rt)
-    if (16 * rt + 16 > n && 16 * rt < n + nr) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int q = rt * 16 + kro<TW>(g, i);
-        if (q >= n && q < n + nr) xt[cl * XLD + NT + q] = acc[rt][i];
-      }
-    }
-}
+// ---- A: the T panel, one wave per pair ------------------------------------------
+// Between the 16-column blocks the trailing columns take the block's 16 steps
+// at once, on the matrix cores, through LDS (one 16-column buffer):
+//   x   the block's multipliers by row (zero for a row from the step on at
+//       which it became a pivot row), read as A operands; then each trailing
+//       block by row (as the registers hold it) and by tile in turn
+//   u   the pivot rows' entries of all trailing columns, solved in place with
+//       the block's unit lower triangle lk, a column per lane
+// v_mfma_*_16x16x4 forms c + a0 b0 + .. + a3 b3 as the chain of fused
+// multiply-adds in that order (measured: equal to it in every bit), and the
+// products run over k upwards, so every entry sees the operations of the
+// rank-1 steps in their order.
+constexpr bool panel_blocked(size_t elem) { return elem == 8; }
 
-// A panel row of the right-hand part: its class (1: a row of block jp, 2: a
-// row of block j, 4: a border row, 0: none) and its row in that block.
-struct RowSrc {
-  int cls, off;
+template <typename TW, int NB>
+struct PanelLds {
+  static constexpr int TILES = (2 * 16 * NB + kNrB + 15) / 16;
+  // column stride: 16 columns' reads of neighbouring rows on different banks
+  static constexpr int RLD = 16 * TILES + 2, ULD = 16 * (NB > 1 ? NB - 1 : 1) + 2;
+  alignas(16) TW x[16 * RLD];
+  alignas(16) TW u[16 * ULD];
+  alignas(16) TW lk[16 * 16];
 };
 
-// the raw source values of one row in right-hand tile t (16 columns of the
-// tile's region; clamped addresses, masked when staged)
-// (the source blocks come as values read from the argument record before
-// the kernel's first store: a batched kernel's record sits in memory, and a
-// field read after a store is fetched again, behind it)
-template <typename TS>
-__device__ __forceinline__ void load_rhs_row(TS (&xs)[16], const TS* sD, const TS* sE, const TS* sB, const TS* sC,
-                                             int n, int nr, int nx, int t, int tA, int j, int jp, RowSrc rs) {
-  const size_t nn = size_t(n) * n, rn = size_t(nr) * n, bn = size_t(n) * nx;
-  const int reg = t < tA ? 0 : t < 2 * tA ? 1 : 2;
-  const int c0 = 16 * (reg == 0 ? t : reg == 1 ? t - tA : t - 2 * tA);
-  const int width = reg == 2 ? nx : n;
-  // region 0: [D_jp | . | C_jp]; region 1: [. | E_j | .]; region 2: [B_jp | B_j | .]
-  const bool valid = reg == 0 ? (rs.cls & 5) != 0 : reg == 1 ? rs.cls == 2 : (rs.cls & 3) != 0;
-  const TS* src = reg == 0 ? (rs.cls == 4 ? sC + jp * rn : sD + jp * nn)
-                : reg == 1 ? sE + j * nn
-                           : sB + (rs.cls == 1 ? jp : j) * bn;
-  src = valid ? src + rs.off : sD + jp * nn;   // a valid address for the rows of zeros
-  const int stride = reg == 0 && rs.cls == 4 ? nr : n;
+// the LDS accesses of a wave are in order; this keeps the compiler's so
+__device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+template <int B, int NB, int RS, typename TW>
+__device__ __forceinline__ void trailing_update(V16<TW> (&V)[RS][NB], PanelLds<TW, NB>& sm, int pos0, int pos1, int n,
+                                                int R, int lane) {
+  constexpr int TILES = PanelLds<TW, NB>::TILES, RLD = PanelLds<TW, NB>::RLD, ULD = PanelLds<TW, NB>::ULD;
+  const int g = lane >> 4, cl = lane & 15;
+  // multipliers by row; the block's pivot rows to u and lk
 #pragma unroll
-  for (int cc = 0; cc < 16; ++cc) xs[cc] = src[(c0 + cc < width ? c0 + cc : width - 1) * stride];
+  for (int s = 0; s < RS; ++s) {
+    const int r = lane + 64 * s;
+    const int p = s == 0 ? pos0 - 16 * B : s == 1 ? pos1 - 16 * B : 16;   // (border rows: no pivots)
+    if (r < 16 * TILES) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) sm.x[k * RLD + r] = keep_if(V[s][B][k], k < p);
+    }
+    if (s < 2 && p >= 0 && p < 16) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) sm.lk[k * 16 + p] = V[s][B][k];
+#pragma unroll
+      for (int bb = B + 1; bb < NB; ++bb)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) sm.u[p * ULD + 16 * (bb - B - 1) + k] = V[s][bb][k];
+    }
+  }
+  lds_order();
+  if (lane < 16 * (NB - 1 - B)) {
+    TW y[16];
+#pragma unroll
+    for (int p = 0; p < 16; ++p) y[p] = sm.u[p * ULD + lane];
+#pragma unroll
+    for (int k = 0; k < 15; ++k) {
+#pragma unroll
+      for (int p = k + 1; p < 16; ++p) y[p] = fma(-sm.lk[k * 16 + p], y[k], y[p]);
+      __builtin_amdgcn_sched_barrier(0);   // (the reads of all columns at once would take every register)
+    }
+#pragma unroll
+    for (int p = 1; p < 16; ++p) sm.u[p * ULD + lane] = y[p];
+  }
+  lds_order();
+  // GS row sets at a time (all, or one where the registers hold no more):
+  // their multipliers to registers, then their rows of each trailing block
+  // through the place they leave
+  constexpr int GS = NB >= 3 ? 1 : RS, GT = 4 * GS < TILES ? 4 * GS : TILES;
+#pragma unroll
+  for (int s0 = 0; s0 < RS; s0 += GS) {
+    V4<TW> av[GT];
+#pragma unroll
+    for (int t = 0; t < GT; ++t)
+      if (4 * s0 + t < TILES) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) av[t][i] = -sm.x[(g + 4 * i) * RLD + 64 * s0 + 16 * t + cl];
+      }
+    lds_order();
+#pragma unroll
+    for (int bb = B + 1; bb < NB; ++bb)
+      if (16 * bb < n && 64 * s0 < R) {
+#pragma unroll
+        for (int s = s0; s < s0 + GS; ++s) {
+          const int r = lane + 64 * s;
+          if (r < 16 * TILES) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) sm.x[k * RLD + r] = V[s][bb][k];
+          }
+        }
+        lds_order();
+        V4<TW> u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u[i] = sm.u[(g + 4 * i) * ULD + 16 * (bb - B - 1) + cl];
+#pragma unroll
+        for (int t = 0; t < GT; ++t)
+          if (4 * s0 + t < TILES && 64 * s0 + 16 * t < R) {
+            TW* const blk = sm.x + cl * RLD + 64 * s0 + 16 * t;
+            V4<TW> acc;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = blk[kro<TW>(g, i)];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc = mfma1(av[t][i], u[i], acc);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) blk[kro<TW>(g, i)] = acc[i];
+          }
+        lds_order();
+#pragma unroll
+        for (int s = s0; s < s0 + GS; ++s) {
+          const int rr = min(lane + 64 * s, 16 * TILES - 1);
+#pragma unroll
+          for (int k = 0; k < 16; ++k) V[s][bb][k] = sm.x[k * RLD + rr];
+        }
+        lds_order();
+      }
+  }
 }
 
-// ---- A: the T panel, one wave per pair ------------------------------------------
 template <typename TS, typename TW, int NB, int RS, int NRMAX>
 __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int p) {
   constexpr int NMAX = 16 * NB;
   static_assert(RS == 2 || RS == 3, "two or three row sets");
   static_assert(NMAX <= 64, "the 2n candidate rows lie in row sets 0 and 1");
-  __shared__ __align__(16) TW stage[(NRMAX + 1) * NMAX];   // border rows C_j, one zero row
+  constexpr bool BLOCKED = panel_blocked(sizeof(TW));
+  // first: border rows C_j and one zero row, NMAX values each
+  constexpr int STAGE = (NRMAX + 1) * NMAX * int(sizeof(TW));
+  using Lds = std::conditional_t<BLOCKED, PanelLds<TW, NB>, char[STAGE]>;
+  static_assert(STAGE <= int(sizeof(Lds)), "the border rows fit the buffer");
+  __shared__ __align__(16) Lds sm;
+  TW* const stage = reinterpret_cast<TW*>(&sm);
   if (p >= a.npairs) return;
   const int lane = threadIdx.x & 63;
   const int n = a.n, nr = a.nr, n2 = 2 * n;
@@ -271,10 +294,9 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
   // (s_set_gpr_idx) and updates the columns of blocks b.. with the pivot
   // row's entries; group g of block b updates its block's columns from
   // GS g + 1 on, those that may not lie after c getting a zero entry.  Each
-  // group's loop stays rolled (one copy of a step per group).  FP32: four
-  // groups (a quarter of the masked in-block updates); FP64: one (the
-  // copies would cost the FP64 panel a wave per SIMD).
-  constexpr int GR = sizeof(TW) == 4 ? 4 : 1, GS = 16 / GR;
+  // group's loop stays rolled (one copy of a step per group; four groups: a
+  // quarter of the masked in-block updates of one).
+  constexpr int GR = 4, GS = 16 / GR;
   // step c of block b; the block's columns from KS on are updated, those
   // before KM masked
   auto step = [&](const int b, const int c, auto KS, auto KM) {
@@ -317,31 +339,62 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
     // columns KS .. 15 of the block (those before are never after c)
     update_after<decltype(KS)::value, decltype(KM)::value, RS, TW>(V[0][b], V[1][b], V[RS - 1][b], sp, who, cc, lv0,
                                                                    lv1, lv2);
+    if constexpr (!BLOCKED) {
 #pragma unroll
-    for (int bb = b + 1; bb < NB; ++bb)
+      for (int bb = b + 1; bb < NB; ++bb)
 #pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const TW u = wave::rl(sp ? V[1][bb][k] : V[0][bb][k], who);
-        V[0][bb][k] = fma(-lv0, u, V[0][bb][k]);
-        V[1][bb][k] = fma(-lv1, u, V[1][bb][k]);
-        if constexpr (RS > 2) V[RS - 1][bb][k] = fma(-lv2, u, V[RS - 1][bb][k]);
-      }
-  };
-  if constexpr (GR == 1) {
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int cend = min(16 * b + 16, n);
-      for (int c = 16 * b; c < cend; ++c) step(b, c, std::integral_constant<int, 1>{}, std::integral_constant<int, 16>{});
+        for (int k = 0; k < 16; ++k) {
+          const TW u = wave::rl(sp ? V[1][bb][k] : V[0][bb][k], who);
+          V[0][bb][k] = fma(-lv0, u, V[0][bb][k]);
+          V[1][bb][k] = fma(-lv1, u, V[1][bb][k]);
+          if constexpr (RS > 2) V[RS - 1][bb][k] = fma(-lv2, u, V[RS - 1][bb][k]);
+        }
     }
-  } else {
-    static_for<0, GR * NB>([&](auto BG) {
-      constexpr int b = decltype(BG)::value / GR, g = decltype(BG)::value % GR;
+  };
+  static_for<0, NB>([&](auto BK) {
+    constexpr int b = decltype(BK)::value;
+    static_for<0, GR>([&](auto G) {
+      constexpr int g = decltype(G)::value;
       const int cend = min(16 * b + GS * g + GS, n);
       for (int c = 16 * b + GS * g; c < cend; ++c)
         step(b, c, std::integral_constant<int, GS * g + 1>{}, std::integral_constant<int, GS * g + GS>{});
     });
-  }
+    if constexpr (BLOCKED && b + 1 < NB) {
+      if (16 * (b + 1) < n) trailing_update<b, NB, RS, TW>(V, sm, pos0, pos1, n, R, lane);
+    }
+  });
   if (zero_pivot && lane == 0) atomicOr(a.status, 1);
+  // the selector's statistics of this panel (FP32 batches): |U_cc| min and
+  // max, |U_rc| max over r <= c, as float bits (non-negative: ordered as
+  // unsigned); the row at final position p < n holds U row p
+  if (sizeof(TW) == 4 && a.pstat != nullptr) {
+    unsigned dmin = 0xffffffffu, dmax = 0u, umax = 0u;
+#pragma unroll
+    for (int s = 0; s < (ONE ? 1 : 2); ++s) {
+      const int q = lane + 64 * s < n2 ? (s == 0 ? pos0 : pos1) : n;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+          const int c = 16 * b + k;
+          const unsigned bits = __float_as_uint(fabsf(float(V[s][b][k])));
+          umax = max(umax, q <= c && c < n ? bits : 0u);
+          if (q == c && c < n) {
+            dmin = min(dmin, bits);
+            dmax = max(dmax, bits);
+          }
+        }
+    }
+    dmin = wave::min_u32(dmin);
+    dmax = wave::max_u32(dmax);
+    umax = wave::max_u32(umax);
+    if (lane == 0) {
+      float* const o = a.pstat + 3 * size_t(j - 1);
+      o[0] = __uint_as_float(dmin);
+      o[1] = __uint_as_float(dmax);
+      o[2] = __uint_as_float(umax);
+    }
+  }
   // T (2n x n, final row order) and C_j U^-1 to their blocks
   TW* Tj = a.Tm + size_t(j) * tsize(n);
 #pragma unroll
@@ -368,18 +421,28 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
 }
 
 // ---- B: the right-hand part on the matrix cores ----------------------------------
-template <typename TS, typename TW, int NB, int RS, int RESTMAX, int NW>
+// LDS of a pair: per wave one staged 16-column tile (rows by final position:
+// top slots [0, NT), rest slots [NT, NT + 16 NRT): reduced rows, border rows;
+// column stride XLD); the inverses of the unit lower diagonal blocks; the
+// final position of every panel row.
+template <typename TW, int NB, int NRT, int NW>
+struct RhsLds {
+  static constexpr int PAD = sizeof(TW) == 8 ? 2 : 4;   // columns' reads on different banks
+  static constexpr int NT = 16 * NB, XLD = NT + 16 * NRT + PAD, DLD = 16 + PAD;
+  alignas(16) TW x[NW][16 * XLD];
+  alignas(16) TW inv[NB][16 * DLD];
+  uint8_t pos[2 * NT];
+};
+
+template <typename TS, typename TW, int NB, int NRT, int NW>
 __device__ __forceinline__ void pair_rhs_body(FactorArgs<TS, TW> const& a, int p) {
-  using G = MfmaGeom<16 * NB, RESTMAX, RS>;
-  constexpr int NT = G::NT, NR = G::NR, LD = G::LD, XLD = G::XLD;
-  __shared__ __align__(16) TW Ls[(NT + NR) * LD];
-  __shared__ __align__(16) TW Xt[NW][16 * XLD];
-  __shared__ unsigned sstat[NW][3];   // per-wave panel statistics
+  using Lds = RhsLds<TW, NB, NRT, NW>;
+  constexpr int NT = Lds::NT, XLD = Lds::XLD, DLD = Lds::DLD, H = 4 * NB;   // H: values per lane of a tile
+  __shared__ Lds sm;
   if (p >= a.npairs) return;   // uniform over the workgroup
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, g = lane >> 4, cl = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int n = a.n, nr = a.nr, nx = a.nx, n2 = 2 * n;
-  const int R = n2 + nr;
   int j, jp, jpp;
   pair_of_uniform(a, p, j, jp, jpp);
   const size_t nn = size_t(n) * n, rn = size_t(nr) * n, bn = size_t(n) * nx;
@@ -391,286 +454,288 @@ __device__ __forceinline__ void pair_rhs_body(FactorArgs<TS, TW> const& a, int p
   // again, a dependent memory round trip in front of the load it addresses)
   const TS *const sD = a.sD, *const sE = a.sE, *const sB = a.sB, *const sC = a.sC;
   TW *const Dm = a.D, *const Em = a.E, *const Bm = a.B, *const Cm = a.C, *const Fm = a.Fpart;
+  const int first = a.first;
   // the final positions of this lane's two panel rows, stored by kernel A
   // after the panel's 2n^2 entries
   const uint8_t* const posb = reinterpret_cast<const uint8_t*>(Tj + size_t(2) * n * n);
   const uint8_t pb0 = posb[lane < n2 ? lane : 0], pb1 = posb[lane + 64 < n2 ? lane + 64 : 0];
 
-  // this lane's two panel rows as right-hand sources, and the first tile's
-  // loads, in flight while the multipliers are staged
-  RowSrc rsrc[RS];
-#pragma unroll
-  for (int s = 0; s < RS; ++s) {
-    const int r = lane + 64 * s;
-    rsrc[s].cls = r < n ? 1 : r < n2 ? 2 : r < R ? 4 : 0;
-    rsrc[s].off = r < n ? r : r < n2 ? r - n : r < R ? r - n2 : 0;
-  }
   const int tA = (n + 15) / 16, tC = (nx + 15) / 16;
   const int ntiles = 2 * tA + tC;
-  // the tile's raw source values, loaded one tile ahead: row lane + 64 s,
-  // column c0 + cc of the tile's region
-  TS xs[RS][16];
-  if (w < ntiles) {
-#pragma unroll
-    for (int s = 0; s < RS; ++s) load_rhs_row(xs[s], sD, sE, sB, sC, n, nr, nx, w, tA, j, jp, rsrc[s]);
-  }
+  // a tile of D_jp or E_j is one run of 16 n values: element e = lane + 64 h
+  // is row e % n of its column e / n (e < 1024: exact through the reciprocal)
+  const unsigned rcp = (65536u + unsigned(n) - 1) / unsigned(n);
+  const unsigned rcpr = nr > 0 ? (65536u + unsigned(nr) - 1) / unsigned(nr) : 0;
 
-  // Ls: top rows (final positions < n) hold -L11 below the diagonal blocks
-  // and the inverses of L11's unit lower 16 x 16 diagonal blocks on them
-  // (set below); rest rows hold -[L21; C_j U^-1].  Rows are final positions,
-  // so every read is a column of T (or of C_j U^-1).
-  // Lanes over the columns k of T (column-major: a lane reads along its
-  // column, and the writes of Ls rows are bank-conflict-free); all loads are
-  // clamped and issued before their first use (T blocks are 4-byte aligned
-  // only: n (2n + 1) floats each).  Top row q < n: L below the diagonal, negated
-  // outside the diagonal blocks; rest row n + i: -T row n + i; border rows
-  // and padding rows below.
-  {
-    const int k = lane, kk = k < n ? k : n - 1;
-    constexpr int PAIRS = (2 * NT + 2 * NW - 1) / (2 * NW);   // row pairs of T per wave
-    V2<TW> tv[PAIRS];
+  // the run of tile t's part: D_jp (region 0), E_j (1), B_jp and B_j (2), and
+  // with the first part the border rows' terms, nr values per column each:
+  // C_jp and its pending slot (region 0), the pending C_jpp the tile adds to
+  // (region 1).  Always issued before the stores of the tile before: a wait
+  // for loads behind stores waits for those too.
+  TS xs[H], cin[2];
+  TW pin[2];
+  auto load_tile = [&](int t, int part) {
+    const int reg = t < tA ? 0 : t < 2 * tA ? 1 : 2;
+    const int c0 = 16 * (reg == 0 ? t : reg == 1 ? t - tA : t - 2 * tA);
+    const int width = min(16, (reg == 2 ? nx : n) - c0);
+    const TS* src = (reg == 0 ? sD + jp * nn : reg == 1 ? sE + j * nn : sB + (part ? j : jp) * bn) + size_t(c0) * n;
 #pragma unroll
-    for (int h = 0; h < PAIRS; ++h) {
-      const int q0 = 2 * (w + NW * h), qc = q0 < n2 ? q0 : 0;
-      tv[h].x = Tj[qc + size_t(kk) * n2];
-      tv[h].y = Tj[qc + 1 + size_t(kk) * n2];
+    for (int h = 0; h < H; ++h) xs[h] = gload(src, unsigned(min(lane + 64 * h, width * n - 1)));
+    if (part == 0 && nr > 0) {
+      const size_t eb = size_t(c0) * nr;
+      const TW* pe = reg == 0 ? pend_prv + jp * rn + eb : pend_cur + jpp * rn + eb;
+      const TS* ce = sC + jp * rn + eb;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const unsigned e = reg < 2 ? min(lane + 64 * h, nr * width - 1) : 0;
+        cin[h] = gload(reg < 2 ? ce : sC, e);
+        pin[h] = gload(reg < 2 ? pe : a.Cpend, e);
+      }
     }
-    // the border rows C_j U^-1 (nr <= kNrB, nr x n column-major), issued with
-    // the T loads; wave 0 stores them
-    TW cv[kNrB];
-    if (nr > 0) {
+  };
+  if (w < ntiles) load_tile(w, 0);
+
+  // A operands, in registers for all tiles of the wave: -L below the diagonal
+  // blocks, -[L21; C_j U^-1] (rows of T are final positions)
+  V4<TW> lb[NB][NB], lr[NRT][NB];
 #pragma unroll
-      for (int ri = 0; ri < kNrB; ++ri) cv[ri] = Cm[j * rn + (ri < nr ? ri : 0) + size_t(kk) * nr];
+  for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+    for (int m = 0; m <= kb; ++m) {
+      if (m == kb && kb % NW != w) continue;   // diagonal blocks: this wave's only
+      const int r = 16 * kb + cl;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = 16 * m + kro<TW>(g, i);
+        const TW v = gload(Tj, (r < n ? r : 0) + unsigned(c < n ? c : 0) * unsigned(n2));
+        const bool ok = r < n && c < n && (m < kb || c < r);
+        lb[kb][m][i] = keep_if(m < kb ? -v : v, ok);
+      }
     }
-    // the selector's statistics of this panel (FP32 batches): |U_qq| min and
-    // max, |U_qk| max over q <= k, as float bits (non-negative: ordered as
-    // unsigned), from the U entries this wave reads anyway
-    const bool stats = sizeof(TW) == 4 && a.pstat != nullptr;
-    unsigned dmin = 0xffffffffu, dmax = 0u, umax = 0u;
+  // (in flight over the inverses where the registers hold them beside those;
+  // where they do not, the inverses stay in LDS too)
+  constexpr bool LATE = NB >= 3;
+  auto load_rest = [&] {
 #pragma unroll
-    for (int h = 0; h < PAIRS; ++h) {
-      const int q0 = 2 * (w + NW * h);
-      if (q0 < n2 && k < NT) {
+    for (int rt = 0; rt < NRT; ++rt) {
+      const int q = 16 * rt + cl;
 #pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          const int q = q0 + d;
-          const TW v = d == 0 ? tv[h].x : tv[h].y;
-          TW x;
-          int row;
-          if (q < n) {
-            row = q;
-            x = k < q ? ((k >> 4) == (q >> 4) ? v : -v) : TW(0);
-            if (stats && k >= q && k < n) {
-              const unsigned bits = __float_as_uint(fabsf(float(v)));
-              umax = max(umax, bits);
-              if (k == q) {
-                dmin = min(dmin, bits);
-                dmax = max(dmax, bits);
-              }
-            }
-          } else {
-            row = NT + q - n;
-            x = -v;
-          }
-          Ls[row * LD + k] = keep_if(x, k < n);
+      for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int c = 16 * kb + kro<TW>(g, i);
+          const TW v = gload(Tj, unsigned(n + (q < n ? q : 0)) + unsigned(c < n ? c : 0) * unsigned(n2));
+          lr[rt][kb][i] = keep_if(-v, q < n && c < n);
         }
+      if (16 * rt + 16 > n && 16 * rt < n + nr) {   // border rows of C_j U^-1
+        const TW* const Cj = Cm + j * rn;
+        const bool bord = q >= n && q < n + nr;
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int c = 16 * kb + kro<TW>(g, i);
+            const TW v = gload(Cj, unsigned(bord ? q - n : 0) + unsigned(c < n ? c : 0) * unsigned(nr));
+            lr[rt][kb][i] += keep_if(-v, bord && c < n);
+          }
       }
     }
-    if (stats) {
-      dmin = wave::min_u32(dmin);
-      dmax = wave::max_u32(dmax);
-      umax = wave::max_u32(umax);
-      if (lane == 0) {
-        sstat[w][0] = dmin;
-        sstat[w][1] = dmax;
-        sstat[w][2] = umax;
-      }
-    }
-    // border rows (C_j U^-1, nr x n column-major) and the zero padding rows
-    if (w == 0 && k < NT) {
+  };
+  if (!LATE) load_rest();
+  // this wave's diagonal blocks, row-major, then their inverses in place:
+  // column lane % 16 of block lane / 16 by forward substitution; rows beyond
+  // n are zero, their inverse rows identity
 #pragma unroll
-      for (int ri = 0; ri < kNrB; ++ri)
-        if (ri < nr) Ls[(NT + n + ri) * LD + k] = keep_if(-cv[ri], k < n);
-      for (int q = n; q < NT; ++q) Ls[q * LD + k] = TW(0);
-      for (int i = n + nr; i < NR; ++i) Ls[(NT + i) * LD + k] = TW(0);
-    }
-  }
-  // the final position of this lane's two rows (kernel A's bytes)
-  const int pos0 = lane < n2 ? int(pb0) : lane, pos1 = lane + 64 < n2 ? int(pb1) : lane + 64;
-  __syncthreads();   // Ls loaded
-  if (sizeof(TW) == 4 && a.pstat != nullptr && w == 0 && lane == 0) {
-    unsigned dmin = sstat[0][0], dmax = sstat[0][1], umax = sstat[0][2];
+  for (int kb = 0; kb < NB; ++kb)
+    if (kb % NW == w) {
 #pragma unroll
-    for (int v = 1; v < NW; ++v) {
-      dmin = min(dmin, sstat[v][0]);
-      dmax = max(dmax, sstat[v][1]);
-      umax = max(umax, sstat[v][2]);
+      for (int i = 0; i < 4; ++i) sm.inv[kb][cl * DLD + kro<TW>(g, i)] = lb[kb][kb][i];
     }
-    float* const o = a.pstat + 3 * size_t(j - 1);
-    o[0] = __uint_as_float(dmin);
-    o[1] = __uint_as_float(dmax);
-    o[2] = __uint_as_float(umax);
+  if (w == 0) {
+    if (lane < n2) sm.pos[lane] = pb0;
+    if (lane + 64 < n2) sm.pos[lane + 64] = pb1;
   }
-  if (lane < NT && (lane >> 4) % NW == w) {
-    // the inverse of diagonal block lane / 16 of L11 (unit lower), column
-    // lane % 16, by forward substitution in place (the blocks dealt out to
-    // the waves); rows beyond n are zero, their inverse rows identity
-    const int b = lane >> 4, jj = lane & 15;
+  TW* const x = sm.x[w];
+#pragma unroll
+  for (int h = 0; h < (16 * XLD + 63) / 64; ++h)
+    if (lane + 64 * h < 16 * XLD) x[lane + 64 * h] = TW(0);   // the padding slots stay zero
+  lds_order();
+  if (lane < 16 * NB && (lane >> 4) % NW == w) {
+    TW* const blk = sm.inv[lane >> 4];
+    const int jj = lane & 15;
     TW y[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) y[i] = TW(0);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const TW* li = Ls + (16 * b + i) * LD + 16 * b;
+      const TW* li = blk + i * DLD;
       TW t0 = TW(0), t1 = TW(0);
 #pragma unroll
-      for (int k0 = 0; k0 < i; k0 += 4) {
-        const V4<TW> l4 = *reinterpret_cast<const V4<TW>*>(li + k0);
-        t0 = fma(l4.x, y[k0], t0);
-        if (k0 + 1 < 16) t1 = fma(l4.y, y[k0 + 1 < 16 ? k0 + 1 : 0], t1);
-        if (k0 + 2 < 16) t0 = fma(l4.z, y[k0 + 2 < 16 ? k0 + 2 : 0], t0);
-        if (k0 + 3 < 16) t1 = fma(l4.w, y[k0 + 3 < 16 ? k0 + 3 : 0], t1);
+      for (int k = 0; k < i; k += 2) {
+        const V2<TW> l2 = *reinterpret_cast<const V2<TW>*>(li + k);
+        // (entries 4m, 4m + 2 and 4m + 1, 4m + 3 in two chains)
+        t0 = fma(l2.x, y[k], t0);
+        t1 = fma(l2.y, y[k + 1], t1);
       }
       y[i] = jj == i ? TW(1) : -(t0 + t1);
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // (not all rows' reads at once)
     }
-    // every lane has read its block rows (reads precede these writes in this wave)
+    // every lane has read its block's rows (reads precede these writes in this wave)
+    lds_order();
 #pragma unroll
-    for (int i = 0; i < 16; ++i) Ls[(16 * b + i) * LD + 16 * b + jj] = y[i];
+    for (int i = 0; i < 16; ++i) blk[i * DLD + jj] = y[i];
   }
-  __syncthreads();   // the diagonal inverses in place
+  __syncthreads();   // the inverses and the row positions in place
+  if (LATE) load_rest();
+  auto inverse = [&](int kb) { return ld4(&sm.inv[kb][cl * DLD], g); };
+  if (!LATE) {
+#pragma unroll
+    for (int kb = 0; kb < NB; ++kb) lb[kb][kb] = inverse(kb);
+  }
+  // where element h of a run goes: as row of block jp (low half), of block j
+  unsigned slot[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const unsigned e = lane + 64 * h, col = (e * rcp) >> 16, row = min(e - col * n, unsigned(n) - 1);
+    const unsigned q0 = sm.pos[row], q1 = sm.pos[n + row];
+    slot[h] = (col * XLD + (q0 < unsigned(n) ? q0 : NT + q0 - n)) | (col * XLD + (q1 < unsigned(n) ? q1 : NT + q1 - n)) << 16;
+  }
 
-  TW* xt = Xt[w];
-  const int g = lane >> 4, cl = lane & 15;
-  int slot[RS];
-#pragma unroll
-  for (int s = 0; s < RS; ++s) {
-    const int r = lane + 64 * s;
-    if (r < n2) {
-      const int q = s == 0 ? pos0 : pos1;
-      slot[s] = q < n ? q : NT + q - n;
-    } else if (r < R) {
-      slot[s] = NT + r - n;
-    } else {   // lanes beyond the panel zero the padding slots
-      const int i = r - R;
-      slot[s] = i < NT - n ? n + i : i - (NT - n) < NR - (n + nr) ? NT + n + nr + (i - (NT - n)) : NT + NR;
-    }
-  }
   for (int t = w; t < ntiles; t += NW) {
     const int reg = t < tA ? 0 : t < 2 * tA ? 1 : 2;
     const int c0 = 16 * (reg == 0 ? t : reg == 1 ? t - tA : t - 2 * tA);
-    const int width = reg == 2 ? nx : n;
-    // stage the tile: column cc at xt[cc * XLD + slot], zeros outside the region's rows
-#pragma unroll
-    for (int s = 0; s < RS; ++s) {
-      const int cls = rsrc[s].cls;
-      const bool valid = reg == 0 ? (cls & 5) != 0 : reg == 1 ? cls == 2 : (cls & 3) != 0;
-      // a whole tile (a uniform test): one row mask for all columns (not for
-      // NB = 2, where the second copy of the loop would cost a wave per SIMD)
-      // (FP32 only: the integer mask is one 32-bit AND per value)
-      if (sizeof(TW) == 4 && NB > 2 && c0 + 16 <= width) {
-        int m = valid ? -1 : 0;
-        asm volatile("" : "+v"(m));
-#pragma unroll
-        for (int cc = 0; cc < 16; ++cc) xt[cc * XLD + slot[s]] = mask_bits(TW(xs[s][cc]), m);
-      } else {
-#pragma unroll
-        for (int cc = 0; cc < 16; ++cc) xt[cc * XLD + slot[s]] = keep_if(TW(xs[s][cc]), valid && c0 + cc < width);
-      }
-    }
-    // the border rows' extra terms, nr x 16 contiguous values each (element
-    // e = border row e % nr, tile column e / nr): pending C_jp (region 0, read
-    // once, cleared for reuse) and the pending C_jpp this tile adds to (region 1)
-    const int m = nr * min(16, width - c0);
+    const int width = min(16, (reg == 2 ? nx : n) - c0);
+    const int cnt = width * n;
+    const int m = nr * width;
     const size_t eb = size_t(c0) * nr;
-    TW pin[2] = {TW(0), TW(0)};
-    if ((reg == 0 && !a.first) || reg == 1) {
-      const TW* pe = reg == 0 ? pend_prv + jp * rn + eb : pend_cur + jpp * rn + eb;
+    // (at the first level nothing is pending in C_jp's slot, and it is clear)
+    TW padd[2] = {TW(0), TW(0)};
+    // element h of a run to its slot, the other block's rows zero
+    auto stage = [&](bool hi, bool clear) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        if (lane + 64 * h < m) pin[h] = pe[lane + 64 * h];
-    }
-    // the next tile's loads fly over this tile's work
-    if (t + NW < ntiles) {
-#pragma unroll
-      for (int s = 0; s < RS; ++s) load_rhs_row(xs[s], sD, sE, sB, sC, n, nr, nx, t + NW, tA, j, jp, rsrc[s]);
-    }
-    if (reg == 0 && !a.first) {   // pending C_jp into the border slots
-      TW* pe = pend_prv + jp * rn + eb;
+      for (int h = 0; h < H; ++h)
+        if (lane + 64 * h < 16 * n) {
+          const unsigned s0 = slot[h] & 0xffffu, s1 = slot[h] >> 16;
+          x[hi ? s1 : s0] = TW(xs[h]);
+          if (clear) x[hi ? s0 : s1] = TW(0);
+        }
+    };
+    stage(reg == 1, reg < 2);
+    if (m > 0) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int e = lane + 64 * h;
-        if (e < m) {
-          const int cc = e / nr, rb = e - cc * nr;
-          xt[cc * XLD + NT + n + rb] += pin[h];
-          pe[e] = TW(0);
+        const unsigned e = lane + 64 * h, cc = (e * rcpr) >> 16;
+        if (e < unsigned(m)) {
+          x[cc * XLD + NT + n + (e - cc * nr)] = reg == 0 ? (first ? TW(cin[h]) : TW(cin[h]) + pin[h]) : TW(0);
+          padd[h] = pin[h];
+          if (reg == 0 && !first) pend_prv[jp * rn + eb + e] = TW(0);   // read once: clear for reuse
         }
       }
     }
-
-    // where this lane's column goes: pivot rows -> block j, reduced rows -> block jp
-    const int kc = c0 + cl;
-    const bool colok = kc < width;
-    TW* const blk = reg == 0 ? Dm : reg == 1 ? Em : Bm;
-    const size_t bsz = reg == 2 ? bn : nn;
-    const int kcs = colok ? kc : 0;
-    TW* const dtop = blk + size_t(j) * bsz + size_t(kcs) * n;
-    TW* const drest = blk + size_t(jp) * bsz + size_t(kcs) * n;
-
+    // the next run's loads fly over this tile's work
+    if (reg == 2) {   // B_j after B_jp
+      load_tile(t, 1);
+      stage(true, false);
+    }
+    if (t + NW < ntiles) load_tile(t + NW, 0);
+    lds_order();
+    const TW* const xc = x + cl * XLD;
     // U12 = L11^-1 X_top by 16-row blocks: u_kb = inv(L_kk) (X_kb - sum_{m<kb}
-    // L_km u_m).  A block of U12 in the accumulator layout (rows 4g + i,
-    // column cl) is the B operand layout of the next products as it stands.
+    // L_km u_m).  A block of U12 in the accumulator layout is the B operand
+    // layout of the next products as it stands.
     V4<TW> u[NB];
 #pragma unroll
     for (int kb = 0; kb < NB; ++kb) {
-      V4<TW> acc = ld4(xt + cl * XLD + kb * 16, g);
+      V4<TW> acc = ld4(xc + 16 * kb, g);
 #pragma unroll
-      for (int mb = 0; mb < kb; ++mb)   // -L_km is in Ls
-        acc = mfma4<TW>(ld4(Ls + (kb * 16 + cl) * LD + mb * 16, g), u[mb], acc);
-      u[kb] = mfma4<TW>(ld4(Ls + (kb * 16 + cl) * LD + kb * 16, g), acc, V4<TW>{TW(0), TW(0), TW(0), TW(0)});
+      for (int mb = 0; mb < kb; ++mb) acc = mfma4<TW>(lb[kb][mb], u[mb], acc);
+      u[kb] = mfma4<TW>(LATE ? inverse(kb) : lb[kb][kb], acc, V4<TW>{TW(0), TW(0), TW(0), TW(0)});
     }
-    if (colok) {
+    // X_rest' = X_rest - [L21; C_j U^-1] U12, ZT tiles' chains side by side,
+    // back to their slots
+    constexpr int ZT = NB == 3 && sizeof(TW) == 8 ? 2 : NRT;
 #pragma unroll
-      for (int kb = 0; kb < NB; ++kb) store_block(dtop, kb, g, u[kb], n);
+    for (int r0 = 0; r0 < NRT; r0 += ZT) {
+      V4<TW> z[ZT];
+#pragma unroll
+      for (int rt = 0; rt < ZT; ++rt)
+        if (r0 + rt < NRT) z[rt] = ld4(xc + NT + 16 * (r0 + rt), g);
+#pragma unroll
+      for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int rt = 0; rt < ZT; ++rt)
+            if (r0 + rt < NRT) z[rt] = mfma1(lr[r0 + rt < NRT ? r0 + rt : 0][kb][i], u[kb][i], z[rt]);
+#pragma unroll
+      for (int rt = 0; rt < ZT; ++rt)
+        if (r0 + rt < NRT) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int q = 16 * (r0 + rt) + kro<TW>(g, i);
+            x[cl * XLD + NT + q] = q < n + nr ? z[rt][i] : TW(0);
+          }
+        }
+      if (ZT < NRT) __builtin_amdgcn_sched_barrier(0);
     }
-    // X_rest' = X_rest - [L21; C_j U^-1] U12 (the minus sign is in Ls), over
-    // the 16-row tiles the n + nr rest rows occupy (one fewer than NR / 16
-    // when n + nr <= NR - 16)
-    if (n + nr <= NR - 16)
-      rest_tiles<NB, NR / 16 - 1, NT, LD, XLD, TW>(u, Ls, xt, cl, g, n, nr, colok, drest);
-    else
-      rest_tiles<NB, NR / 16, NT, LD, XLD, TW>(u, Ls, xt, cl, g, n, nr, colok, drest);
+    // pivot rows -> block j, reduced rows -> block jp, through the tile's
+    // place in LDS as whole runs
+#pragma unroll
+    for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int q = 16 * kb + kro<TW>(g, i);
+        x[cl * XLD + q] = q < n ? u[kb][i] : TW(0);
+      }
+    lds_order();
+    TW* const blk = (reg == 0 ? Dm : reg == 1 ? Em : Bm) + size_t(c0) * n;
+    const size_t bsz = reg == 2 ? bn : nn;
+    TW *const dj = blk + size_t(j) * bsz, *const djp = blk + size_t(jp) * bsz;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const unsigned e = lane + 64 * h, o = e + ((e * rcp) >> 16) * unsigned(XLD - n);
+      if (e < unsigned(cnt)) {
+        dj[e] = x[o];
+        djp[e] = x[o + NT];
+      }
+    }
     // border rows: C_jp' (region 0), pending C_jpp += (region 1), F partial (region 2)
     TW* const bdst = reg == 0 ? Cm + jp * rn + eb : reg == 1 ? pend_cur + jpp * rn + eb
                                                               : Fm + size_t(j) * nr * nx + eb;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int e = lane + 64 * h;
-      if (e < m) {
-        const int cc = e / nr, rb = e - cc * nr;
-        const TW v = xt[cc * XLD + NT + n + rb];
-        bdst[e] = reg == 1 ? pin[h] + v : v;
+      const unsigned e = lane + 64 * h, cc = (e * rcpr) >> 16;
+      if (e < unsigned(m)) {
+        const TW v = x[cc * XLD + NT + n + (e - cc * nr)];
+        bdst[e] = reg == 1 ? padd[h] + v : v;
       }
     }
+    lds_order();
   }
 }
 
+// waves per SIMD the panel's registers have to leave room for
+constexpr int panel_waves(int nb, size_t elem) { return elem == 8 && nb == 3 ? 2 : 1; }
+
 template <typename TS, typename TW, int NB, int RS, int NRMAX>
-__global__ void __launch_bounds__(64) pair_lu_t_kernel(FactorArgs<TS, TW> a) {
+__global__ void __launch_bounds__(64, panel_waves(NB, sizeof(TW))) pair_lu_t_kernel(FactorArgs<TS, TW> a) {
   pair_lu_t_body<TS, TW, NB, RS, NRMAX>(a, blockIdx.x);
 }
 template <typename TS, typename TW, int NB, int RS, int NRMAX>
-__global__ void __launch_bounds__(64) pair_lu_t_batched(BatchTable<FactorArgs<TS, TW>> t) {
+__global__ void __launch_bounds__(64, panel_waves(NB, sizeof(TW))) pair_lu_t_batched(BatchTable<FactorArgs<TS, TW>> t) {
   const int e = t.entry[blockIdx.x];
   pair_lu_t_body<TS, TW, NB, RS, NRMAX>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
-template <typename TS, typename TW, int NB, int RS, int RESTMAX, int NW>
-__global__ void __launch_bounds__(64 * NW) pair_rhs_mfma_kernel(FactorArgs<TS, TW> a) {
-  pair_rhs_body<TS, TW, NB, RS, RESTMAX, NW>(a, blockIdx.x);
+constexpr int rhs_waves(int nb, size_t elem) { return elem == 8 ? (nb <= 3 ? 2 : 1) : nb <= 2 ? 4 : nb == 3 ? 3 : 2; }
+
+template <typename TS, typename TW, int NB, int NRT, int NW>
+__global__ void __launch_bounds__(64 * NW, rhs_waves(NB, sizeof(TW))) pair_rhs_mfma_kernel(FactorArgs<TS, TW> a) {
+  pair_rhs_body<TS, TW, NB, NRT, NW>(a, blockIdx.x);
 }
-template <typename TS, typename TW, int NB, int RS, int RESTMAX, int NW>
-__global__ void __launch_bounds__(64 * NW) pair_rhs_mfma_batched(BatchTable<FactorArgs<TS, TW>> t) {
+template <typename TS, typename TW, int NB, int NRT, int NW>
+__global__ void __launch_bounds__(64 * NW, rhs_waves(NB, sizeof(TW))) pair_rhs_mfma_batched(BatchTable<FactorArgs<TS, TW>> t) {
   const int e = t.entry[blockIdx.x];
-  pair_rhs_body<TS, TW, NB, RS, RESTMAX, NW>(t.args[e], int(blockIdx.x) - t.first[e]);
+  pair_rhs_body<TS, TW, NB, NRT, NW>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
 
 // waves per pair in the right-hand kernel
@@ -689,40 +754,32 @@ int mfma_variant(int n, int nr, int nx) {
 
 }  // namespace
 
-bool pair_lu_mfma_fits(int n, int nr, int nx, bool fp64) {
-  const int v = mfma_variant(n, nr, nx);
-  return fp64 ? v == 1 || v == 2 : v != 0;
-}
+bool pair_lu_mfma_fits(int n, int nr, int nx) { return mfma_variant(n, nr, nx) != 0; }
 
 namespace {
-// the A and B launches of shape variant V (FP64 factors: V = 1, 2; the T
-// panel of V = 3 would need 384 registers per lane in FP64)
+// the A and B launches of shape variant V
 template <int V, typename TS, typename TW>
 void launch_pair(FactorArgs<TS, TW> const& a, hipStream_t st) {
-  constexpr int NB = V + 1, RS = V == 3 ? 3 : 2, RESTMAX = 32 + 16 * V;
+  constexpr int NB = V + 1, RS = V == 3 ? 3 : 2, NRT = V + 2;   // NRT: tiles of the n + nr rest rows
   hipLaunchKernelGGL((pair_lu_t_kernel<TS, TW, NB, RS, kNrB>), dim3(a.npairs), dim3(64), 0, st, a);
-  hipLaunchKernelGGL((pair_rhs_mfma_kernel<TS, TW, NB, RS, RESTMAX, kRhsWaves>), dim3(a.npairs), dim3(64 * kRhsWaves),
+  hipLaunchKernelGGL((pair_rhs_mfma_kernel<TS, TW, NB, NRT, kRhsWaves>), dim3(a.npairs), dim3(64 * kRhsWaves),
                      0, st, a);
 }
 template <int V, typename TS, typename TW>
 void launch_pair_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, hipStream_t st) {
-  constexpr int NB = V + 1, RS = V == 3 ? 3 : 2, RESTMAX = 32 + 16 * V;
+  constexpr int NB = V + 1, RS = V == 3 ? 3 : 2, NRT = V + 2;   // NRT: tiles of the n + nr rest rows
   hipLaunchKernelGGL((pair_lu_t_batched<TS, TW, NB, RS, kNrB>), dim3(nblocks), dim3(64), 0, st, t);
-  hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, RS, RESTMAX, kRhsWaves>), dim3(nblocks), dim3(64 * kRhsWaves),
+  hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWaves>), dim3(nblocks), dim3(64 * kRhsWaves),
                      0, st, t);
 }
 }  // namespace
 
 template <typename TS, typename TW>
 bool launch_pair_lu_mfma(FactorArgs<TS, TW> const& a, hipStream_t st, hipError_t* err) {
-  constexpr bool f64 = sizeof(TW) == 8;
   switch (mfma_variant(a.n, a.nr, a.nx)) {
     case 1: launch_pair<1>(a, st); break;
     case 2: launch_pair<2>(a, st); break;
-    case 3:
-      if constexpr (f64) return false;
-      else launch_pair<3>(a, st);
-      break;
+    case 3: launch_pair<3>(a, st); break;
     default:
       return false;
   }
@@ -733,14 +790,10 @@ bool launch_pair_lu_mfma(FactorArgs<TS, TW> const& a, hipStream_t st, hipError_t
 template <typename TS, typename TW>
 bool launch_pair_lu_mfma_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, int n, int nx, int nr,
                                  hipStream_t st, hipError_t* err) {
-  constexpr bool f64 = sizeof(TW) == 8;
   switch (mfma_variant(n, nr, nx)) {
     case 1: launch_pair_batched<1>(t, nblocks, st); break;
     case 2: launch_pair_batched<2>(t, nblocks, st); break;
-    case 3:
-      if constexpr (f64) return false;
-      else launch_pair_batched<3>(t, nblocks, st);
-      break;
+    case 3: launch_pair_batched<3>(t, nblocks, st); break;
     default:
       return false;
   }

@@ -32,10 +32,9 @@ bool pair_lu_cols_fits(int n, int nr, int nx);
 template <typename TS, typename TW>
 bool launch_pair_lu_cols(FactorArgs<TS, TW> const& a, hipStream_t st, hipError_t* err);
 // the matrix-core pair: one wave factors T, the right-hand columns are
-// blocked triangular solves and GEMMs on the matrix cores.  FP32 factors:
-// n <= 64, n + nr <= 80, nr <= 8, nx <= 16; FP64 factors: n <= 48,
-// n + nr <= 64; false otherwise
-bool pair_lu_mfma_fits(int n, int nr, int nx, bool fp64);
+// blocked triangular solves and GEMMs on the matrix cores.  n <= 64,
+// n + nr <= 80, nr <= 8, nx <= 16; false otherwise
+bool pair_lu_mfma_fits(int n, int nr, int nx);
 template <typename TS, typename TW>
 bool launch_pair_lu_mfma(FactorArgs<TS, TW> const& a, hipStream_t st, hipError_t* err);
 
