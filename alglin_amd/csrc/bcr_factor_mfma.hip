@@ -21,7 +21,8 @@
 //     with the blocked update (loads and stores alone are 0.4 ms).  Rows do
 //     not move; each row is stored at its final position (T, C_j U^-1, perm),
 //     and the positions themselves go to the unused tail of T (one byte per
-//     row).
+//     row).  pair_lu_tw: the same by a wave per block, FP64 beyond n = 48 and
+//     small FP32 launches beyond n = 32.
 //  B. pair_rhs_mfma: the right-hand part X = [col jp | col jpp | xb], two
 //     waves per pair, 16-column tiles, each inside one of the three column
 //     blocks.  -L11 below its diagonal blocks, the inverses of those unit
@@ -94,19 +95,89 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // Columns before KM may lie at or before cc and are masked; the later ones
 // always lie after it.
-template <int K, int KM, int RS, typename TW>
+template <int K, int KM, int RS, int SP, typename TW>
 __device__ __forceinline__ void update_after(V16<TW>& v0, V16<TW>& v1, V16<TW>& v2, bool sp, int who, int cc, TW lv0,
                                              TW lv1, TW lv2) {
   if constexpr (K < 16) {
-    const TW u = K < KM ? rl_after<K>(sp ? v1[K] : v0[K], who, cc) : wave::rl(sp ? v1[K] : v0[K], who);
+    const TW x = SP == 2 ? (sp ? v1[K] : v0[K]) : SP ? v1[K] : v0[K];
+    const TW u = K < KM ? rl_after<K>(x, who, cc) : wave::rl(x, who);
     v0[K] = fma(-lv0, u, v0[K]);
     v1[K] = fma(-lv1, u, v1[K]);
     if constexpr (RS > 2) v2[K] = fma(-lv2, u, v2[K]);
-    update_after<K + 1, KM, RS, TW>(v0, v1, v2, sp, who, cc, lv0, lv1, lv2);
+    update_after<K + 1, KM, RS, SP, TW>(v0, v1, v2, sp, who, cc, lv0, lv1, lv2);
   }
 }
 
-// ---- A: the T panel, one wave per pair ------------------------------------------
+// ---- A: the T panel ---------------------------------------------------------------
+// One pivot step of a 16-column block held by row (row sets 0 and 1 the 2n
+// candidates, a third the border rows): cc the column in the block, c the
+// step; v0[cc], v1[cc], v2[cc] become the final column, the block's columns
+// from KS on are updated (those before KM masked).  Leaves the pivot lane, its
+// row set and the multipliers for columns outside the block.  BRANCH: the
+// pivot's row set, which is uniform, chosen by a branch instead of a select per
+// entry; two FP64 blocks only (N = 100000, n = 32, first level 750 -> 730 us;
+// with three blocks or row sets the compiler spills the two forms).
+template <typename TW>
+struct PanelRows {
+  int pos0, pos1;      // positions of rows lane, lane + 64
+  int myperm = 0;      // lane c: ipiv of step c
+  bool zero_pivot = false;
+};
+template <typename TW>
+struct PivotStep {
+  int who;
+  bool sp;
+  TW l0, l1, l2;
+};
+template <int RS, bool ONE, bool BRANCH, int KS, int KM, typename TW>
+__device__ __forceinline__ PivotStep<TW> panel_step(V16<TW>& v0, V16<TW>& v1, V16<TW>& v2, PanelRows<TW>& w, int c,
+                                                    int cc, int n2, int lane) {
+  const TW x0 = v0[cc], x1 = v1[cc];
+  const TW x2 = RS > 2 ? v2[cc] : TW(0);   // border rows (row set 2)
+  const bool c0 = lane < n2 && w.pos0 >= c;
+  const bool c1 = !ONE && lane + 64 < n2 && w.pos1 >= c;
+  unsigned h0, l0, h1, l1;
+  wave::abs_key(x0, h0, l0);
+  wave::abs_key(x1, h1, l1);
+  // the better of this lane's two candidates (ties to the smaller position)
+  const bool b1 = c1 & (!c0 | (h1 > h0) | ((h1 == h0) & ((l1 > l0) | ((l1 == l0) & (w.pos1 < w.pos0)))));
+  bool zero;
+  PivotStep<TW> o;
+  o.who = wave::argmax_pos<(sizeof(TW) > 4)>(c0 | c1, b1 ? h1 : h0, b1 ? l1 : l0, b1 ? w.pos1 : w.pos0, lane, zero);
+  const int P = __builtin_amdgcn_readlane(b1 ? w.pos1 : w.pos0, o.who);
+  o.sp = !ONE && __builtin_amdgcn_readlane(int(b1), o.who) != 0;
+  w.zero_pivot = w.zero_pivot || zero;
+  w.myperm = lane == c ? P + 1 : w.myperm;
+  // the pivot row moves to position c, the row at c to the pivot's old place
+  w.pos0 = w.pos0 == c ? P : w.pos0 == P ? c : w.pos0;
+  if constexpr (!ONE) w.pos1 = w.pos1 == c ? P : w.pos1 == P ? c : w.pos1;
+  const TW pv = wave::rl(o.sp ? x1 : x0, o.who);
+  const TW rinv = pv != TW(0) ? TW(1) / pv : TW(0);
+  // rows below the pivot get the multiplier, the others keep column c
+  // (border and padding rows hold positions r >= 2n > c: always below;
+  // the padding rows are zero and never stored)
+  const bool u0 = w.pos0 > c;
+  const bool u1 = w.pos1 > c;
+  const TW m0 = x0 * rinv, m1 = x1 * rinv;
+  o.l0 = u0 ? m0 : TW(0);
+  o.l1 = u1 ? m1 : TW(0);
+  v0[cc] = u0 ? m0 : x0;
+  v1[cc] = u1 ? m1 : x1;
+  o.l2 = TW(0);
+  if constexpr (RS > 2) {   // border (and zero padding) rows: never pivots, always updated
+    o.l2 = x2 * rinv;
+    v2[cc] = o.l2;
+  }
+  // columns KS .. 15 of the block (those before are never after c)
+  if (BRANCH && !ONE) {
+    if (o.sp) update_after<KS, KM, RS, 1, TW>(v0, v1, v2, o.sp, o.who, cc, o.l0, o.l1, o.l2);
+    else update_after<KS, KM, RS, 0, TW>(v0, v1, v2, o.sp, o.who, cc, o.l0, o.l1, o.l2);
+  } else {
+    update_after<KS, KM, RS, ONE ? 0 : 2, TW>(v0, v1, v2, o.sp, o.who, cc, o.l0, o.l1, o.l2);
+  }
+  return o;
+}
+
 // Between the 16-column blocks the trailing columns take the block's 16 steps
 // at once, on the matrix cores, through LDS (one 16-column buffer):
 //   x   the block's multipliers by row (zero for a row from the step on at
@@ -283,12 +354,10 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
         }
     }
   }
-  int pos0 = lane, pos1 = lane + 64;   // positions of rows lane, lane + 64
+  PanelRows<TW> rows{lane, lane + 64};
   // 2n <= 64: every pivot candidate sits in row set 0 (row set 1 holds
   // border rows only), and the pivot row's entries come from it unselected
   constexpr bool ONE = 2 * NMAX <= 64;
-  int myperm = 0;
-  bool zero_pivot = false;
   // Steps in blocks of 16, each in GR groups of GS steps: step c of block b
   // reads and rewrites column c through a uniform register index
   // (s_set_gpr_idx) and updates the columns of blocks b.. with the pivot
@@ -300,54 +369,17 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
   // step c of block b; the block's columns from KS on are updated, those
   // before KM masked
   auto step = [&](const int b, const int c, auto KS, auto KM) {
-    const int cc = c - 16 * b;
-    const TW x0 = V[0][b][cc], x1 = V[1][b][cc];
-    const TW x2 = RS > 2 ? V[RS - 1][b][cc] : TW(0);   // border rows (row set 2)
-    const bool c0 = lane < n2 && pos0 >= c;
-    const bool c1 = !ONE && lane + 64 < n2 && pos1 >= c;
-    unsigned h0, l0, h1, l1;
-    wave::abs_key(x0, h0, l0);
-    wave::abs_key(x1, h1, l1);
-    // the better of this lane's two candidates (ties to the smaller position)
-    const bool b1 = c1 & (!c0 | (h1 > h0) | ((h1 == h0) & ((l1 > l0) | ((l1 == l0) & (pos1 < pos0)))));
-    bool zero;
-    const int who = wave::argmax_pos<(sizeof(TW) > 4)>(c0 | c1, b1 ? h1 : h0, b1 ? l1 : l0, b1 ? pos1 : pos0, lane,
-                                                        zero);
-    const int P = __builtin_amdgcn_readlane(b1 ? pos1 : pos0, who);
-    const bool sp = !ONE && __builtin_amdgcn_readlane(int(b1), who) != 0;
-    zero_pivot = zero_pivot || zero;
-    myperm = lane == c ? P + 1 : myperm;
-    // the pivot row moves to position c, the row at c to the pivot's old place
-    pos0 = pos0 == c ? P : pos0 == P ? c : pos0;
-    if constexpr (!ONE) pos1 = pos1 == c ? P : pos1 == P ? c : pos1;
-    const TW pv = wave::rl(sp ? x1 : x0, who);
-    const TW rinv = pv != TW(0) ? TW(1) / pv : TW(0);
-    // rows below the pivot get the multiplier, the others keep column c
-    // (border and padding rows hold positions r >= 2n > c: always below;
-    // the padding rows are zero and never stored)
-    const bool u0 = pos0 > c;
-    const bool u1 = pos1 > c;
-    const TW m0 = x0 * rinv, m1 = x1 * rinv;
-    const TW lv0 = u0 ? m0 : TW(0), lv1 = u1 ? m1 : TW(0);
-    V[0][b][cc] = u0 ? m0 : x0;
-    V[1][b][cc] = u1 ? m1 : x1;
-    TW lv2 = TW(0);
-    if constexpr (RS > 2) {   // border (and zero padding) rows: never pivots, always updated
-      lv2 = x2 * rinv;
-      V[RS - 1][b][cc] = lv2;
-    }
-    // columns KS .. 15 of the block (those before are never after c)
-    update_after<decltype(KS)::value, decltype(KM)::value, RS, TW>(V[0][b], V[1][b], V[RS - 1][b], sp, who, cc, lv0,
-                                                                   lv1, lv2);
+    const PivotStep<TW> o = panel_step<RS, ONE, BLOCKED && NB == 2, decltype(KS)::value, decltype(KM)::value, TW>(
+        V[0][b], V[1][b], V[RS - 1][b], rows, c, c - 16 * b, n2, lane);
     if constexpr (!BLOCKED) {
 #pragma unroll
       for (int bb = b + 1; bb < NB; ++bb)
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
-          const TW u = wave::rl(sp ? V[1][bb][k] : V[0][bb][k], who);
-          V[0][bb][k] = fma(-lv0, u, V[0][bb][k]);
-          V[1][bb][k] = fma(-lv1, u, V[1][bb][k]);
-          if constexpr (RS > 2) V[RS - 1][bb][k] = fma(-lv2, u, V[RS - 1][bb][k]);
+          const TW u = wave::rl(o.sp ? V[1][bb][k] : V[0][bb][k], o.who);
+          V[0][bb][k] = fma(-o.l0, u, V[0][bb][k]);
+          V[1][bb][k] = fma(-o.l1, u, V[1][bb][k]);
+          if constexpr (RS > 2) V[RS - 1][bb][k] = fma(-o.l2, u, V[RS - 1][bb][k]);
         }
     }
   };
@@ -360,10 +392,11 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
         step(b, c, std::integral_constant<int, GS * g + 1>{}, std::integral_constant<int, GS * g + GS>{});
     });
     if constexpr (BLOCKED && b + 1 < NB) {
-      if (16 * (b + 1) < n) trailing_update<b, NB, RS, TW>(V, sm, pos0, pos1, n, R, lane);
+      if (16 * (b + 1) < n) trailing_update<b, NB, RS, TW>(V, sm, rows.pos0, rows.pos1, n, R, lane);
     }
   });
-  if (zero_pivot && lane == 0) atomicOr(a.status, 1);
+  const int pos0 = rows.pos0, pos1 = rows.pos1;
+  if (rows.zero_pivot && lane == 0) atomicOr(a.status, 1);
   // the selector's statistics of this panel (FP32 batches): |U_cc| min and
   // max, |U_rc| max over r <= c, as float bits (non-negative: ordered as
   // unsigned); the row at final position p < n holds U row p
@@ -411,13 +444,203 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
           if (16 * b + k < n) dst[size_t(16 * b + k) * stride] = V[s][b][k];
     }
   }
-  if (lane < n) a.perm[size_t(j) * n + lane] = myperm;
+  if (lane < n) a.perm[size_t(j) * n + lane] = rows.myperm;
   // the final position of every panel row, one byte each after the panel's
   // 2n^2 entries (the LU pair leaves that tail of T unused): kernel B reads
   // them instead of replaying the swap sequence
   uint8_t* const posb = reinterpret_cast<uint8_t*>(Tj + size_t(2) * n * n);
   if (lane < n2) posb[lane] = uint8_t(pos0);
   if (lane + 64 < n2) posb[lane + 64] = uint8_t(pos1);
+}
+
+// The same panel by NB waves, one per 16-column block.  Wave b holds block b as
+// tiles in the accumulator layout until its turn; it then factors it by row and
+// publishes multipliers, pivot triangle and row positions (two sets, by the
+// parity of b), and the waves behind update their blocks from them while wave
+// b + 1, done with its own, goes on.  One barrier per block, NB for each wave.
+// A wave's tiles are dead before its rows come to life, so 64 FP64 columns
+// take 168 registers and three waves share a SIMD; one wave needed 512 and
+// spilled.  What is left is the chain of the steps.  Times of one level:
+//                         one wave              a wave per block
+//   FP64, n = 53          643 / 98 us           442 / 60 us     (4500 / 1 pairs)
+//   FP64, n = 40          342 / 43 us           523 / 41 us     (10000 / 1)
+//   FP64, n = 32          746 / 25 us           845 / 26 us     (50000 / 1)
+//   FP32, n = 60          248, 90, 60 us        302, 65, 48 us  (5000, 625, 1)
+//   FP32, n = 40          199, 53, 34 us        253, 47, 29 us  (10000, 1250, 1)
+template <typename TW, int NB, int RS>
+struct PanelWavesLds {
+  static constexpr int TILES = (2 * 16 * NB + kNrB + 15) / 16, RLD = 16 * TILES + 2, ULD = 18;
+  // (two blocks: wave 1 is the only reader of block 0, and needs no second set)
+  static constexpr int SETS = NB == 2 ? 1 : 2;
+  alignas(16) TW x[SETS][16 * RLD];     // multipliers by row (as in PanelLds::x)
+  alignas(16) TW u[NB - 1][16 * ULD];   // waves 1 ..: the pivot rows of their blocks
+  alignas(16) TW lk[SETS][16 * 16];
+  uint8_t pos[2][128];
+};
+
+template <typename TS, typename TW, int NB, int RS>
+__device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int p) {
+  using Lds = PanelWavesLds<TW, NB, RS>;
+  constexpr int TILES = Lds::TILES, RLD = Lds::RLD, ULD = Lds::ULD;
+  __shared__ Lds sm;
+  if (p >= a.npairs) return;   // uniform over the workgroup
+  const int lane = threadIdx.x & 63, g = lane >> 4, cl = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int n = a.n, nr = a.nr, n2 = 2 * n, R = n2 + nr;   // 16 (NB - 1) < n <= 16 NB
+  int j, jp, jpp;
+  pair_of_uniform(a, p, j, jp, jpp);
+  const size_t nn = size_t(n) * n, rn = size_t(nr) * n;
+  TW* const Tj = a.Tm + size_t(j) * tsize(n);
+  V16<TW> V[RS];
+  {
+    const TW* pend_cur = a.Cpend + size_t(a.slot_cur) * (a.N + 1) * rn + j * rn;
+    const TW* pend_prv = a.Cpend + size_t(a.slot_cur ^ 1) * (a.N + 1) * rn + j * rn;
+    const TS *const Ejp = a.sE + jp * nn, *const Dj = a.sD + j * nn, *const Cj = a.sC + j * rn;
+    // this wave's block as tiles: rows 16 t + g + 4 i, column 16 w + cl
+    const int col = 16 * w + cl;
+    const unsigned coff = col < n ? unsigned(col) * unsigned(n) : 0;
+    V4<TW> T[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * t + kro<TW>(g, i);
+        // rows of block jp: E_jp; rows of block j: D_j; border rows below
+        const TS* src = r < n ? Ejp + r : Dj + (r < n2 ? r - n : 0);
+        T[t][i] = keep_if(TW(src[coff]), r < n2 && col < n);
+      }
+#pragma unroll
+    for (int t = 2 * NB - 2; t < TILES; ++t)
+      if (16 * t + 16 > n2 && 16 * t < R) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 16 * t + kro<TW>(g, i);
+          const bool ok = r >= n2 && r < R && col < n;
+          const unsigned off = ok ? unsigned(r - n2) + unsigned(col) * unsigned(nr) : 0;
+          TW v = TW(gload(Cj, off));
+          if (!a.first) v += gload(pend_prv, off) + gload(pend_cur, off);
+          T[t][i] += keep_if(v, ok);
+        }
+      }
+
+    for (int b = 0; b < w; ++b) {
+      __syncthreads();
+      TW const* const x = sm.x[b & (Lds::SETS - 1)];
+      TW const* const lk = sm.lk[b & (Lds::SETS - 1)];
+      // the block's pivot rows of this wave's columns, solved with its unit
+      // lower triangle, a column per lane
+      TW* const u = sm.u[w - 1];
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+        if (16 * t < n2) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const unsigned q = unsigned(sm.pos[b & 1][(16 * t + kro<TW>(g, i)) & 127]) - 16u * b;
+            if (q < 16u && 16 * t + kro<TW>(g, i) < n2) u[q * ULD + cl] = T[t][i];
+          }
+        }
+      lds_order();
+      if (lane < 16) {
+        TW y[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) y[q] = u[q * ULD + lane];
+#pragma unroll
+        for (int k = 0; k < 15; ++k) {
+#pragma unroll
+          for (int q = k + 1; q < 16; ++q) y[q] = fma(-lk[k * 16 + q], y[k], y[q]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 1; q < 16; ++q) u[q * ULD + lane] = y[q];
+      }
+      lds_order();
+      V4<TW> uv;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) uv[i] = u[(4 * i + g) * ULD + cl];
+#pragma unroll
+      for (int t = 0; t < TILES; ++t)
+        if (16 * t < R) {
+          V4<TW> av;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) av[i] = -x[(4 * i + g) * RLD + 16 * t + cl];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) T[t] = mfma1(av[i], uv[i], T[t]);
+        }
+      lds_order();
+    }
+
+    // to the row layout through the place its multipliers will take (its last
+    // readers have passed the barrier before)
+    TW* const x = sm.x[w & (Lds::SETS - 1)];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[cl * RLD + 16 * t + kro<TW>(g, i)] = T[t][i];
+    lds_order();
+#pragma unroll
+    for (int s = 0; s < RS; ++s) {
+      const int r = lane + 64 * s;
+      V[s] = V16<TW>(TW(0));
+      if (r < 16 * TILES) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) V[s][k] = x[k * RLD + r];
+      }
+    }
+  }
+  PanelRows<TW> rows{lane, lane + 64};
+  if (w > 0) {
+    rows.pos0 = sm.pos[(w & 1) ^ 1][lane];
+    rows.pos1 = sm.pos[(w & 1) ^ 1][lane + 64];
+  }
+  static_for<0, 4>([&](auto G) {
+    constexpr int gs = 4 * decltype(G)::value;
+    const int cend = min(16 * w + gs + 4, n);
+    for (int c = 16 * w + gs; c < cend; ++c)
+      panel_step<RS, false, false, gs + 1, gs + 4, TW>(V[0], V[1], V[RS - 1], rows, c, c - 16 * w, n2, lane);
+  });
+  if (rows.zero_pivot && lane == 0) atomicOr(a.status, 1);
+  // columns 16 w .. of the interchanges
+  if (lane >= 16 * w && lane < min(16 * w + 16, n)) a.perm[size_t(j) * n + lane] = rows.myperm;
+  sm.pos[w & 1][lane] = uint8_t(rows.pos0);
+  sm.pos[w & 1][lane + 64] = uint8_t(rows.pos1);
+  if (w < NB - 1) {
+    TW* const x = sm.x[w & (Lds::SETS - 1)];
+    lds_order();
+#pragma unroll
+    for (int s = 0; s < RS; ++s) {
+      const int r = lane + 64 * s;
+      const int q = s == 0 ? rows.pos0 - 16 * w : s == 1 ? rows.pos1 - 16 * w : 16;   // (border rows: no pivots)
+      if (r < 16 * TILES) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k * RLD + r] = keep_if(V[s][k], k < q);
+      }
+      if (s < 2 && q >= 0 && q < 16) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) sm.lk[w & (Lds::SETS - 1)][k * 16 + q] = V[s][k];
+      }
+    }
+  }
+  for (int b = w; b < NB; ++b) __syncthreads();
+
+  // T (2n x n, final row order) and C_j U^-1 to their blocks
+  const int pos0 = sm.pos[(NB - 1) & 1][lane], pos1 = sm.pos[(NB - 1) & 1][lane + 64];
+#pragma unroll
+  for (int s = 0; s < RS; ++s) {
+    const int r = lane + 64 * s;
+    const int q = r < n2 ? (s == 0 ? pos0 : pos1) : r;
+    if (r < R) {
+      TW* dst = q < n2 ? Tj + q : a.C + j * rn + (q - n2);
+      const int stride = q < n2 ? n2 : nr;
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+        if (16 * w + k < n) dst[size_t(16 * w + k) * stride] = V[s][k];
+    }
+  }
+  uint8_t* const posb = reinterpret_cast<uint8_t*>(Tj + size_t(2) * n * n);
+  if (w == 0) {
+    if (lane < n2) posb[lane] = uint8_t(pos0);
+    if (lane + 64 < n2) posb[lane + 64] = uint8_t(pos1);
+  }
 }
 
 // ---- B: the right-hand part on the matrix cores ----------------------------------
@@ -726,6 +949,22 @@ __global__ void __launch_bounds__(64, panel_waves(NB, sizeof(TW))) pair_lu_t_bat
   const int e = t.entry[blockIdx.x];
   pair_lu_t_body<TS, TW, NB, RS, NRMAX>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
+// The panel by waves: in FP64 for n > 48; in FP32 (where one wave's registers
+// hold the panel, and fewer instructions fill a large launch better) for n > 32
+// and at most kWavesPairs pairs.  Both sides' times stand at pair_lu_tw_body.
+constexpr bool panel_by_waves_always(int nb, size_t elem) { return nb >= 4 && elem == 8; }
+constexpr bool panel_by_waves_few(int nb, size_t elem) { return nb >= 3 && elem == 4; }
+constexpr int kWavesPairs = 1024;
+
+template <typename TS, typename TW, int NB, int RS>
+__global__ void __launch_bounds__(64 * NB, 3) pair_lu_tw_kernel(FactorArgs<TS, TW> a) {
+  pair_lu_tw_body<TS, TW, NB, RS>(a, blockIdx.x);
+}
+template <typename TS, typename TW, int NB, int RS>
+__global__ void __launch_bounds__(64 * NB, 3) pair_lu_tw_batched(BatchTable<FactorArgs<TS, TW>> t) {
+  const int e = t.entry[blockIdx.x];
+  pair_lu_tw_body<TS, TW, NB, RS>(t.args[e], int(blockIdx.x) - t.first[e]);
+}
 constexpr int rhs_waves(int nb, size_t elem) { return elem == 8 ? (nb <= 3 ? 2 : 1) : nb <= 2 ? 4 : nb == 3 ? 3 : 2; }
 
 template <typename TS, typename TW, int NB, int NRT, int NW>
@@ -738,8 +977,12 @@ __global__ void __launch_bounds__(64 * NW, rhs_waves(NB, sizeof(TW))) pair_rhs_m
   pair_rhs_body<TS, TW, NB, NRT, NW>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
 
-// waves per pair in the right-hand kernel
-constexpr int kRhsWaves = 2;
+// Waves per pair in the right-hand kernel: two (each holds the operands of L,
+// and more waves load them more often: n = 53, 4500 pairs 598 us with two, 874
+// with four), four where a launch of at most one pair per CU leaves SIMDs idle
+// (one pair, FP64: n = 32 15 -> 12 us, n = 40 28 -> 19, n = 53 53 -> 40).
+constexpr int kRhsWaves = 2, kRhsWavesFew = 4;
+constexpr int kFewPairs = 256;
 
 // shapes: 1: n <= 32, n + nr <= 48 (two 16-column blocks); 2: n <= 48,
 // n + nr <= 64 (three); 3: n <= 64, n + nr <= 80 (four, and a third row set
@@ -761,16 +1004,31 @@ namespace {
 template <int V, typename TS, typename TW>
 void launch_pair(FactorArgs<TS, TW> const& a, hipStream_t st) {
   constexpr int NB = V + 1, RS = V == 3 ? 3 : 2, NRT = V + 2;   // NRT: tiles of the n + nr rest rows
-  hipLaunchKernelGGL((pair_lu_t_kernel<TS, TW, NB, RS, kNrB>), dim3(a.npairs), dim3(64), 0, st, a);
-  hipLaunchKernelGGL((pair_rhs_mfma_kernel<TS, TW, NB, NRT, kRhsWaves>), dim3(a.npairs), dim3(64 * kRhsWaves),
-                     0, st, a);
+  const dim3 pairs(a.npairs);
+  const auto by_waves = [&] { hipLaunchKernelGGL((pair_lu_tw_kernel<TS, TW, NB, RS>), pairs, dim3(64 * NB), 0, st, a); };
+  const auto by_one = [&] { hipLaunchKernelGGL((pair_lu_t_kernel<TS, TW, NB, RS, kNrB>), pairs, dim3(64), 0, st, a); };
+  if constexpr (panel_by_waves_always(NB, sizeof(TW))) {
+    by_waves();
+  } else if constexpr (panel_by_waves_few(NB, sizeof(TW))) {
+    if (a.npairs <= kWavesPairs && a.pstat == nullptr) by_waves();
+    else by_one();
+  } else {
+    by_one();
+  }
+  if (a.npairs <= kFewPairs) hipLaunchKernelGGL((pair_rhs_mfma_kernel<TS, TW, NB, NRT, kRhsWavesFew>), pairs, dim3(64 * kRhsWavesFew), 0, st, a);
+  else hipLaunchKernelGGL((pair_rhs_mfma_kernel<TS, TW, NB, NRT, kRhsWaves>), pairs, dim3(64 * kRhsWaves), 0, st, a);
 }
 template <int V, typename TS, typename TW>
 void launch_pair_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, hipStream_t st) {
   constexpr int NB = V + 1, RS = V == 3 ? 3 : 2, NRT = V + 2;   // NRT: tiles of the n + nr rest rows
-  hipLaunchKernelGGL((pair_lu_t_batched<TS, TW, NB, RS, kNrB>), dim3(nblocks), dim3(64), 0, st, t);
-  hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWaves>), dim3(nblocks), dim3(64 * kRhsWaves),
-                     0, st, t);
+  const dim3 pairs(nblocks);
+  // (FP32 batches: one wave, which also leaves the selector's statistics)
+  if constexpr (panel_by_waves_always(NB, sizeof(TW)))
+    hipLaunchKernelGGL((pair_lu_tw_batched<TS, TW, NB, RS>), pairs, dim3(64 * NB), 0, st, t);
+  else
+    hipLaunchKernelGGL((pair_lu_t_batched<TS, TW, NB, RS, kNrB>), pairs, dim3(64), 0, st, t);
+  if (nblocks <= kFewPairs) hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWavesFew>), pairs, dim3(64 * kRhsWavesFew), 0, st, t);
+  else hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWaves>), pairs, dim3(64 * kRhsWaves), 0, st, t);
 }
 }  // namespace
 

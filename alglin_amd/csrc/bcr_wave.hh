@@ -71,12 +71,19 @@ __device__ __forceinline__ int argmax_pos(bool cand, unsigned khi, unsigned klo,
   khi = cand ? (khi | 0x80000000u) : 0u;
   klo = cand ? klo : 0u;
   const unsigned hmax = max_u32(khi);
-  const unsigned lmax = LO ? max_u32(khi == hmax ? klo : 0u) : 0u;
-  const unsigned long long tie = __ballot(khi == hmax && klo == lmax);
-  int who;
-  if (__popcll(tie) == 1) {
+  unsigned long long tie = __ballot(khi == hmax);
+  int who = __ffsll(static_cast<long long>(tie)) - 1;
+  // The low word decides only where high words tie, which real data seldom
+  // do: a uniform branch spares its reduction.
+  unsigned lmax = 0;
+  if (LO && __popcll(tie) > 1) {
+    lmax = max_u32(khi == hmax ? klo : 0u);
+    tie = __ballot(khi == hmax && klo == lmax);
     who = __ffsll(static_cast<long long>(tie)) - 1;
-  } else {
+  } else if (LO) {
+    lmax = unsigned(__builtin_amdgcn_readlane(int(klo), __builtin_amdgcn_readfirstlane(who)));
+  }
+  if (__popcll(tie) > 1) {
     const bool mine = (tie >> lane) & 1ull;
     const unsigned pm = min_u32(mine ? unsigned(pos) : 0xffffffffu);
     who = __ffsll(static_cast<long long>(__ballot(mine && unsigned(pos) == pm))) - 1;
