@@ -131,6 +131,9 @@ template <typename TS, typename TW>
 bool launch_pair_lu_mfma_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, int n, int nx, int nr,
                                  hipStream_t st, hipError_t* err);
 template <typename TS, typename TW>
+void launch_pair_qr_rhs_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, int n, int nr, int nx,
+                                hipStream_t st);
+template <typename TS, typename TW>
 bool launch_pair_qr_batched(int method, BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, int n, int nr, int nx,
                             size_t lds_limit, hipStream_t st, hipError_t* err);
 template <typename TS, typename TW>

@@ -46,6 +46,11 @@
 //     n = 32 FP64, first level), the operands live in registers instead of
 //     LDS (more pairs per CU), and stores are whole runs (1.41 ms with
 //     operands in LDS and stores by column; now 0.97 ms, 3.2 TB/s).
+//     The right-hand part of a QR pair (pair_qr_rhs) is the same kernel with
+//     other products: 16 reflectors at a time as I - V T V^T (dlarft), V in
+//     LDS, x + V (-T^T (V^T x)) with the tile's rows in registers throughout.
+//     The LDS a pair needs sets how many share a CU: N = 20000, n = 32 FP64,
+//     first level 401 us.
 // The right-hand results differ from the rank-1 kernels in rounding only
 // (other summation order, the inverted diagonal blocks).  A pivot whose
 // reciprocal overflows (a subnormal pivot) turns the finished T columns into
@@ -656,10 +661,20 @@ struct RhsLds {
   alignas(16) TW inv[NB][16 * DLD];
   uint8_t pos[2 * NT];
 };
+// Of a QR pair: inv holds -T^T of each 16-column block (below), v the
+// reflectors by column (rows [0, n) in slots [0, NT), rows [n, 2n) from slot
+// NT on, zero elsewhere), cb the border rows of C_j R^-1 by column, as rows of
+// the two 16-row rest tiles they can lie in.
+template <typename TW, int NB, int NRT, int NW>
+struct QrRhsLds : RhsLds<TW, NB, NRT, NW> {
+  static constexpr int VLD = 2 * 16 * NB + RhsLds<TW, NB, NRT, NW>::PAD, CLD = 32 + RhsLds<TW, NB, NRT, NW>::PAD;
+  alignas(16) TW v[16 * NB * VLD];
+  alignas(16) TW cb[16 * NB * CLD];
+};
 
-template <typename TS, typename TW, int NB, int NRT, int NW>
+template <typename TS, typename TW, int NB, int NRT, int NW, bool QR>
 __device__ __forceinline__ void pair_rhs_body(FactorArgs<TS, TW> const& a, int p) {
-  using Lds = RhsLds<TW, NB, NRT, NW>;
+  using Lds = std::conditional_t<QR, QrRhsLds<TW, NB, NRT, NW>, RhsLds<TW, NB, NRT, NW>>;
   constexpr int NT = Lds::NT, XLD = Lds::XLD, DLD = Lds::DLD, H = 4 * NB;   // H: values per lane of a tile
   __shared__ Lds sm;
   if (p >= a.npairs) return;   // uniform over the workgroup
@@ -718,100 +733,172 @@ __device__ __forceinline__ void pair_rhs_body(FactorArgs<TS, TW> const& a, int p
   };
   if (w < ntiles) load_tile(w, 0);
 
-  // A operands, in registers for all tiles of the wave: -L below the diagonal
-  // blocks, -[L21; C_j U^-1] (rows of T are final positions)
-  V4<TW> lb[NB][NB], lr[NRT][NB];
-#pragma unroll
-  for (int kb = 0; kb < NB; ++kb)
-#pragma unroll
-    for (int m = 0; m <= kb; ++m) {
-      if (m == kb && kb % NW != w) continue;   // diagonal blocks: this wave's only
-      const int r = 16 * kb + cl;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = 16 * m + kro<TW>(g, i);
-        const TW v = gload(Tj, (r < n ? r : 0) + unsigned(c < n ? c : 0) * unsigned(n2));
-        const bool ok = r < n && c < n && (m < kb || c < r);
-        lb[kb][m][i] = keep_if(m < kb ? -v : v, ok);
-      }
-    }
+  // LU: A operands, in registers for all tiles of the wave: -L below the
+  // diagonal blocks, -[L21; C_j U^-1] (rows of T are final positions)
+  V4<TW> lb[QR ? 1 : NB][NB], lr[QR ? 1 : NRT][NB];
   // (in flight over the inverses where the registers hold them beside those;
   // where they do not, the inverses stay in LDS too)
   constexpr bool LATE = NB >= 3;
-  auto load_rest = [&] {
+  TW* const x = sm.x[w];
+  auto clear_tile = [&] {   // (the padding slots stay zero)
 #pragma unroll
-    for (int rt = 0; rt < NRT; ++rt) {
-      const int q = 16 * rt + cl;
+    for (int h = 0; h < (16 * XLD + 63) / 64; ++h)
+      if (lane + 64 * h < 16 * XLD) x[lane + 64 * h] = TW(0);
+  };
+  if constexpr (QR) {
+    // the reflectors (unit lower trapezoid; R above it left out) by whole
+    // columns, and the border rows of C_j R^-1
+    clear_tile();
+    for (int e = threadIdx.x; e < 16 * NB * Lds::CLD; e += 64 * NW) sm.cb[e] = TW(0);
+    constexpr int CH = 4;   // columns in flight
+    for (int k0 = w; k0 < 16 * NB; k0 += CH * NW) {
+      TW t0[CH], t1[CH];
 #pragma unroll
-      for (int kb = 0; kb < NB; ++kb)
+      for (int q = 0; q < CH; ++q) {
+        const unsigned k = k0 + q * NW, kc = k < unsigned(n) ? k : 0;
+        t0[q] = gload(Tj, kc * unsigned(n2) + unsigned(lane < n ? lane : 0));
+        t1[q] = gload(Tj, kc * unsigned(n2) + unsigned(n + (lane < n ? lane : 0)));
+      }
+#pragma unroll
+      for (int q = 0; q < CH; ++q) {
+        const int k = k0 + q * NW;
+        if (k < 16 * NB && lane < NT) {
+          TW* const vk = sm.v + k * Lds::VLD;
+          vk[lane] = k < n && lane <= k ? (lane == k ? TW(1) : TW(0)) : keep_if(t0[q], k < n && lane < n);
+          vk[NT + lane] = keep_if(t1[q], k < n && lane < n);
+        }
+      }
+    }
+    __syncthreads();
+    const int b0 = n & 15;   // the border rows' first row in their tiles
+    for (int k = threadIdx.x; k < n; k += 64 * NW)
+      for (int i = 0; i < nr; ++i) sm.cb[k * Lds::CLD + b0 + i] = -Cm[j * rn + size_t(k) * nr + i];
+    // T of I - V T V^T = H_0 .. H_15 per 16-column block, from the products
+    // V^T V (dlarft's recurrence T(0:c, c) = -tau_c T(0:c, 0:c) (V^T V)(0:c, c)),
+    // row lane % 16 of block lane / 16 in a lane's registers; stored negated,
+    // so that H^T x = x + V (-T^T (V^T x))
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      if (b % NW == w) {
+        V4<TW> acc{TW(0), TW(0), TW(0), TW(0)};
+#pragma unroll
+        for (int t = b; t < 2 * NB; ++t) {
+          const V4<TW> vt = ld4(sm.v + (16 * b + cl) * Lds::VLD + 16 * t, g);
+          acc = mfma4<TW>(vt, vt, acc);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sm.inv[b][cl * DLD + kro<TW>(g, i)] = acc[i];
+      }
+    lds_order();
+    if (lane < 16 * NB && (lane >> 4) % NW == w) {
+      TW* const blk = sm.inv[lane >> 4];
+      const int ri = lane & 15, c0 = lane & ~15;
+      TW y[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) {
+        TW t0 = TW(0), t1 = TW(0);
+#pragma unroll
+        for (int k = 0; k < c; k += 2) {
+          const V2<TW> g2 = *reinterpret_cast<const V2<TW>*>(blk + c * DLD + k);
+          t0 = fma(g2.x, y[k], t0);
+          if (k + 1 < c) t1 = fma(g2.y, y[k + 1], t1);
+        }
+        const TW tau = keep_if(gload(Tj, unsigned(n2) * unsigned(n) + unsigned(c0 + c < n ? c0 + c : 0)), c0 + c < n);
+        y[c] = ri == c ? tau : ri < c ? -tau * (t0 + t1) : TW(0);
+        if (c % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+      lds_order();
+#pragma unroll
+      for (int c = 0; c < 16; ++c) blk[c * DLD + ri] = -y[c];
+    }
+    __syncthreads();   // V, T and the border rows in place
+  } else {
+#pragma unroll
+    for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+      for (int m = 0; m <= kb; ++m) {
+        if (m == kb && kb % NW != w) continue;   // diagonal blocks: this wave's only
+        const int r = 16 * kb + cl;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int c = 16 * kb + kro<TW>(g, i);
-          const TW v = gload(Tj, unsigned(n + (q < n ? q : 0)) + unsigned(c < n ? c : 0) * unsigned(n2));
-          lr[rt][kb][i] = keep_if(-v, q < n && c < n);
+          const int c = 16 * m + kro<TW>(g, i);
+          const TW v = gload(Tj, (r < n ? r : 0) + unsigned(c < n ? c : 0) * unsigned(n2));
+          const bool ok = r < n && c < n && (m < kb || c < r);
+          lb[kb][m][i] = keep_if(m < kb ? -v : v, ok);
         }
-      if (16 * rt + 16 > n && 16 * rt < n + nr) {   // border rows of C_j U^-1
-        const TW* const Cj = Cm + j * rn;
-        const bool bord = q >= n && q < n + nr;
+      }
+    auto load_rest = [&] {
+#pragma unroll
+      for (int rt = 0; rt < NRT; ++rt) {
+        const int q = 16 * rt + cl;
 #pragma unroll
         for (int kb = 0; kb < NB; ++kb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int c = 16 * kb + kro<TW>(g, i);
-            const TW v = gload(Cj, unsigned(bord ? q - n : 0) + unsigned(c < n ? c : 0) * unsigned(nr));
-            lr[rt][kb][i] += keep_if(-v, bord && c < n);
+            const TW v = gload(Tj, unsigned(n + (q < n ? q : 0)) + unsigned(c < n ? c : 0) * unsigned(n2));
+            lr[rt][kb][i] = keep_if(-v, q < n && c < n);
           }
+        if (16 * rt + 16 > n && 16 * rt < n + nr) {   // border rows of C_j U^-1
+          const TW* const Cj = Cm + j * rn;
+          const bool bord = q >= n && q < n + nr;
+#pragma unroll
+          for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int c = 16 * kb + kro<TW>(g, i);
+              const TW v = gload(Cj, unsigned(bord ? q - n : 0) + unsigned(c < n ? c : 0) * unsigned(nr));
+              lr[rt][kb][i] += keep_if(-v, bord && c < n);
+            }
+        }
       }
-    }
-  };
-  if (!LATE) load_rest();
-  // this wave's diagonal blocks, row-major, then their inverses in place:
-  // column lane % 16 of block lane / 16 by forward substitution; rows beyond
-  // n are zero, their inverse rows identity
+    };
+    if (!LATE) load_rest();
+    // this wave's diagonal blocks, row-major, then their inverses in place:
+    // column lane % 16 of block lane / 16 by forward substitution; rows beyond
+    // n are zero, their inverse rows identity
 #pragma unroll
-  for (int kb = 0; kb < NB; ++kb)
-    if (kb % NW == w) {
+    for (int kb = 0; kb < NB; ++kb)
+      if (kb % NW == w) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sm.inv[kb][cl * DLD + kro<TW>(g, i)] = lb[kb][kb][i];
-    }
-  if (w == 0) {
-    if (lane < n2) sm.pos[lane] = pb0;
-    if (lane + 64 < n2) sm.pos[lane + 64] = pb1;
-  }
-  TW* const x = sm.x[w];
-#pragma unroll
-  for (int h = 0; h < (16 * XLD + 63) / 64; ++h)
-    if (lane + 64 * h < 16 * XLD) x[lane + 64 * h] = TW(0);   // the padding slots stay zero
-  lds_order();
-  if (lane < 16 * NB && (lane >> 4) % NW == w) {
-    TW* const blk = sm.inv[lane >> 4];
-    const int jj = lane & 15;
-    TW y[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) y[i] = TW(0);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const TW* li = blk + i * DLD;
-      TW t0 = TW(0), t1 = TW(0);
-#pragma unroll
-      for (int k = 0; k < i; k += 2) {
-        const V2<TW> l2 = *reinterpret_cast<const V2<TW>*>(li + k);
-        // (entries 4m, 4m + 2 and 4m + 1, 4m + 3 in two chains)
-        t0 = fma(l2.x, y[k], t0);
-        t1 = fma(l2.y, y[k + 1], t1);
+        for (int i = 0; i < 4; ++i) sm.inv[kb][cl * DLD + kro<TW>(g, i)] = lb[kb][kb][i];
       }
-      y[i] = jj == i ? TW(1) : -(t0 + t1);
-      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // (not all rows' reads at once)
+    if (w == 0) {
+      if (lane < n2) sm.pos[lane] = pb0;
+      if (lane + 64 < n2) sm.pos[lane + 64] = pb1;
     }
-    // every lane has read its block's rows (reads precede these writes in this wave)
+    clear_tile();
     lds_order();
+    if (lane < 16 * NB && (lane >> 4) % NW == w) {
+      TW* const blk = sm.inv[lane >> 4];
+      const int jj = lane & 15;
+      TW y[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) blk[i * DLD + jj] = y[i];
+      for (int i = 0; i < 16; ++i) y[i] = TW(0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const TW* li = blk + i * DLD;
+        TW t0 = TW(0), t1 = TW(0);
+#pragma unroll
+        for (int k = 0; k < i; k += 2) {
+          const V2<TW> l2 = *reinterpret_cast<const V2<TW>*>(li + k);
+          // (entries 4m, 4m + 2 and 4m + 1, 4m + 3 in two chains)
+          t0 = fma(l2.x, y[k], t0);
+          t1 = fma(l2.y, y[k + 1], t1);
+        }
+        y[i] = jj == i ? TW(1) : -(t0 + t1);
+        if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // (not all rows' reads at once)
+      }
+      // every lane has read its block's rows (reads precede these writes in this wave)
+      lds_order();
+#pragma unroll
+      for (int i = 0; i < 16; ++i) blk[i * DLD + jj] = y[i];
+    }
+    __syncthreads();   // the inverses and the row positions in place
+    if (LATE) load_rest();
   }
-  __syncthreads();   // the inverses and the row positions in place
-  if (LATE) load_rest();
   auto inverse = [&](int kb) { return ld4(&sm.inv[kb][cl * DLD], g); };
-  if (!LATE) {
+  if constexpr (!LATE && !QR) {
 #pragma unroll
     for (int kb = 0; kb < NB; ++kb) lb[kb][kb] = inverse(kb);
   }
@@ -820,7 +907,7 @@ __device__ __forceinline__ void pair_rhs_body(FactorArgs<TS, TW> const& a, int p
 #pragma unroll
   for (int h = 0; h < H; ++h) {
     const unsigned e = lane + 64 * h, col = (e * rcp) >> 16, row = min(e - col * n, unsigned(n) - 1);
-    const unsigned q0 = sm.pos[row], q1 = sm.pos[n + row];
+    const unsigned q0 = QR ? row : sm.pos[row], q1 = QR ? n + row : sm.pos[n + row];
     slot[h] = (col * XLD + (q0 < unsigned(n) ? q0 : NT + q0 - n)) | (col * XLD + (q1 < unsigned(n) ? q1 : NT + q1 - n)) << 16;
   }
 
@@ -863,43 +950,89 @@ __device__ __forceinline__ void pair_rhs_body(FactorArgs<TS, TW> const& a, int p
     if (t + NW < ntiles) load_tile(t + NW, 0);
     lds_order();
     const TW* const xc = x + cl * XLD;
-    // U12 = L11^-1 X_top by 16-row blocks: u_kb = inv(L_kk) (X_kb - sum_{m<kb}
-    // L_km u_m).  A block of U12 in the accumulator layout is the B operand
-    // layout of the next products as it stands.
     V4<TW> u[NB];
+    if constexpr (QR) {
+      // H^T x = x + V (-T^T (V^T x)), a block of 16 reflectors at a time, the
+      // tile's rows in registers in the B operand layout throughout
+      V4<TW> z[NRT];
 #pragma unroll
-    for (int kb = 0; kb < NB; ++kb) {
-      V4<TW> acc = ld4(xc + 16 * kb, g);
+      for (int t = 0; t < NB; ++t) u[t] = ld4(xc + 16 * t, g);
 #pragma unroll
-      for (int mb = 0; mb < kb; ++mb) acc = mfma4<TW>(lb[kb][mb], u[mb], acc);
-      u[kb] = mfma4<TW>(LATE ? inverse(kb) : lb[kb][kb], acc, V4<TW>{TW(0), TW(0), TW(0), TW(0)});
-    }
-    // X_rest' = X_rest - [L21; C_j U^-1] U12, ZT tiles' chains side by side,
-    // back to their slots
-    constexpr int ZT = NB == 3 && sizeof(TW) == 8 ? 2 : NRT;
+      for (int t = 0; t < NRT; ++t) z[t] = ld4(xc + NT + 16 * t, g);
 #pragma unroll
-    for (int r0 = 0; r0 < NRT; r0 += ZT) {
-      V4<TW> z[ZT];
+      for (int b = 0; b < NB; ++b) {
+        V4<TW> acc[2];   // V^T x in two chains: top and rest rows
+        acc[0] = acc[1] = V4<TW>{TW(0), TW(0), TW(0), TW(0)};
 #pragma unroll
-      for (int rt = 0; rt < ZT; ++rt)
-        if (r0 + rt < NRT) z[rt] = ld4(xc + NT + 16 * (r0 + rt), g);
+        for (int t = 0; t < NB; ++t) {
+          if (t >= b) acc[0] = mfma4<TW>(ld4(sm.v + (16 * b + cl) * Lds::VLD + 16 * t, g), u[t], acc[0]);
+          acc[1] = mfma4<TW>(ld4(sm.v + (16 * b + cl) * Lds::VLD + NT + 16 * t, g), z[t], acc[1]);
+        }
+        const V4<TW> y = mfma4<TW>(ld4(&sm.inv[b][cl * DLD], g), acc[0] + acc[1], V4<TW>{TW(0), TW(0), TW(0), TW(0)});
 #pragma unroll
-      for (int kb = 0; kb < NB; ++kb)
+        for (int i = 0; i < 4; ++i) {
+          const TW* const vk = sm.v + (16 * b + kro<TW>(g, i)) * Lds::VLD + cl;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int rt = 0; rt < ZT; ++rt)
-            if (r0 + rt < NRT) z[rt] = mfma1(lr[r0 + rt < NRT ? r0 + rt : 0][kb][i], u[kb][i], z[rt]);
-#pragma unroll
-      for (int rt = 0; rt < ZT; ++rt)
-        if (r0 + rt < NRT) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int q = 16 * (r0 + rt) + kro<TW>(g, i);
-            x[cl * XLD + NT + q] = q < n + nr ? z[rt][i] : TW(0);
+          for (int t = 0; t < NB; ++t) {
+            if (t >= b) u[t] = mfma1(vk[16 * t], y[i], u[t]);
+            z[t] = mfma1(vk[NT + 16 * t], y[i], z[t]);
           }
         }
-      if (ZT < NRT) __builtin_amdgcn_sched_barrier(0);
+      }
+      // the border rows lose the final top rows
+#pragma unroll
+      for (int t = 0; t < NRT; ++t) {
+        const int o = 16 * t + 16 > n && 16 * t < n + nr ? 16 * (t - n / 16) : -1;
+        if (o >= 0) {
+#pragma unroll
+          for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) z[t] = mfma1(sm.cb[(16 * kb + kro<TW>(g, i)) * Lds::CLD + o + cl], u[kb][i], z[t]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int q = 16 * t + kro<TW>(g, i);
+          x[cl * XLD + NT + q] = q < n + nr ? z[t][i] : TW(0);
+        }
+      }
+    } else {
+      // U12 = L11^-1 X_top by 16-row blocks: u_kb = inv(L_kk) (X_kb - sum_{m<kb}
+      // L_km u_m).  A block of U12 in the accumulator layout is the B operand
+      // layout of the next products as it stands.
+#pragma unroll
+      for (int kb = 0; kb < NB; ++kb) {
+        V4<TW> acc = ld4(xc + 16 * kb, g);
+#pragma unroll
+        for (int mb = 0; mb < kb; ++mb) acc = mfma4<TW>(lb[kb][mb], u[mb], acc);
+        u[kb] = mfma4<TW>(LATE ? inverse(kb) : lb[kb][kb], acc, V4<TW>{TW(0), TW(0), TW(0), TW(0)});
+      }
+      // X_rest' = X_rest - [L21; C_j U^-1] U12, ZT tiles' chains side by side,
+      // back to their slots
+      constexpr int ZT = NB == 3 && sizeof(TW) == 8 ? 2 : NRT;
+#pragma unroll
+      for (int r0 = 0; r0 < NRT; r0 += ZT) {
+        V4<TW> z[ZT];
+#pragma unroll
+        for (int rt = 0; rt < ZT; ++rt)
+          if (r0 + rt < NRT) z[rt] = ld4(xc + NT + 16 * (r0 + rt), g);
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int rt = 0; rt < ZT; ++rt)
+              if (r0 + rt < NRT) z[rt] = mfma1(lr[r0 + rt < NRT ? r0 + rt : 0][kb][i], u[kb][i], z[rt]);
+#pragma unroll
+        for (int rt = 0; rt < ZT; ++rt)
+          if (r0 + rt < NRT) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int q = 16 * (r0 + rt) + kro<TW>(g, i);
+              x[cl * XLD + NT + q] = q < n + nr ? z[rt][i] : TW(0);
+            }
+          }
+        if (ZT < NRT) __builtin_amdgcn_sched_barrier(0);
+      }
     }
     // pivot rows -> block j, reduced rows -> block jp, through the tile's
     // place in LDS as whole runs
@@ -969,12 +1102,23 @@ constexpr int rhs_waves(int nb, size_t elem) { return elem == 8 ? (nb <= 3 ? 2 :
 
 template <typename TS, typename TW, int NB, int NRT, int NW>
 __global__ void __launch_bounds__(64 * NW, rhs_waves(NB, sizeof(TW))) pair_rhs_mfma_kernel(FactorArgs<TS, TW> a) {
-  pair_rhs_body<TS, TW, NB, NRT, NW>(a, blockIdx.x);
+  pair_rhs_body<TS, TW, NB, NRT, NW, false>(a, blockIdx.x);
 }
 template <typename TS, typename TW, int NB, int NRT, int NW>
 __global__ void __launch_bounds__(64 * NW, rhs_waves(NB, sizeof(TW))) pair_rhs_mfma_batched(BatchTable<FactorArgs<TS, TW>> t) {
   const int e = t.entry[blockIdx.x];
-  pair_rhs_body<TS, TW, NB, NRT, NW>(t.args[e], int(blockIdx.x) - t.first[e]);
+  pair_rhs_body<TS, TW, NB, NRT, NW, false>(t.args[e], int(blockIdx.x) - t.first[e]);
+}
+
+constexpr int qr_rhs_waves(int nb, size_t elem) { return elem == 8 ? (nb <= 3 ? 2 : 1) : nb <= 2 ? 4 : nb == 3 ? 3 : 2; }
+template <typename TS, typename TW, int NB, int NRT, int NW>
+__global__ void __launch_bounds__(64 * NW, qr_rhs_waves(NB, sizeof(TW))) pair_qr_rhs_kernel(FactorArgs<TS, TW> a) {
+  pair_rhs_body<TS, TW, NB, NRT, NW, true>(a, blockIdx.x);
+}
+template <typename TS, typename TW, int NB, int NRT, int NW>
+__global__ void __launch_bounds__(64 * NW, qr_rhs_waves(NB, sizeof(TW))) pair_qr_rhs_batched(BatchTable<FactorArgs<TS, TW>> t) {
+  const int e = t.entry[blockIdx.x];
+  pair_rhs_body<TS, TW, NB, NRT, NW, true>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
 
 // Waves per pair in the right-hand kernel: two (each holds the operands of L,
@@ -1005,15 +1149,13 @@ template <int V, typename TS, typename TW>
 void launch_pair(FactorArgs<TS, TW> const& a, hipStream_t st) {
   constexpr int NB = V + 1, RS = V == 3 ? 3 : 2, NRT = V + 2;   // NRT: tiles of the n + nr rest rows
   const dim3 pairs(a.npairs);
-  const auto by_waves = [&] { hipLaunchKernelGGL((pair_lu_tw_kernel<TS, TW, NB, RS>), pairs, dim3(64 * NB), 0, st, a); };
-  const auto by_one = [&] { hipLaunchKernelGGL((pair_lu_t_kernel<TS, TW, NB, RS, kNrB>), pairs, dim3(64), 0, st, a); };
-  if constexpr (panel_by_waves_always(NB, sizeof(TW))) {
-    by_waves();
-  } else if constexpr (panel_by_waves_few(NB, sizeof(TW))) {
-    if (a.npairs <= kWavesPairs && a.pstat == nullptr) by_waves();
-    else by_one();
-  } else {
-    by_one();
+  bool by_waves = panel_by_waves_always(NB, sizeof(TW));
+  if constexpr (panel_by_waves_few(NB, sizeof(TW))) by_waves = a.npairs <= kWavesPairs && a.pstat == nullptr;
+  if constexpr (panel_by_waves_always(NB, sizeof(TW)) || panel_by_waves_few(NB, sizeof(TW))) {
+    if (by_waves) hipLaunchKernelGGL((pair_lu_tw_kernel<TS, TW, NB, RS>), pairs, dim3(64 * NB), 0, st, a);
+  }
+  if constexpr (!panel_by_waves_always(NB, sizeof(TW))) {
+    if (!by_waves) hipLaunchKernelGGL((pair_lu_t_kernel<TS, TW, NB, RS, kNrB>), pairs, dim3(64), 0, st, a);
   }
   if (a.npairs <= kFewPairs) hipLaunchKernelGGL((pair_rhs_mfma_kernel<TS, TW, NB, NRT, kRhsWavesFew>), pairs, dim3(64 * kRhsWavesFew), 0, st, a);
   else hipLaunchKernelGGL((pair_rhs_mfma_kernel<TS, TW, NB, NRT, kRhsWaves>), pairs, dim3(64 * kRhsWaves), 0, st, a);
@@ -1058,6 +1200,32 @@ bool launch_pair_lu_mfma_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nb
   *err = hipGetLastError();
   return true;
 }
+
+template <typename TS, typename TW>
+void launch_pair_qr_rhs(FactorArgs<TS, TW> const& a, hipStream_t st) {
+  const dim3 g(a.npairs);
+  switch (mfma_variant(a.n, a.nr, a.nx)) {
+    case 1: hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 2, 3, 2>), g, dim3(128), 0, st, a); break;
+    case 2: hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 3, 4, 2>), g, dim3(128), 0, st, a); break;
+    case 3: hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 4, 5, 2>), g, dim3(128), 0, st, a); break;
+  }
+}
+template <typename TS, typename TW>
+void launch_pair_qr_rhs_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, int n, int nr, int nx, hipStream_t st) {
+  const dim3 g(nblocks);
+  switch (mfma_variant(n, nr, nx)) {
+    case 1: hipLaunchKernelGGL((pair_qr_rhs_batched<TS, TW, 2, 3, 2>), g, dim3(128), 0, st, t); break;
+    case 2: hipLaunchKernelGGL((pair_qr_rhs_batched<TS, TW, 3, 4, 2>), g, dim3(128), 0, st, t); break;
+    case 3: hipLaunchKernelGGL((pair_qr_rhs_batched<TS, TW, 4, 5, 2>), g, dim3(128), 0, st, t); break;
+  }
+}
+#define BCR_QR_RHS(TS, TW)                                                                                       \
+  template void launch_pair_qr_rhs<TS, TW>(FactorArgs<TS, TW> const&, hipStream_t);                              \
+  template void launch_pair_qr_rhs_batched<TS, TW>(BatchTable<FactorArgs<TS, TW>> const&, int, int, int, int, hipStream_t);
+BCR_QR_RHS(float, float)
+BCR_QR_RHS(double, float)
+BCR_QR_RHS(double, double)
+#undef BCR_QR_RHS
 
 template bool launch_pair_lu_mfma<float, float>(FactorArgs<float, float> const&, hipStream_t, hipError_t*);
 template bool launch_pair_lu_mfma<double, float>(FactorArgs<double, float> const&, hipStream_t, hipError_t*);

@@ -11,7 +11,9 @@
 //     (dlarfg), its application to the columns c+1..n-1 of T, and the
 //     elimination of row c from the border rows (l = C[i][c] / R[c][c]);
 //     one barrier per column (see the step loop).
-//  2. The right-hand columns [col jp | col jpp | xb] (2n + nx of them), in
+//  2. Beyond n = 16 a second launch (launch_pair_qr_rhs, blocks of 16
+//     reflectors on the matrix cores).  Otherwise the right-hand columns
+//     [col jp | col jpp | xb] (2n + nx of them), in
 //     chunks of CW columns staged in LDS next to T: every column goes
 //     through H_0 .. H_{n-1} and the border eliminations on its own, so a
 //     group of G lanes (4 to 16: as many as keep every column of the chunk
@@ -134,7 +136,8 @@ __device__ __forceinline__ void zero_rows(TW* dst, int r0, int r1, int cols, int
   for (int e = tid; e < h * cols; e += 256) dst[r0 + e % h + (e / h) * ld] = TW(0);
 }
 
-template <typename TS, typename TW, int METHOD>
+// PANEL: phase 1 only (launch_pair_qr_rhs does the right-hand columns)
+template <typename TS, typename TW, int METHOD, bool PANEL>
 __device__ __forceinline__ void pair_qr_body(FactorArgs<TS, TW> const& a, int cw, int p) {
   extern __shared__ __align__(16) unsigned char qr_smem[];
   __shared__ TW s_vn1[64], s_vn2[64], s_tau[64];
@@ -278,7 +281,7 @@ __device__ __forceinline__ void pair_qr_body(FactorArgs<TS, TW> const& a, int cw
   // ---- phase 2: the right-hand columns, CW at a time ----------------------------
   // column g of [col jp | col jpp | xb]: region 0 (g < n) D_jp on top, C_jp in
   // the border rows; region 1 (g < 2n) E_j at the bottom; region 2 B_jp, B_j
-  for (int g0 = 0; g0 < Wr; g0 += cw) {
+  for (int g0 = 0; !PANEL && g0 < Wr; g0 += cw) {
     const int w = min(cw, Wr - g0);
     {
       const int a0 = g0, a1 = min(g0 + w, n);   // region 0 columns
@@ -369,15 +372,15 @@ __device__ __forceinline__ void pair_qr_body(FactorArgs<TS, TW> const& a, int cw
   }
 }
 
-template <typename TS, typename TW, int METHOD>
+template <typename TS, typename TW, int METHOD, bool PANEL>
 __global__ void __launch_bounds__(256) pair_qr_kernel(FactorArgs<TS, TW> a, int cw) {
-  pair_qr_body<TS, TW, METHOD>(a, cw, blockIdx.x);
+  pair_qr_body<TS, TW, METHOD, PANEL>(a, cw, blockIdx.x);
 }
 
-template <typename TS, typename TW, int METHOD>
+template <typename TS, typename TW, int METHOD, bool PANEL>
 __global__ void __launch_bounds__(256) pair_qr_batched(BatchTable<FactorArgs<TS, TW>> t, int cw) {
   const int e = t.entry[blockIdx.x];
-  pair_qr_body<TS, TW, METHOD>(t.args[e], cw, int(blockIdx.x) - t.first[e]);
+  pair_qr_body<TS, TW, METHOD, PANEL>(t.args[e], cw, int(blockIdx.x) - t.first[e]);
 }
 
 }  // namespace
@@ -401,14 +404,27 @@ bool pair_qr_plan(int n, int nr, int nx, size_t elem, size_t lds_limit, int* cw,
   return false;
 }
 
+// Two launches, the right-hand columns on the matrix cores, beyond n = 16:
+// one FP64 level of 10000 and of a few pairs takes 2482 / 190 us at n = 32
+// with one launch (the LDS chunks and their column groups bound it), 1456 /
+// 126 with two; n = 64, 2000 pairs: 5534 / 672 against 1429 / 250.  Smaller blocks leave most of a 16 x 16
+// tile empty (n = 16: 502 / 50 us against 540 / 45, n = 8: 308 / 34 against
+// 454 / 40) and stay with one.
+static bool split_pair(int n, int nr, int nx) { return n > 16 && pair_lu_mfma_fits(n, nr, nx); }
+
 template <typename TS, typename TW>
 bool launch_pair_qr(int method, FactorArgs<TS, TW> const& a, size_t lds_limit, hipStream_t st, hipError_t* err) {
-  int cw = 0;
-  size_t bytes = 0;
+  int cw;
+  size_t bytes;
   if (method == kLU || !pair_qr_plan(a.n, a.nr, a.nx, sizeof(TW), lds_limit, &cw, &bytes)) return false;
   const dim3 g(a.npairs), b(256);
-  if (method == kQR) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQR>), g, b, bytes, st, a, cw);
-  else hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQRP>), g, b, bytes, st, a, cw);
+  const bool two = split_pair(a.n, a.nr, a.nx);
+  if (two) bytes = size_t((2 * a.n + a.nr) | 1) * a.n * sizeof(TW);
+  if (two && method == kQR) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQR, true>), g, b, bytes, st, a, 0);
+  else if (two) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQRP, true>), g, b, bytes, st, a, 0);
+  else if (method == kQR) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQR, false>), g, b, bytes, st, a, cw);
+  else hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQRP, false>), g, b, bytes, st, a, cw);
+  if (two) launch_pair_qr_rhs(a, st);
   *err = hipGetLastError();
   return true;
 }
@@ -416,12 +432,17 @@ bool launch_pair_qr(int method, FactorArgs<TS, TW> const& a, size_t lds_limit, h
 template <typename TS, typename TW>
 bool launch_pair_qr_batched(int method, BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, int n, int nr, int nx,
                             size_t lds_limit, hipStream_t st, hipError_t* err) {
-  int cw = 0;
-  size_t bytes = 0;
+  int cw;
+  size_t bytes;
   if (method == kLU || !pair_qr_plan(n, nr, nx, sizeof(TW), lds_limit, &cw, &bytes)) return false;
   const dim3 g(nblocks), b(256);
-  if (method == kQR) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQR>), g, b, bytes, st, t, cw);
-  else hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQRP>), g, b, bytes, st, t, cw);
+  const bool two = split_pair(n, nr, nx);
+  if (two) bytes = size_t((2 * n + nr) | 1) * n * sizeof(TW);
+  if (two && method == kQR) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQR, true>), g, b, bytes, st, t, 0);
+  else if (two) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQRP, true>), g, b, bytes, st, t, 0);
+  else if (method == kQR) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQR, false>), g, b, bytes, st, t, cw);
+  else hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQRP, false>), g, b, bytes, st, t, cw);
+  if (two) launch_pair_qr_rhs_batched(t, nblocks, n, nr, nx, st);
   *err = hipGetLastError();
   return true;
 }

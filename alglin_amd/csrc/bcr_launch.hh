@@ -15,6 +15,10 @@ template <typename TA> struct MvArgs;
 bool pair_qr_plan(int n, int nr, int nx, size_t elem, size_t lds_limit, int* cw, size_t* bytes);
 template <typename TS, typename TW>
 bool launch_pair_qr(int method, FactorArgs<TS, TW> const& a, size_t lds_limit, hipStream_t st, hipError_t* err);
+// the right-hand columns of a QR pair whose panel is factored (shapes of
+// pair_lu_mfma_fits)
+template <typename TS, typename TW>
+void launch_pair_qr_rhs(FactorArgs<TS, TW> const& a, hipStream_t st);
 template <typename TS, typename TW>
 hipError_t launch_pair_generic(int method, FactorArgs<TS, TW> const& a, TW* gscratch, size_t lds_limit,
                                hipStream_t st);
