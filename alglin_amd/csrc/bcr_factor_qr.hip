@@ -6,7 +6,8 @@
 // [row jp; row j; border], columns [T = col j | col jp | col jpp | xb].  One
 // 256-thread workgroup per pair, in two phases:
 //
-//  1. The T panel [E_jp; D_j; C_j] (R x n) in LDS: per column c the pivot
+//  1. (For 16 < n <= 32 a wave with the columns in registers does this phase:
+//     pair_qr_wave_body.)  The T panel [E_jp; D_j; C_j] (R x n) in LDS: per column c the pivot
 //     column (QRP: largest partial norm, dlaqp2 downdating), the reflector
 //     (dlarfg), its application to the columns c+1..n-1 of T, and the
 //     elimination of row c from the border rows (l = C[i][c] / R[c][c]);
@@ -34,6 +35,7 @@
 
 #include "bcr_launch.hh"
 #include "bcr_batch_kernels.hh"
+#include "bcr_wave.hh"
 
 namespace bcr {
 namespace {
@@ -383,6 +385,235 @@ __global__ void __launch_bounds__(256) pair_qr_batched(BatchTable<FactorArgs<TS,
   pair_qr_body<TS, TW, METHOD, PANEL>(t.args[e], cw, int(blockIdx.x) - t.first[e]);
 }
 
+// The panel alone for n <= 32, one wave per pair with the columns in registers:
+// lane (column l % 32, half l / 32) holds the rows r = 2 k + l / 32 of its
+// column, so v^T x is a chain per lane and one exchange of halves, and the
+// column norms and the QRP downdating are one value per lane.  A step hands the
+// pivot column round through LDS (two lanes write it, every lane reads its
+// half), forms the reflector in every lane and stores the finished column; no
+// barrier, no exchange over more than two lanes except QRP's search.  Physical
+// columns stay in their lanes; logi is the logical one.  Steps come in four
+// groups of eight, rolled within a group (rows before the group's first are
+// left out at compile time).  The chain of a step bounds small levels.  Times
+// of one level of 10000 and of a few pairs, n = 32 FP64, QRP: workgroup kernel
+// above 1055 / 104 us, this one 367 / 45.
+template <typename TW>
+struct QrWaveLds {
+  static constexpr int LD = 2 * 32 + 8 + 1;      // odd: a column per lane reads conflict-free
+  alignas(16) TW panel[32 * LD];
+  alignas(16) TW v[2][32 + 4];                   // the pivot column by halves, border rows last
+};
+
+// s + the other half's s, the same bits in both halves
+__device__ __forceinline__ double half_sum(double s) {
+  const long long b = __double_as_longlong(s);
+  const auto lo = __builtin_amdgcn_permlane32_swap(unsigned(b & 0xffffffffu), unsigned(b & 0xffffffffu), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(unsigned(b >> 32), unsigned(b >> 32), false, false);
+  return __hiloint2double(int(hi[0]), int(lo[0])) + __hiloint2double(int(hi[1]), int(lo[1]));
+}
+__device__ __forceinline__ float half_sum(float s) {
+  const unsigned b = __float_as_uint(s);
+  const auto p = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+
+// the steps 8 G .. 8 G + 7 of the panel (those before n)
+template <int G, int METHOD, typename TW>
+__device__ __forceinline__ void qr_wave_steps(QrWaveLds<TW>& sm, TW (&x)[32], TW (&xb)[4], int& logi, TW& vn1, TW& vn2,
+                                              bool& singular, TW* Tj, TW* Cj, int n, int nr, int lane) {
+  if constexpr (G < 4) {
+    constexpr int K0 = 4 * G;
+    const int col = lane & 31, h = lane >> 5, n2 = 2 * n;
+    const TW tol3z = sqrt(TW(sizeof(TW) == 8 ? 2.220446049250313e-16 : 1.1920929e-07));
+    const int cend = min(8 * G + 8, n);
+    for (int c = 8 * G; c < cend; ++c) {
+      int who = c;
+      if constexpr (METHOD == kQRP) {
+        // the largest partial norm among logical columns c.., ties to the
+        // smaller logical index (LAPACK's idamax)
+        unsigned khi, klo;
+        wave::abs_key(vn1, khi, klo);
+        bool zero;
+        who = wave::argmax_pos<(sizeof(TW) > 4)>(lane < n && logi >= c, khi, klo, logi, lane, zero);
+        const int old = __builtin_amdgcn_readlane(logi, who);
+        logi = col == who ? c : logi == c ? old : logi;
+      }
+      const bool active = col < n && logi > c;
+      if (col == who) {
+#pragma unroll
+        for (int k = 0; k < 32; ++k) sm.v[h][k] = x[k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sm.v[h][32 + k] = xb[k];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      TW v[32], vb[4];
+#pragma unroll
+      for (int k = K0; k < 32; ++k) v[k] = sm.v[h][k];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) vb[k] = sm.v[h][32 + k];
+      const TW alpha = sm.v[c & 1][c >> 1];
+      const TW mine = sm.v[lane & 1][lane >> 1], mineb = sm.v[lane & 1][32 + ((lane >> 1) & 3)];   // row lane, border row lane
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      // the rows after c (dlarfg's x)
+#pragma unroll
+      for (int k = K0; k < K0 + 4; ++k) v[k] = keep_if(v[k], 2 * k + h > c);
+      TW s[4] = {TW(0), TW(0), TW(0), TW(0)};
+#pragma unroll
+      for (int k = K0; k < 32; ++k) s[k & 3] = fma(v[k], v[k], s[k & 3]);
+      const TW ss = half_sum((s[0] + s[1]) + (s[2] + s[3]));
+      TW tau = 0, scal = 1, beta = alpha;
+      if (ss != TW(0)) {
+        const TW nrm = sqrt(alpha * alpha + ss);
+        beta = alpha >= TW(0) ? -nrm : nrm;
+        tau = (beta - alpha) / beta;
+        scal = TW(1) / (alpha - beta);
+      }
+      const TW rinv = beta != TW(0) ? TW(1) / beta : TW(0);
+      singular = singular || beta == TW(0);
+#pragma unroll
+      for (int k = K0; k < 32; ++k) v[k] *= scal;
+#pragma unroll
+      for (int k = K0; k < K0 + 4; ++k) v[k] = 2 * k + h == c ? TW(1) : v[k];
+      // the finished column, a row per lane
+      TW* const Tc = Tj + size_t(c) * n2;
+      if (lane < n2) Tc[lane] = lane < c ? mine : lane == c ? beta : mine * scal;
+      if (lane < nr) Cj[size_t(c) * nr + lane] = mineb * rinv;
+      if (lane == 0) Tj[size_t(n2) * n + c] = tau;
+      // H_c on the columns after c, and their border rows lose row c
+#pragma unroll
+      for (int k = 0; k < 4; ++k) s[k] = TW(0);
+#pragma unroll
+      for (int k = K0; k < 32; ++k) s[k & 3] = fma(v[k], x[k], s[k & 3]);
+      const TW d = half_sum((s[0] + s[1]) + (s[2] + s[3]));
+      const TW w = active && tau != TW(0) ? d * tau : TW(0);
+#pragma unroll
+      for (int k = K0; k < 32; ++k) x[k] = fma(-v[k], w, x[k]);
+      TW nc = TW(0);
+#pragma unroll
+      for (int k = K0; k < K0 + 4; ++k) nc = 2 * k + h == c ? x[k] : nc;
+      nc = keep_if(half_sum(nc), active);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) xb[k] = fma(-(vb[k] * rinv), nc, xb[k]);
+      if constexpr (METHOD == kQRP) {
+        // dlaqp2 norm downdating (LAWN 176)
+        const bool down = active && vn1 != TW(0);
+        TW t = dev_abs(nc) / vn1;
+        t = TW(1) - t * t;
+        t = t < TW(0) ? TW(0) : t;
+        const TW qq = vn1 / vn2;
+        const bool again = down && t * qq * qq <= tol3z;
+        if (__ballot(again)) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) s[k] = TW(0);
+#pragma unroll
+          for (int k = K0; k < 32; ++k) {
+            const TW xk = k < K0 + 4 ? keep_if(x[k], 2 * k + h > c) : x[k];
+            s[k & 3] = fma(xk, xk, s[k & 3]);
+          }
+          const TW nv = sqrt(half_sum((s[0] + s[1]) + (s[2] + s[3])));
+          vn2 = again ? nv : vn2;
+          vn1 = again ? nv : down ? vn1 * sqrt(t) : vn1;
+        } else {
+          vn1 = down ? vn1 * sqrt(t) : vn1;
+        }
+      }
+    }
+    qr_wave_steps<G + 1, METHOD, TW>(sm, x, xb, logi, vn1, vn2, singular, Tj, Cj, n, nr, lane);
+  }
+}
+
+template <typename TS, typename TW, int METHOD>
+__device__ __forceinline__ void pair_qr_wave_body(FactorArgs<TS, TW> const& a, int p) {
+  constexpr int LD = QrWaveLds<TW>::LD;
+  __shared__ QrWaveLds<TW> sm;
+  if (p >= a.npairs) return;
+  const int lane = threadIdx.x & 63, col = lane & 31, h = lane >> 5;
+  const int n = a.n, nr = a.nr, n2 = 2 * n;   // n <= 32, nr <= 8
+  int j, jp, jpp;
+  pair_of_uniform(a, p, j, jp, jpp);
+  const size_t nn = size_t(n) * n, rn = size_t(nr) * n;
+  TW* const Tj = a.Tm + size_t(j) * tsize(n);
+  {
+    // E_jp over D_j over C_j, whole blocks as they lie, by column into LDS
+    // (e < 1024: exact through the reciprocals)
+    const TS *const Ejp = a.sE + jp * nn, *const Dj = a.sD + j * nn, *const Cs = a.sC + j * rn;
+    const TW* const pend_cur = a.Cpend + size_t(a.slot_cur) * (a.N + 1) * rn + j * rn;
+    const TW* const pend_prv = a.Cpend + size_t(a.slot_cur ^ 1) * (a.N + 1) * rn + j * rn;
+    const unsigned rcp = (65536u + unsigned(n) - 1) / unsigned(n);
+    const unsigned rcpr = nr > 0 ? (65536u + unsigned(nr) - 1) / unsigned(nr) : 0;
+    TS e1[16], d1[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const unsigned e = min(unsigned(lane + 64 * i), unsigned(n * n - 1));
+      e1[i] = gload(Ejp, e);
+      d1[i] = gload(Dj, e);
+    }
+    if (nr > 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned e = min(unsigned(lane + 64 * i), unsigned(nr * n - 1));
+        TW c = TW(gload(Cs, e));
+        if (!a.first) c += gload(pend_prv, e) + gload(pend_cur, e);
+        const unsigned k = (e * rcpr) >> 16;
+        if (lane + 64 * i < nr * n) sm.panel[k * LD + n2 + (e - k * nr)] = c;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const unsigned e = lane + 64 * i, k = (e * rcp) >> 16;
+      if (e < unsigned(n * n)) {
+        sm.panel[k * LD + (e - k * n)] = TW(e1[i]);
+        sm.panel[k * LD + n + (e - k * n)] = TW(d1[i]);
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  TW x[32], xb[4];
+  const TW* const pc = sm.panel + (col < n ? col : 0) * LD;
+#pragma unroll
+  for (int k = 0; k < 32; ++k) {
+    const int r = 2 * k + h;
+    x[k] = keep_if(pc[r < n2 ? r : 0], r < n2 && col < n);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = 2 * k + h;
+    xb[k] = keep_if(pc[i < nr ? n2 + i : 0], i < nr && col < n);
+  }
+  TW vn1 = TW(0), vn2 = TW(0);
+  if constexpr (METHOD == kQRP) {
+    TW s[4] = {TW(0), TW(0), TW(0), TW(0)};
+#pragma unroll
+    for (int k = 0; k < 32; ++k) s[k & 3] = fma(x[k], x[k], s[k & 3]);
+    vn1 = vn2 = sqrt(half_sum((s[0] + s[1]) + (s[2] + s[3])));
+  }
+  int logi = col;
+  bool singular = false;
+  qr_wave_steps<0, METHOD, TW>(sm, x, xb, logi, vn1, vn2, singular, Tj, a.C + j * rn, n, nr, lane);
+  if (singular && lane == 0) atomicOr(a.status, 1);
+  if constexpr (METHOD == kQRP) {
+    // permutation -> exchange list (BABD_BorderedCR.hxx:265-275): column i is
+    // at position logi of lane i; step i exchanges it with position i's
+    int mine = 0;
+    for (int i = 0; i < n; ++i) {
+      const int jj = __builtin_amdgcn_readlane(logi, i);
+      mine = lane == i ? jj : mine;
+      logi = col == i ? i : logi == i ? jj : logi;
+    }
+    if (lane < n) a.perm[size_t(j) * n + lane] = mine;
+  }
+}
+
+template <typename TS, typename TW, int METHOD>
+__global__ void __launch_bounds__(64, 2) pair_qr_wave_kernel(FactorArgs<TS, TW> a) {
+  pair_qr_wave_body<TS, TW, METHOD>(a, blockIdx.x);
+}
+template <typename TS, typename TW, int METHOD>
+__global__ void __launch_bounds__(64, 2) pair_qr_wave_batched(BatchTable<FactorArgs<TS, TW>> t) {
+  const int e = t.entry[blockIdx.x];
+  pair_qr_wave_body<TS, TW, METHOD>(t.args[e], int(blockIdx.x) - t.first[e]);
+}
+
 }  // namespace
 
 bool pair_qr_plan(int n, int nr, int nx, size_t elem, size_t lds_limit, int* cw, size_t* bytes) {
@@ -406,8 +637,8 @@ bool pair_qr_plan(int n, int nr, int nx, size_t elem, size_t lds_limit, int* cw,
 
 // Two launches, the right-hand columns on the matrix cores, beyond n = 16:
 // one FP64 level of 10000 and of a few pairs takes 2482 / 190 us at n = 32
-// with one launch (the LDS chunks and their column groups bound it), 1456 /
-// 126 with two; n = 64, 2000 pairs: 5534 / 672 against 1429 / 250.  Smaller blocks leave most of a 16 x 16
+// with one launch (the LDS chunks and their column groups bound it), 766 /
+// 66 with two; n = 64, 2000 pairs: 5534 / 672 against 1429 / 250.  Smaller blocks leave most of a 16 x 16
 // tile empty (n = 16: 502 / 50 us against 540 / 45, n = 8: 308 / 34 against
 // 454 / 40) and stay with one.
 static bool split_pair(int n, int nr, int nx) { return n > 16 && pair_lu_mfma_fits(n, nr, nx); }
@@ -420,7 +651,9 @@ bool launch_pair_qr(int method, FactorArgs<TS, TW> const& a, size_t lds_limit, h
   const dim3 g(a.npairs), b(256);
   const bool two = split_pair(a.n, a.nr, a.nx);
   if (two) bytes = size_t((2 * a.n + a.nr) | 1) * a.n * sizeof(TW);
-  if (two && method == kQR) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQR, true>), g, b, bytes, st, a, 0);
+  if (two && a.n <= 32 && method == kQR) hipLaunchKernelGGL((pair_qr_wave_kernel<TS, TW, kQR>), g, dim3(64), 0, st, a);
+  else if (two && a.n <= 32) hipLaunchKernelGGL((pair_qr_wave_kernel<TS, TW, kQRP>), g, dim3(64), 0, st, a);
+  else if (two && method == kQR) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQR, true>), g, b, bytes, st, a, 0);
   else if (two) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQRP, true>), g, b, bytes, st, a, 0);
   else if (method == kQR) hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQR, false>), g, b, bytes, st, a, cw);
   else hipLaunchKernelGGL((pair_qr_kernel<TS, TW, kQRP, false>), g, b, bytes, st, a, cw);
@@ -438,7 +671,9 @@ bool launch_pair_qr_batched(int method, BatchTable<FactorArgs<TS, TW>> const& t,
   const dim3 g(nblocks), b(256);
   const bool two = split_pair(n, nr, nx);
   if (two) bytes = size_t((2 * n + nr) | 1) * n * sizeof(TW);
-  if (two && method == kQR) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQR, true>), g, b, bytes, st, t, 0);
+  if (two && n <= 32 && method == kQR) hipLaunchKernelGGL((pair_qr_wave_batched<TS, TW, kQR>), g, dim3(64), 0, st, t);
+  else if (two && n <= 32) hipLaunchKernelGGL((pair_qr_wave_batched<TS, TW, kQRP>), g, dim3(64), 0, st, t);
+  else if (two && method == kQR) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQR, true>), g, b, bytes, st, t, 0);
   else if (two) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQRP, true>), g, b, bytes, st, t, 0);
   else if (method == kQR) hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQR, false>), g, b, bytes, st, t, cw);
   else hipLaunchKernelGGL((pair_qr_batched<TS, TW, kQRP, false>), g, b, bytes, st, t, cw);
