@@ -590,6 +590,8 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
       if (method_ == kLU && sweep_fast_ &&
           ((sweep_mfma(n, nrhs, a.npairs) && launch_sweep_lu_mfma(true, a, st_, &e)) || launch_sweep_lu_fast(true, a, st_, &e) || launch_sweep_lu_stream(true, a, st_, &e)))
         hip_check(e, "forward_fast");
+      else if (method_ != kLU && sweep_fast_ && launch_forward_qr(a, st_, &e))
+        hip_check(e, "forward_qr");
       else hip_check(launch_forward(method_, a, st_), "forward");
     });
   }

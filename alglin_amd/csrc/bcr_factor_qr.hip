@@ -404,17 +404,9 @@ struct QrWaveLds {
   alignas(16) TW v[2][32 + 4];                   // the pivot column by halves, border rows last
 };
 
-// s + the other half's s, the same bits in both halves
-__device__ __forceinline__ double half_sum(double s) {
-  const long long b = __double_as_longlong(s);
-  const auto lo = __builtin_amdgcn_permlane32_swap(unsigned(b & 0xffffffffu), unsigned(b & 0xffffffffu), false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap(unsigned(b >> 32), unsigned(b >> 32), false, false);
-  return __hiloint2double(int(hi[0]), int(lo[0])) + __hiloint2double(int(hi[1]), int(lo[1]));
-}
-__device__ __forceinline__ float half_sum(float s) {
-  const unsigned b = __float_as_uint(s);
-  const auto p = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+template <typename TW>
+__device__ __forceinline__ TW sum8(TW const (&s)[8]) {
+  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 }
 
 // the steps 8 G .. 8 G + 7 of the panel (those before n)
@@ -457,10 +449,10 @@ __device__ __forceinline__ void qr_wave_steps(QrWaveLds<TW>& sm, TW (&x)[32], TW
       // the rows after c (dlarfg's x)
 #pragma unroll
       for (int k = K0; k < K0 + 4; ++k) v[k] = keep_if(v[k], 2 * k + h > c);
-      TW s[4] = {TW(0), TW(0), TW(0), TW(0)};
+      TW s[8] = {TW(0), TW(0), TW(0), TW(0), TW(0), TW(0), TW(0), TW(0)};
 #pragma unroll
-      for (int k = K0; k < 32; ++k) s[k & 3] = fma(v[k], v[k], s[k & 3]);
-      const TW ss = half_sum((s[0] + s[1]) + (s[2] + s[3]));
+      for (int k = K0; k < 32; ++k) s[k & 7] = fma(v[k], v[k], s[k & 7]);
+      const TW ss = wave::swap_add<false>(sum8(s));
       TW tau = 0, scal = 1, beta = alpha;
       if (ss != TW(0)) {
         const TW nrm = sqrt(alpha * alpha + ss);
@@ -481,17 +473,17 @@ __device__ __forceinline__ void qr_wave_steps(QrWaveLds<TW>& sm, TW (&x)[32], TW
       if (lane == 0) Tj[size_t(n2) * n + c] = tau;
       // H_c on the columns after c, and their border rows lose row c
 #pragma unroll
-      for (int k = 0; k < 4; ++k) s[k] = TW(0);
+      for (int k = 0; k < 8; ++k) s[k] = TW(0);
 #pragma unroll
-      for (int k = K0; k < 32; ++k) s[k & 3] = fma(v[k], x[k], s[k & 3]);
-      const TW d = half_sum((s[0] + s[1]) + (s[2] + s[3]));
+      for (int k = K0; k < 32; ++k) s[k & 7] = fma(v[k], x[k], s[k & 7]);
+      const TW d = wave::swap_add<false>(sum8(s));
       const TW w = active && tau != TW(0) ? d * tau : TW(0);
 #pragma unroll
       for (int k = K0; k < 32; ++k) x[k] = fma(-v[k], w, x[k]);
       TW nc = TW(0);
 #pragma unroll
       for (int k = K0; k < K0 + 4; ++k) nc = 2 * k + h == c ? x[k] : nc;
-      nc = keep_if(half_sum(nc), active);
+      nc = keep_if(wave::swap_add<false>(nc), active);
 #pragma unroll
       for (int k = 0; k < 4; ++k) xb[k] = fma(-(vb[k] * rinv), nc, xb[k]);
       if constexpr (METHOD == kQRP) {
@@ -504,13 +496,13 @@ __device__ __forceinline__ void qr_wave_steps(QrWaveLds<TW>& sm, TW (&x)[32], TW
         const bool again = down && t * qq * qq <= tol3z;
         if (__ballot(again)) {
 #pragma unroll
-          for (int k = 0; k < 4; ++k) s[k] = TW(0);
+          for (int k = 0; k < 8; ++k) s[k] = TW(0);
 #pragma unroll
           for (int k = K0; k < 32; ++k) {
             const TW xk = k < K0 + 4 ? keep_if(x[k], 2 * k + h > c) : x[k];
-            s[k & 3] = fma(xk, xk, s[k & 3]);
+            s[k & 7] = fma(xk, xk, s[k & 7]);
           }
-          const TW nv = sqrt(half_sum((s[0] + s[1]) + (s[2] + s[3])));
+          const TW nv = sqrt(wave::swap_add<false>(sum8(s)));
           vn2 = again ? nv : vn2;
           vn1 = again ? nv : down ? vn1 * sqrt(t) : vn1;
         } else {
@@ -582,10 +574,10 @@ __device__ __forceinline__ void pair_qr_wave_body(FactorArgs<TS, TW> const& a, i
   }
   TW vn1 = TW(0), vn2 = TW(0);
   if constexpr (METHOD == kQRP) {
-    TW s[4] = {TW(0), TW(0), TW(0), TW(0)};
+    TW s[8] = {TW(0), TW(0), TW(0), TW(0), TW(0), TW(0), TW(0), TW(0)};
 #pragma unroll
-    for (int k = 0; k < 32; ++k) s[k & 3] = fma(x[k], x[k], s[k & 3]);
-    vn1 = vn2 = sqrt(half_sum((s[0] + s[1]) + (s[2] + s[3])));
+    for (int k = 0; k < 32; ++k) s[k & 7] = fma(x[k], x[k], s[k & 7]);
+    vn1 = vn2 = sqrt(wave::swap_add<false>(sum8(s)));
   }
   int logi = col;
   bool singular = false;

@@ -13,6 +13,7 @@
 //            the lanes that hold them), then x_j = U^{-1} s bottom up.
 #include "bcr_launch.hh"
 #include "bcr_batch_kernels.hh"
+#include "bcr_wave.hh"
 
 namespace bcr {
 namespace {
@@ -110,6 +111,81 @@ __device__ __forceinline__ void forward_lu_stream_body(SolveArgs<TW, TX> a, int 
         for (int i = 0; i < nr; ++i) {
           const double s = wsum(lane < n ? double(Cj[i + size_t(lane) * nr]) * double(x0[b]) : 0.0);
           if (lane == 0) a.Xpart[size_t(j) * nr * nrhs + i + size_t(q) * nr] = TX(-s);
+        }
+      }
+    }
+  }
+}
+
+// The forward sweep of a QR or QRP pair, x <- H_{n-1} .. H_0 x (ormqr 'L','T',
+// cc:962-971), in the same layout: rows l and l + 64 of [x_jp; x_j] in lane l
+// (ONE: 2n <= 64), the reflectors streamed kChunk columns at a time, v^T x as a
+// wave sum.  The chain of the n sums bounds a small level (n = 32 FP64: a
+// workgroup with T in LDS and ds_bpermute sums 30 us, this 8); the first
+// level of 10000 pairs 253 -> 52 us (164 MB of factors).
+template <typename TW, typename TX, bool ONE, int QB>
+__device__ __forceinline__ void forward_qr_stream_body(SolveArgs<TW, TX> const& a, int bid) {
+  const int lane = threadIdx.x & 63;
+  const int p = bid * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));   // wave-uniform
+  if (p >= a.npairs) return;   // uniform over the wavefront
+  const int n = a.n, n2 = 2 * n, nr = a.nr, nrhs = a.nrhs;
+  int j, jp, jpp;
+  pair_of_uniform(a, p, j, jp, jpp);
+  const TW* Tj = a.Tm + size_t(j) * tsize(n);
+  const bool v0 = lane < n2, v1 = !ONE && lane + 64 < n2;
+  const int r0c = v0 ? lane : 0, r1c = v1 ? lane + 64 : 0;
+  TW t0[kChunk], t1[ONE ? 1 : kChunk];
+  auto load_chunk = [&](int c0) {
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) {
+      const unsigned cc = unsigned(c0 + i < n ? c0 + i : 0) * n2;
+      t0[i] = gload(Tj, r0c + cc);
+      if constexpr (!ONE) t1[i] = gload(Tj, r1c + cc);
+    }
+  };
+  load_chunk(0);
+  const TW taul = gload(Tj, unsigned(n2) * n + unsigned(lane < n ? lane : 0));   // tau_c in lane c
+  const size_t in0 = r0c < n ? size_t(jp) * n + r0c : size_t(j) * n + (r0c - n);
+  const size_t out0 = r0c < n ? size_t(j) * n + r0c : size_t(jp) * n + (r0c - n);
+  // (row lane + 64 >= n always: 2n > 64 needs n > 32, and n <= 64)
+  const size_t in1 = size_t(j) * n + (r1c < n ? 0 : r1c - n), out1 = size_t(jp) * n + (r1c < n ? 0 : r1c - n);
+  const TW* Cj = a.C + size_t(j) * nr * n;
+  for (int q0 = 0; q0 < nrhs; q0 += QB) {
+    TX x0[QB], x1[QB];
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      const TX* x = a.x + size_t(q0 + b < nrhs ? q0 + b : nrhs - 1) * a.ldx;
+      x0[b] = v0 ? x[in0] : TX(0);
+      x1[b] = v1 ? x[in1] : TX(0);
+    }
+    for (int c0 = 0; c0 < n; c0 += kChunk) {
+      if (c0 > 0 || q0 > 0) load_chunk(c0);
+#pragma unroll
+      for (int i = 0; i < kChunk; ++i) {
+        const int c = c0 + i;
+        if (c < n) {
+          const TX tau = TX(wave::rl(taul, c));
+          const TX u0 = lane == c ? TX(1) : keep_if(TX(t0[i]), lane > c && v0);
+          const TX u1 = ONE ? TX(0) : keep_if(TX(t1[ONE ? 0 : i]), v1);
+#pragma unroll
+          for (int b = 0; b < QB; ++b) {
+            const TX w = wave::sum(ONE ? u0 * x0[b] : fma(u0, x0[b], u1 * x1[b])) * tau;
+            x0[b] = fma(-u0, w, x0[b]);
+            if constexpr (!ONE) x1[b] = fma(-u1, w, x1[b]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      const int q = q0 + b;
+      if (q < nrhs) {
+        TX* x = a.x + size_t(q) * a.ldx;
+        if (v0) x[out0] = x0[b];
+        if (v1) x[out1] = x1[b];
+        for (int i = 0; i < nr; ++i) {
+          const TX s = wave::sum(lane < n ? TX(Cj[i + size_t(lane) * nr]) * x0[b] : TX(0));
+          if (lane == 0) a.Xpart[size_t(j) * nr * nrhs + i + size_t(q) * nr] = -s;
         }
       }
     }
@@ -388,6 +464,10 @@ __device__ __forceinline__ void backward_lu_stream2_body(SolveArgs<TW, TX> a, in
   if (row) x[size_t(j) * n + r] = s;
 }
 
+template <typename TW, typename TX, bool ONE, int QB>
+__global__ void __launch_bounds__(256) forward_qr_stream_kernel(SolveArgs<TW, TX> a) {
+  forward_qr_stream_body<TW, TX, ONE, QB>(a, blockIdx.x);
+}
 template <typename TW, typename TX, bool FWD, int QB>
 __global__ void __launch_bounds__(256) sweep_lu_stream_kernel(SolveArgs<TW, TX> a) {
   if (FWD) forward_lu_stream_body<TW, TX, QB>(a, blockIdx.x);
@@ -411,6 +491,18 @@ __global__ void __launch_bounds__(128) sweep_lu_stream2_back_batched(BatchTable<
 }
 
 }  // namespace
+
+template <typename TW, typename TX>
+bool launch_forward_qr(SolveArgs<TW, TX> const& a, hipStream_t st, hipError_t* err) {
+  if (a.n < 1 || a.n > 64 || a.npairs < 1) return false;
+  const dim3 g((a.npairs + 3) / 4), b(256);
+  if (a.n <= 32 && a.nrhs > 1) hipLaunchKernelGGL((forward_qr_stream_kernel<TW, TX, true, 4>), g, b, 0, st, a);
+  else if (a.n <= 32) hipLaunchKernelGGL((forward_qr_stream_kernel<TW, TX, true, 1>), g, b, 0, st, a);
+  else if (a.nrhs > 1) hipLaunchKernelGGL((forward_qr_stream_kernel<TW, TX, false, 4>), g, b, 0, st, a);
+  else hipLaunchKernelGGL((forward_qr_stream_kernel<TW, TX, false, 1>), g, b, 0, st, a);
+  *err = hipGetLastError();
+  return true;
+}
 
 template <typename TW, typename TX>
 bool launch_sweep_lu_stream(bool forward, SolveArgs<TW, TX> const& a, hipStream_t st, hipError_t* err) {
@@ -442,6 +534,7 @@ bool launch_sweep_lu_stream_batched(bool forward, BatchTable<SolveArgs<TW, TX>> 
 
 #define BCR_INST(TW, TX)                                                                                         \
   template bool launch_sweep_lu_stream<TW, TX>(bool, SolveArgs<TW, TX> const&, hipStream_t, hipError_t*);       \
+  template bool launch_forward_qr<TW, TX>(SolveArgs<TW, TX> const&, hipStream_t, hipError_t*);                    \
   template bool launch_sweep_lu_stream_batched<TW, TX>(bool, BatchTable<SolveArgs<TW, TX>> const&, int, int,     \
                                                        hipStream_t, hipError_t*);
 BCR_INST(double, double)

@@ -40,6 +40,44 @@ __device__ __forceinline__ unsigned min_u32(unsigned x) {
   return unsigned(__builtin_amdgcn_readlane(int(x), 63));
 }
 
+// sum over the 64 lanes, the same bits in every lane: DPP within rows of 16,
+// lane swaps across them (a butterfly of ds_bpermute exchanges takes five
+// times as long)
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = int(mov<CTRL>(unsigned(b & 0xffffffff), 0u)), hi = int(mov<CTRL>(unsigned(b >> 32), 0u));
+  return v + __hiloint2double(hi, lo);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __uint_as_float(mov<CTRL>(__float_as_uint(v), 0u));
+}
+template <bool ROW16>
+__device__ __forceinline__ auto lane_swap(unsigned x) {
+  if constexpr (ROW16) return __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  else return __builtin_amdgcn_permlane32_swap(x, x, false, false);
+}
+template <bool ROW16>
+__device__ __forceinline__ double swap_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const auto lo = lane_swap<ROW16>(unsigned(b & 0xffffffff)), hi = lane_swap<ROW16>(unsigned(b >> 32));
+  return __hiloint2double(int(hi[0]), int(lo[0])) + __hiloint2double(int(hi[1]), int(lo[1]));
+}
+template <bool ROW16>
+__device__ __forceinline__ float swap_add(float v) {
+  const auto p = lane_swap<ROW16>(__float_as_uint(v));
+  return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+template <typename T>
+__device__ __forceinline__ T sum(T v) {
+  v = dpp_add<kQuad1032>(v);
+  v = dpp_add<kQuad2301>(v);
+  v = dpp_add<kHalfMirror>(v);
+  v = dpp_add<kMirror>(v);
+  return swap_add<false>(swap_add<true>(v));
+}
+
 // lane l's value, uniform (two SGPRs for a double)
 __device__ __forceinline__ double rl(double v, int l) {
   const long long b = __double_as_longlong(v);
