@@ -15,8 +15,8 @@ Candidates (alglin_batch_set_class_kernel codes):
   class 4, FP32 factors: the matrix-core pair (0), column-split waves with
                          4 / 8 / 16 waves per pair (1), register tiles (2)
   class 3, FP64 factors: the matrix-core pair (0), the two-wave split (1)
-  class 4, FP64 factors: the matrix-core pair (0, n <= 48), column-split
-                         waves 4 / 8 / 16 (1), register tiles (2)
+  class 4, FP64 factors: the matrix-core pair (0), column-split waves
+                         4 / 8 / 16 (1), register tiles (2)
 
 Usage: python -m alglin_amd.autotune [--nsys 1024] [--seed 3] [--reps 3] [--out alglin_amd/tuning.json]
 """

@@ -521,7 +521,7 @@ void BatchEngine<TA, TW>::factorize_impl(std::vector<hipEvent_t>* ev) {
   hip_check(launch_convert<TA, double>(pF_, Feff_.p, tot_[kbF], st_), "F");
   hip_check(launch_reduce_batched<TW, double>(fred_, ns, st_), "reduce F");
   hip_check(launch_assemble_last_batched<TW, TA>(asm_, ns, st_), "assemble last");
-  hip_check(launch_lu_last_batched(lu_, stptr_, ns, Ncmax_, lds_limit_, st_), "lu last");
+  hip_check(launch_lu_last_batched(lu_, stptr_, ns, Ncmax_, st_), "lu last");
 }
 
 template <typename TA, typename TW>

@@ -156,7 +156,7 @@ hipError_t launch_sweep_generic_batched(bool forward, int method, BatchTable<Sol
 template <typename TW, typename TA>
 hipError_t launch_assemble_last_batched(const AssembleArgs<TW, TA>* args, int nsys, hipStream_t st);
 hipError_t launch_lu_last_batched(const LastSolveArgs<double>* args, int32_t* const* status, int nsys, int Ncmax,
-                                  size_t lds_limit, hipStream_t st);
+                                  hipStream_t st);
 template <typename TX>
 hipError_t launch_last_solve_batched(const LastSolveArgs<TX>* args, int nsys, int Nrmax, int Ncmax, size_t lds_limit,
                                      hipStream_t st);

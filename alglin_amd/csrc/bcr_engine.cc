@@ -510,7 +510,7 @@ void Engine<TA, TW>::factorize_async() {
     if (last2_)
       hip_check(launch_convert<double, double>(Hm_.p, Hm2_.p, int64_t(d_.Nr()) * d_.Nc(), st_), "copy last block");
     switch (last_method_) {
-      case kLastLU: hip_check(launch_lu_last(Hm_.p, d_.Nc(), ipiv_.p, status_.p, lds_limit_, st_), "lu last"); break;
+      case kLastLU: hip_check(launch_lu_last(Hm_.p, d_.Nc(), ipiv_.p, status_.p, st_), "lu last"); break;
       case kLastLUPQ:
         hip_check(launch_lupq_last(Hm_.p, d_.Nc(), ipiv_.p, jpiv_.p, status_.p, lds_limit_, st_), "lupq last");
         break;

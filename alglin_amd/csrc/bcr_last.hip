@@ -10,7 +10,7 @@
 //
 // assemble_last_kernel builds it (folding the pending C_N contributions and
 // the summed F partials), lu_last_kernel factors it with partial pivoting in
-// one workgroup (LDS-resident when it fits, else in place in HBM/L2),
+// one workgroup (lu_last_regs in registers up to 192 columns, else in place),
 // last_solve_kernel gathers the last-block right-hand side straight from the
 // solution vector, solves, and scatters (x_0, x_N, q, xb) back (the
 // reference's swap of x[0:n] with x[(N-1)n:Nn], cc:1392-1423, is the same
@@ -27,18 +27,14 @@ __global__ void __launch_bounds__(256) assemble_last_kernel(AssembleArgs<TW, TA>
 
 // LU with partial pivoting (dgetf2 order: first max, whole-row swaps,
 // reciprocal scaling) of the square Nc x Nc last block.
-template <bool IN_LDS>
+// Past 192 columns (up to there lu_last_regs), in place: too large for LDS.
 __device__ __forceinline__ void lu_last_body(double* __restrict__ Hm, int Nc, int32_t* __restrict__ ipiv,
                                              int32_t* __restrict__ status) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ int s_piv;
   const int tid = threadIdx.x, nth = blockDim.x;
   const int lane = tid & 63, wid = tid >> 6;
   const int ld = Nc;
-  double* A = IN_LDS ? reinterpret_cast<double*>(smem_raw) : Hm;
-  if (IN_LDS)
-    for (int i = tid; i < Nc * Nc; i += nth) A[i] = Hm[i];
-  __syncthreads();
+  double* A = Hm;
   for (int c = 0; c < Nc; ++c) {
     if (wid == 0) {
       double best = -1;
@@ -79,8 +75,6 @@ __device__ __forceinline__ void lu_last_body(double* __restrict__ Hm, int Nc, in
     }
     __syncthreads();
   }
-  if (IN_LDS)
-    for (int i = tid; i < Nc * Nc; i += nth) Hm[i] = A[i];
 }
 
 // A_LDS: the factored last block is staged in LDS; otherwise (Nr*Nc*8 bytes
@@ -92,10 +86,9 @@ __device__ __forceinline__ void lu_last_body(double* __restrict__ Hm, int Nc, in
 //   LUPQ row swaps P, L, U, column swaps Q in reverse
 //   QR   y = Q^T b (reflectors in order), R^{-1} y      (ormqr + trsv)
 //   QRP  as QR, then x[jpvt[i]] = y[i]
-template <bool IN_LDS>
 __global__ void __launch_bounds__(1024) lu_last_kernel(double* __restrict__ Hm, int Nc, int32_t* __restrict__ ipiv,
                                                         int32_t* __restrict__ status) {
-  lu_last_body<IN_LDS>(Hm, Nc, ipiv, status);
+  lu_last_body(Hm, Nc, ipiv, status);
 }
 
 template <typename TX, bool A_LDS>
@@ -241,10 +234,9 @@ __global__ void __launch_bounds__(256) assemble_last_batched(const AssembleArgs<
   assemble_last_body<TW, TA>(args[blockIdx.x], threadIdx.x, blockDim.x);
 }
 
-template <bool IN_LDS>
 __global__ void __launch_bounds__(1024) lu_last_batched(const LastSolveArgs<double>* args, int32_t* const* status) {
   const LastSolveArgs<double>& a = args[blockIdx.x];
-  lu_last_body<IN_LDS>(const_cast<double*>(a.Hm), a.Nc, const_cast<int32_t*>(a.P), status[blockIdx.x]);
+  lu_last_body(const_cast<double*>(a.Hm), a.Nc, const_cast<int32_t*>(a.P), status[blockIdx.x]);
 }
 
 template <typename TX, bool A_LDS>
@@ -293,7 +285,7 @@ __global__ void __launch_bounds__(64 * NWV) lu_last_regs(double* Hm, int Nc, int
 // args[s].Hm / .P (ipiv) / .Nc describe the square last block of system s;
 // Ncmax is the largest of the launch
 hipError_t launch_lu_last_batched(const LastSolveArgs<double>* args, int32_t* const* status, int nsys, int Ncmax,
-                                  size_t lds_limit, hipStream_t st) {
+                                  hipStream_t st) {
   if (Ncmax <= 64) {
     hipLaunchKernelGGL((lu_last_regs_batched<1, 1>), dim3(nsys), dim3(64), 0, st, args, status);
     return hipGetLastError();
@@ -306,11 +298,7 @@ hipError_t launch_lu_last_batched(const LastSolveArgs<double>* args, int32_t* co
     hipLaunchKernelGGL((lu_last_regs_batched<2, 4>), dim3(nsys), dim3(256), 0, st, args, status);
     return hipGetLastError();
   }
-  const size_t bytes = size_t(Ncmax) * Ncmax * sizeof(double);
-  if (bytes <= lds_limit)
-    hipLaunchKernelGGL((lu_last_batched<true>), dim3(nsys), dim3(1024), bytes, st, args, status);
-  else
-    hipLaunchKernelGGL((lu_last_batched<false>), dim3(nsys), dim3(1024), 0, st, args, status);
+  hipLaunchKernelGGL(lu_last_batched, dim3(nsys), dim3(1024), 0, st, args, status);
   return hipGetLastError();
 }
 
@@ -354,18 +342,14 @@ hipError_t launch_assemble_last(AssembleArgs<TW, TA> const& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_lu_last(double* Hm, int Nc, int32_t* ipiv, int32_t* status, size_t lds_limit, hipStream_t st) {
+hipError_t launch_lu_last(double* Hm, int Nc, int32_t* ipiv, int32_t* status, hipStream_t st) {
   if (Nc <= 192) {   // in registers, 16 columns per wavefront
     if (Nc <= 64) hipLaunchKernelGGL((lu_last_regs<1, 4>), dim3(1), dim3(256), 0, st, Hm, Nc, ipiv, status);
     else if (Nc <= 128) hipLaunchKernelGGL((lu_last_regs<2, 8>), dim3(1), dim3(512), 0, st, Hm, Nc, ipiv, status);
     else hipLaunchKernelGGL((lu_last_regs<3, 12>), dim3(1), dim3(768), 0, st, Hm, Nc, ipiv, status);
     return hipGetLastError();
   }
-  const size_t bytes = size_t(Nc) * Nc * sizeof(double);
-  if (bytes <= lds_limit)
-    hipLaunchKernelGGL((lu_last_kernel<true>), dim3(1), dim3(1024), bytes, st, Hm, Nc, ipiv, status);
-  else
-    hipLaunchKernelGGL((lu_last_kernel<false>), dim3(1), dim3(1024), 0, st, Hm, Nc, ipiv, status);
+  hipLaunchKernelGGL(lu_last_kernel, dim3(1), dim3(1024), 0, st, Hm, Nc, ipiv, status);
   return hipGetLastError();
 }
 

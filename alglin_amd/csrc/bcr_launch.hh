@@ -9,9 +9,10 @@ template <typename TW, typename TX> struct SolveArgs;
 template <typename TW, typename TA> struct AssembleArgs;
 template <typename TA> struct MvArgs;
 
-// Householder QR / QRP pair elimination for every n <= 64, nr <= 16: T in
-// LDS, the right-hand columns in chunks of cw next to it (pair_qr_plan picks
-// cw and the LDS bytes); false for LU or a shape beyond
+// Householder QR / QRP pair elimination for every n <= 64, nr <= 16: beyond
+// n = 16 (nr <= 8, nx <= 16) a panel launch and one for the right-hand columns,
+// else T in LDS and the right-hand columns in chunks of cw next to it
+// (pair_qr_plan picks cw and the LDS bytes); false for LU or a shape beyond
 bool pair_qr_plan(int n, int nr, int nx, size_t elem, size_t lds_limit, int* cw, size_t* bytes);
 template <typename TS, typename TW>
 bool launch_pair_qr(int method, FactorArgs<TS, TW> const& a, size_t lds_limit, hipStream_t st, hipError_t* err);
@@ -64,7 +65,7 @@ hipError_t launch_reduce(const TP* part, int first, int count, int m, TP* tmp, i
 
 template <typename TW, typename TA>
 hipError_t launch_assemble_last(AssembleArgs<TW, TA> const& a, hipStream_t st);
-hipError_t launch_lu_last(double* Hm, int Nc, int32_t* ipiv, int32_t* status, size_t lds_limit, hipStream_t st);
+hipError_t launch_lu_last(double* Hm, int Nc, int32_t* ipiv, int32_t* status, hipStream_t st);
 template <typename TX>
 hipError_t launch_last_solve(LastSolveArgs<TX> const& a, size_t lds_limit, hipStream_t st);
 hipError_t launch_lupq_last(double* Hm, int Nc, int32_t* P, int32_t* Q, int32_t* status, size_t lds_limit,
