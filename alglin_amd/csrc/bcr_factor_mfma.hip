@@ -1230,9 +1230,18 @@ bool launch_pair_lu_mfma_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nb
 template <typename TS, typename TW>
 void launch_pair_qr_rhs(FactorArgs<TS, TW> const& a, hipStream_t st) {
   const dim3 g(a.npairs);
+  // (four waves as in launch_pair: FP64 levels of a few pairs 22 -> 17 us at
+  // n = 32, 39 -> 26 at n = 40; beyond n = 48 V leaves the LDS for two tiles)
+  const bool few = a.npairs <= kFewPairs;
   switch (mfma_variant(a.n, a.nr, a.nx)) {
-    case 1: hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 2, 3, 2>), g, dim3(128), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 3, 4, 2>), g, dim3(128), 0, st, a); break;
+    case 1:
+      if (few) hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 2, 3, 4>), g, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 2, 3, 2>), g, dim3(128), 0, st, a);
+      break;
+    case 2:
+      if (few) hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 3, 4, 4>), g, dim3(256), 0, st, a);
+      else hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 3, 4, 2>), g, dim3(128), 0, st, a);
+      break;
     case 3: hipLaunchKernelGGL((pair_qr_rhs_kernel<TS, TW, 4, 5, 2>), g, dim3(128), 0, st, a); break;
   }
 }
