@@ -198,11 +198,31 @@ __global__ void __launch_bounds__(128) backward_kernel(SolveArgs<TW, TX> a) {
 template <typename TP, typename TD>
 __global__ void __launch_bounds__(256) reduce_partial_kernel(const TP* __restrict__ part, int first, int count,
                                                              int m, TP* __restrict__ tmp, int nchunks) {
-  // pass 1: chunk b sums rows [lo, hi) of part for every i < m
-  const int b = blockIdx.x;
+  // pass 1: chunk b sums rows [lo, hi) of part for every i < m.  Narrow rows
+  // are taken several at a time, 256 / m of them side by side (whole runs of
+  // memory; a thread per column left most idle behind a chain of loads: N =
+  // 100000, m = 16 42 us, so 7), and their sums added in a fixed order.
+  __shared__ TP red[256];
+  const int b = blockIdx.x, t = threadIdx.x;
   const int per = (count + nchunks - 1) / nchunks;
   const int lo = first + b * per, hi = min(first + count, lo + per);
-  for (int i = threadIdx.x; i < m; i += blockDim.x) {
+  if (m <= 128) {
+    const int G = 256 / m, sub = t / m, i = t - sub * m;
+    TP s = 0;
+    if (sub < G)
+      for (int k = lo + sub; k < hi; k += G) s += part[size_t(k) * m + i];
+    red[t] = s;
+    __syncthreads();
+    for (int g = G; g > 1;) {
+      const int h = (g + 1) / 2;
+      if (sub < g - h) red[t] += red[t + h * m];
+      __syncthreads();
+      g = h;
+    }
+    if (t < m) tmp[size_t(b) * m + t] = red[t];
+    return;
+  }
+  for (int i = t; i < m; i += 256) {
     TP s = 0;
     for (int k = lo; k < hi; ++k) s += part[size_t(k) * m + i];
     tmp[size_t(b) * m + i] = s;
