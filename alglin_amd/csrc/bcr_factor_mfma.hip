@@ -483,7 +483,10 @@ struct PanelWavesLds {
   uint8_t pos[2][128];
 };
 
-template <typename TS, typename TW, int NB, int RS>
+// BATCH: a launch takes the NB of its largest n, so 16 (NB - 1) < n holds for a
+// single system only, and with it the first tile the border rows can lie in
+// (every tile tried for a single system too: n = 53, 9001 rows 4255 -> 4284 us).
+template <typename TS, typename TW, int NB, int RS, bool BATCH>
 __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int p) {
   using Lds = PanelWavesLds<TW, NB, RS>;
   constexpr int TILES = Lds::TILES, RLD = Lds::RLD, ULD = Lds::ULD;
@@ -491,7 +494,7 @@ __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int
   if (p >= a.npairs) return;   // uniform over the workgroup
   const int lane = threadIdx.x & 63, g = lane >> 4, cl = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int n = a.n, nr = a.nr, n2 = 2 * n, R = n2 + nr;   // 16 (NB - 1) < n <= 16 NB
+  const int n = a.n, nr = a.nr, n2 = 2 * n, R = n2 + nr;   // n <= 16 NB
   int j, jp, jpp;
   pair_of_uniform(a, p, j, jp, jpp);
   const size_t nn = size_t(n) * n, rn = size_t(nr) * n;
@@ -515,7 +518,7 @@ __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int
         T[t][i] = keep_if(TW(src[coff]), r < n2 && col < n);
       }
 #pragma unroll
-    for (int t = 2 * NB - 2; t < TILES; ++t)
+    for (int t = BATCH ? 0 : 2 * NB - 2; t < TILES; ++t)
       if (16 * t + 16 > n2 && 16 * t < R) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -1117,12 +1120,12 @@ constexpr int kWavesPairs = 1024;
 
 template <typename TS, typename TW, int NB, int RS>
 __global__ void __launch_bounds__(64 * NB, 3) pair_lu_tw_kernel(FactorArgs<TS, TW> a) {
-  pair_lu_tw_body<TS, TW, NB, RS>(a, blockIdx.x);
+  pair_lu_tw_body<TS, TW, NB, RS, false>(a, blockIdx.x);
 }
 template <typename TS, typename TW, int NB, int RS>
 __global__ void __launch_bounds__(64 * NB, 3) pair_lu_tw_batched(BatchTable<FactorArgs<TS, TW>> t) {
   const int e = t.entry[blockIdx.x];
-  pair_lu_tw_body<TS, TW, NB, RS>(t.args[e], int(blockIdx.x) - t.first[e]);
+  pair_lu_tw_body<TS, TW, NB, RS, true>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
 constexpr int rhs_waves(int nb, size_t elem) { return elem == 8 ? (nb <= 3 ? 2 : 1) : nb <= 2 ? 4 : nb == 3 ? 3 : 2; }
 
