@@ -103,6 +103,7 @@ __device__ __forceinline__ void last_solve_body(LastSolveArgs<TX> const& a) {
   const double* A = A_LDS ? sm : a.Hm;
   double* X = A_LDS ? sm + size_t(Nr) * Nc : sm;   // R x 16
   double* Z = X + size_t(R) * 16;                   // Nc x 16 (QRP permutation)
+  double* s_w = Z + size_t(Nc) * 16;                // 16 (a reflector's products)
   constexpr int QC = 16;
   if (A_LDS)
     for (int i = tid; i < Nr * Nc; i += nth) sm[i] = a.Hm[i];
@@ -164,7 +165,6 @@ __device__ __forceinline__ void last_solve_body(LastSolveArgs<TX> const& a) {
       for (int k = 0; k < Nc; ++k) {
         const double tk = a.tau[k];
         if (tk != 0.0) {
-          __shared__ double s_w[QC];
           if (wid < nq) {
             double s = 0;
             for (int r = k + lane; r < Nr; r += 64) s += (r == k ? 1.0 : A[r + k * ld]) * X[r + wid * R];
@@ -302,11 +302,16 @@ hipError_t launch_lu_last_batched(const LastSolveArgs<double>* args, int32_t* co
   return hipGetLastError();
 }
 
+// LDS of the last solve beside the factored block: the columns X and Z, and
+// the products of a reflector
+static size_t last_solve_bytes(int Nr, int Nc) {
+  return (size_t(Nr > Nc ? Nr : Nc) + Nc + 1) * 16 * sizeof(double);
+}
+
 template <typename TX>
 hipError_t launch_last_solve_batched(const LastSolveArgs<TX>* args, int nsys, int Nrmax, int Ncmax, size_t lds_limit,
                                      hipStream_t st) {
-  const int R = Nrmax > Ncmax ? Nrmax : Ncmax;
-  const size_t xbytes = (size_t(R) + Ncmax) * 16 * sizeof(double);
+  const size_t xbytes = last_solve_bytes(Nrmax, Ncmax);
   const size_t bytes = size_t(Nrmax) * Ncmax * sizeof(double) + xbytes;
   if (xbytes > lds_limit) return hipErrorInvalidConfiguration;
   if (bytes <= lds_limit)
@@ -362,8 +367,7 @@ hipError_t launch_last_solve(LastSolveArgs<TX> const& a, size_t lds_limit, hipSt
     else hipLaunchKernelGGL((last_solve_lu_wave<TX, 4>), dim3(a.nrhs), dim3(64), 0, st, a);
     return hipGetLastError();
   }
-  const int R = a.Nr > a.Nc ? a.Nr : a.Nc;
-  const size_t xbytes = (size_t(R) + a.Nc) * 16 * sizeof(double);
+  const size_t xbytes = last_solve_bytes(a.Nr, a.Nc);
   const size_t bytes = size_t(a.Nr) * a.Nc * sizeof(double) + xbytes;
   if (xbytes > lds_limit) return hipErrorInvalidConfiguration;
   if (bytes <= lds_limit)
