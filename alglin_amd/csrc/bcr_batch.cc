@@ -118,7 +118,7 @@ bool BatchEngine<TA, TW>::panel_fits(SysDims const& d, size_t lds_limit) {
   int cw = 0;
   size_t bytes = 0;
   if (d.method != kLU && pair_qr_plan(d.n, d.nr, d.nx, sizeof(TW), lds_limit, &cw, &bytes)) return true;
-  return size_t(2 * d.n + d.nr) * (3 * d.n + d.nx) * sizeof(TW) <= lds_limit;
+  return pair_generic_lds(d.method, d.n, d.nr, d.nx, sizeof(TW)) <= lds_limit;
 }
 
 template <typename TA, typename TW>
@@ -503,10 +503,7 @@ void BatchEngine<TA, TW>::factorize_impl(std::vector<hipEvent_t>* ev) {
         else if (l.method != kLU &&
                  launch_pair_qr_batched(l.method, t, l.nblocks, l.nmax, l.nrmax, l.nxmax, lds_limit_, s, &e))
           ok = true;
-        else {
-          const size_t bytes = size_t(2 * l.nmax + l.nrmax) * (3 * l.nmax + l.nxmax) * sizeof(TW);
-          e = launch_pair_generic_batched(l.method, t, l.nblocks, bytes, lds_limit_, s);
-        }
+        else e = launch_pair_generic_batched(l.method, t, l.nblocks, l.nmax, l.nrmax, l.nxmax, lds_limit_, s);
         if (!ok) throw HipError("batch factorize: no kernel for a class");
         stats = stats && wrote;
       };

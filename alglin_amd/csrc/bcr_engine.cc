@@ -394,8 +394,8 @@ void Engine<TA, TW>::level_factor(Level const& l) {
       hip_check(e, "pair_qr");
       return;
     }
-    const size_t bytes = size_t(2 * d_.n + d_.nr) * (3 * d_.n + d_.nx) * sizeof(TW);
-    if (bytes > lds_limit_) gscratch_.resize(size_t(npairs) * (bytes / sizeof(TW)));
+    if (pair_generic_lds(method_, d_.n, d_.nr, d_.nx, sizeof(TW)) > lds_limit_)
+      gscratch_.resize(size_t(npairs) * (2 * d_.n + d_.nr) * (3 * d_.n + d_.nx));
     hip_check(launch_pair_generic(method_, a, gscratch_.p, lds_limit_, st_), "pair_generic");
   };
   if (first) {

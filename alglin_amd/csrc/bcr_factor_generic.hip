@@ -39,6 +39,8 @@
 //   - x = N is never read by a pair; the last-block assembly reads it.
 #include "bcr_launch.hh"
 
+#include <algorithm>
+
 namespace bcr {
 
 // wave-level argmax over (value, index); ties keep the smaller index
@@ -327,13 +329,43 @@ __global__ void __launch_bounds__(256) pair_generic_kernel(FactorArgs<TS, TW> a,
 }
 
 
+template <typename TS, typename TW, int METHOD>
+__global__ void __launch_bounds__(256) pair_generic_batched(BatchTable<FactorArgs<TS, TW>> t) {
+  const int e = t.entry[blockIdx.x];
+  pair_generic_body<TS, TW, METHOD, true>(t.args[e], nullptr, int(blockIdx.x) - t.first[e]);
+}
+
+// LDS a kernel declares itself, which a launch needs beside its dynamic bytes
+template <typename K>
+static size_t declared_lds(K kernel) {
+  hipFuncAttributes at{};
+  if (hipFuncGetAttributes(&at, reinterpret_cast<const void*>(kernel)) != hipSuccess) return 4096;   // more than any here
+  return at.sharedSizeBytes;
+}
+
+template <typename TW, int METHOD>
+static size_t generic_tables() {
+  static const size_t b = std::max(declared_lds(pair_generic_kernel<TW, TW, METHOD, true>),
+                                   declared_lds(pair_generic_batched<TW, TW, METHOD>));
+  return b;
+}
+
+size_t pair_generic_lds(int method, int n, int nr, int nx, size_t elem) {
+  const size_t panel = size_t(2 * n + nr) * (3 * n + nx) * elem;
+  if (elem == sizeof(double))
+    return panel + (method == kLU ? generic_tables<double, kLU>() : method == kQR ? generic_tables<double, kQR>()
+                                                                                   : generic_tables<double, kQRP>());
+  return panel + (method == kLU ? generic_tables<float, kLU>() : method == kQR ? generic_tables<float, kQR>()
+                                                                                : generic_tables<float, kQRP>());
+}
+
 template <typename TS, typename TW>
 hipError_t launch_pair_generic(int method, FactorArgs<TS, TW> const& a, TW* gscratch, size_t lds_limit,
                                hipStream_t st) {
   const int R = 2 * a.n + a.nr, Wc = 3 * a.n + a.nx;
   const size_t bytes = size_t(R) * Wc * sizeof(TW);
   dim3 grid(a.npairs), block(256);
-  const bool lds = bytes <= lds_limit;
+  const bool lds = pair_generic_lds(method, a.n, a.nr, a.nx, sizeof(TW)) <= lds_limit;
   if (!lds && gscratch == nullptr) return hipErrorInvalidValue;
 #define BCR_LAUNCH(M)                                                                                    \
   if (lds) hipLaunchKernelGGL((pair_generic_kernel<TS, TW, M, true>), grid, block, bytes, st, a, gscratch); \
@@ -345,17 +377,12 @@ hipError_t launch_pair_generic(int method, FactorArgs<TS, TW> const& a, TW* gscr
   return hipGetLastError();
 }
 
-template <typename TS, typename TW, int METHOD>
-__global__ void __launch_bounds__(256) pair_generic_batched(BatchTable<FactorArgs<TS, TW>> t) {
-  const int e = t.entry[blockIdx.x];
-  pair_generic_body<TS, TW, METHOD, true>(t.args[e], nullptr, int(blockIdx.x) - t.first[e]);
-}
-
-// panels staged in LDS only: `bytes` is the largest panel of the launch
+// panels staged in LDS only: n, nr, nx are the largest of the launch
 template <typename TS, typename TW>
-hipError_t launch_pair_generic_batched(int method, BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, size_t bytes,
-                                       size_t lds_limit, hipStream_t st) {
-  if (bytes > lds_limit) return hipErrorInvalidValue;
+hipError_t launch_pair_generic_batched(int method, BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, int n, int nr,
+                                       int nx, size_t lds_limit, hipStream_t st) {
+  const size_t bytes = size_t(2 * n + nr) * (3 * n + nx) * sizeof(TW);
+  if (pair_generic_lds(method, n, nr, nx, sizeof(TW)) > lds_limit) return hipErrorInvalidValue;
   if (method == kLU) hipLaunchKernelGGL((pair_generic_batched<TS, TW, kLU>), dim3(nblocks), dim3(256), bytes, st, t);
   else if (method == kQR) hipLaunchKernelGGL((pair_generic_batched<TS, TW, kQR>), dim3(nblocks), dim3(256), bytes, st, t);
   else hipLaunchKernelGGL((pair_generic_batched<TS, TW, kQRP>), dim3(nblocks), dim3(256), bytes, st, t);
@@ -363,11 +390,14 @@ hipError_t launch_pair_generic_batched(int method, BatchTable<FactorArgs<TS, TW>
 }
 
 template hipError_t launch_pair_generic_batched<double, double>(int, BatchTable<FactorArgs<double, double>> const&, int,
-                                                                size_t, size_t, hipStream_t);
+                                                                int, int, int,
+                                                                size_t, hipStream_t);
 template hipError_t launch_pair_generic_batched<float, float>(int, BatchTable<FactorArgs<float, float>> const&, int,
-                                                              size_t, size_t, hipStream_t);
+                                                              int, int, int,
+                                                                size_t, hipStream_t);
 template hipError_t launch_pair_generic_batched<double, float>(int, BatchTable<FactorArgs<double, float>> const&, int,
-                                                               size_t, size_t, hipStream_t);
+                                                               int, int, int,
+                                                                size_t, hipStream_t);
 template hipError_t launch_pair_generic<double, double>(int, FactorArgs<double, double> const&, double*, size_t, hipStream_t);
 template hipError_t launch_pair_generic<float, float>(int, FactorArgs<float, float> const&, float*, size_t, hipStream_t);
 template hipError_t launch_pair_generic<double, float>(int, FactorArgs<double, float> const&, float*, size_t, hipStream_t);

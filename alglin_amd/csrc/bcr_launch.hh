@@ -20,6 +20,8 @@ bool launch_pair_qr(int method, FactorArgs<TS, TW> const& a, size_t lds_limit, h
 // pair_lu_mfma_fits)
 template <typename TS, typename TW>
 void launch_pair_qr_rhs(FactorArgs<TS, TW> const& a, hipStream_t st);
+// LDS of a workgroup that stages a whole pair panel (and its step tables)
+size_t pair_generic_lds(int method, int n, int nr, int nx, size_t elem);
 template <typename TS, typename TW>
 hipError_t launch_pair_generic(int method, FactorArgs<TS, TW> const& a, TW* gscratch, size_t lds_limit,
                                hipStream_t st);

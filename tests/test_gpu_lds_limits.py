@@ -1,7 +1,7 @@
 """Shapes whose LDS arrays come out at exactly the limit of a workgroup
 (163840 bytes), one below and one beyond: the last solve's block and columns
-(Nc = 128 with 16 columns; Nc = 640 the columns alone).  A drawn solution x,
-b = A x: |x' - x| <= 50 eps cond relative to the largest entry."""
+(Nc = 128 with 16 columns; Nc = 640 the columns alone) and a whole pair panel
+(n = 32, nx = 224 in FP64).  A drawn solution x, b = A x: |x' - x| <= 50 eps cond relative to the largest entry."""
 import numpy as np
 import pytest
 
@@ -66,3 +66,31 @@ def test_last_solve_columns(Nc, fits):
     else:
         with pytest.raises(AlglinError):
             bt.solve(DeviceArray.from_host(b), Xd, max_iter=0, graph=False)
+
+
+@pytest.mark.parametrize("nx,fits", [(223, True), (224, False), (225, False)])
+def test_pair_panel(nx, fits):
+    """Beyond the limit a single system's panels go through global scratch;
+    a batch, which has none, refuses the plan."""
+    N, n = 5, 32
+    print(f"case panel n={n} nx={nx}", flush=True)
+    s = systems.gaussian_system(N, n, nx, 0, 0, nx, shift=4.0, seed=nx)
+    x, B = drawn(s, 3)
+    g = BorderedCR(np.float64)
+    g.load_system(s)
+    assert g.factorize(), g.last_error()
+    ok, X = g.solve_n(B)
+    assert ok and close(s, X, x)
+    bt = Batch(mixed=False)
+    dims = [(N, n, nx, 0, 0, nx, 0)]
+    if not fits:
+        with pytest.raises(AlglinError):
+            bt.plan(dims)
+        return
+    bt.plan(dims)
+    bt.load_system(0, s)
+    Xd = DeviceArray(bt.size("x"))
+    b = np.zeros(bt.size("x"))
+    b[:B.shape[0]] = B[:, 0]
+    bt.solve(DeviceArray.from_host(b), Xd, max_iter=0, graph=False)
+    assert close(s, Xd.to_host()[:x.shape[0]], x[:, 0])
