@@ -658,7 +658,7 @@ void BatchEngine<TA, TW>::solve_async(double* X) {
       if (!launch_sweep_lu_stream_batched(fwd, t, l.nblocks, l.nmax, s, &e))
         throw HipError("batch solve: no sweep kernel");
     } else {
-      e = launch_sweep_generic_batched(fwd, l.method, t, l.nblocks, l.nmax, l.nxmax, s);
+      e = launch_sweep_generic_batched(fwd, l.method, t, l.nblocks, l.nmax, l.nxmax, lds_limit_, s);
     }
     hip_check(e, fwd ? "batch forward" : "batch backward");
   };

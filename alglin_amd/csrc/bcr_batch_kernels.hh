@@ -150,7 +150,7 @@ bool launch_sweep_lu_stream_batched(bool forward, BatchTable<SolveArgs<TW, TX>> 
                                     hipStream_t st, hipError_t* err);
 template <typename TW, typename TX>
 hipError_t launch_sweep_generic_batched(bool forward, int method, BatchTable<SolveArgs<TW, TX>> const& t, int nblocks,
-                                        int n, int nx, hipStream_t st);
+                                        int n, int nx, size_t lds_limit, hipStream_t st);
 
 // last block, one workgroup per system
 template <typename TW, typename TA>

@@ -108,8 +108,11 @@ __global__ void __launch_bounds__(128) forward_kernel(SolveArgs<TW, TX> a) {
 }
 
 
-template <typename TW, typename TX, int METHOD>
+// WIDE: one column at a time and B_j read where it lies, for borders (nx) whose
+// B_j and 16 columns of x_b do not fit the LDS beside D_j, E_j and U
+template <typename TW, typename TX, int METHOD, bool WIDE>
 __device__ __forceinline__ void backward_body(SolveArgs<TW, TX> a, int bid) {
+  constexpr int CHUNK = WIDE ? 1 : kRhsChunk;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int p = bid;
   if (p >= a.npairs) return;
@@ -122,8 +125,8 @@ __device__ __forceinline__ void backward_body(SolveArgs<TW, TX> a, int bid) {
   TW* sE = sD + nn;
   TW* sU = sE + nn;
   TW* sB = sU + nn;
-  TX* Xs = reinterpret_cast<TX*>(smem_raw + align16((3 * nn + size_t(n) * nx) * sizeof(TW)));  // inputs
-  TX* Y = Xs + size_t(3 * n + nx) * kRhsChunk;
+  TX* Xs = reinterpret_cast<TX*>(smem_raw + align16((3 * nn + (WIDE ? 0 : size_t(n) * nx)) * sizeof(TW)));  // inputs
+  TX* Y = Xs + size_t(3 * n + nx) * CHUNK;
   __shared__ int s_perm[64];
 
   const TW* Tj = a.Tm + size_t(j) * tsize(n);
@@ -133,14 +136,16 @@ __device__ __forceinline__ void backward_body(SolveArgs<TW, TX> a, int bid) {
     const int r = i % n, c = i / n;
     sU[i] = Tj[r + c * n2];
   }
-  for (int i = tid; i < n * nx; i += nth) sB[i] = a.B[size_t(j) * n * nx + i];
+  const TW* const Bj = WIDE ? a.B + size_t(j) * n * nx : sB;
+  if (!WIDE)
+    for (int i = tid; i < n * nx; i += nth) sB[i] = a.B[size_t(j) * n * nx + i];
   if (METHOD == kQRP)
     for (int i = tid; i < n; i += nth) s_perm[i] = a.perm[size_t(j) * n + i];
   const size_t xbrow = size_t(a.N + 1) * n + a.qx;   // cc:1812
   const int W = 3 * n + nx;
 
-  for (int q0 = 0; q0 < a.nrhs; q0 += kRhsChunk) {
-    const int nq = min(kRhsChunk, a.nrhs - q0);
+  for (int q0 = 0; q0 < a.nrhs; q0 += CHUNK) {
+    const int nq = min(CHUNK, a.nrhs - q0);
     for (int i = tid; i < W * nq; i += nth) {
       const int r = i % W, q = i / W;
       size_t row;
@@ -156,7 +161,7 @@ __device__ __forceinline__ void backward_body(SolveArgs<TW, TX> a, int bid) {
       const TX* xq = Xs + q * W;
       TX acc = xq[r];
       for (int c = 0; c < n; ++c) acc -= TX(sD[r + c * n]) * xq[n + c] + TX(sE[r + c * n]) * xq[2 * n + c];
-      for (int c = 0; c < nx; ++c) acc -= TX(sB[r + c * n]) * xq[3 * n + c];
+      for (int c = 0; c < nx; ++c) acc -= TX(Bj[r + size_t(c) * n]) * xq[3 * n + c];
       Xs[r + q * W] = acc;
     }
     __syncthreads();
@@ -189,7 +194,7 @@ __device__ __forceinline__ void backward_body(SolveArgs<TW, TX> a, int bid) {
 
 template <typename TW, typename TX, int METHOD>
 __global__ void __launch_bounds__(128) backward_kernel(SolveArgs<TW, TX> a) {
-  backward_body<TW, TX, METHOD>(a, blockIdx.x);
+  backward_body<TW, TX, METHOD, false>(a, blockIdx.x);
 }
 
 
@@ -263,22 +268,30 @@ hipError_t launch_backward(int method, SolveArgs<TW, TX> const& a, hipStream_t s
   return hipGetLastError();
 }
 
-template <typename TW, typename TX, int METHOD, bool FWD>
+template <typename TW, typename TX, int METHOD, bool FWD, bool WIDE = false>
 __global__ void __launch_bounds__(128) sweep_generic_batched(BatchTable<SolveArgs<TW, TX>> t) {
   const int e = t.entry[blockIdx.x];
   if (skipped(t.args[e].skip)) return;
   if (FWD) forward_body<TW, TX, METHOD>(t.args[e], int(blockIdx.x) - t.first[e]);
-  else backward_body<TW, TX, METHOD>(t.args[e], int(blockIdx.x) - t.first[e]);
+  else backward_body<TW, TX, METHOD, WIDE>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
 
-// one workgroup per pair; n is the largest block size of the launch
+// one workgroup per pair; n and nx are the largest of the launch
 template <typename TW, typename TX>
 hipError_t launch_sweep_generic_batched(bool forward, int method, BatchTable<SolveArgs<TW, TX>> const& t, int nblocks,
-                                        int n, int nx, hipStream_t st) {
+                                        int n, int nx, size_t lds_limit, hipStream_t st) {
+  constexpr size_t kPerm = 64 * sizeof(int);   // the kernels' own s_perm
   const size_t nn = size_t(n) * n;
   const size_t fbytes = align16(tsize(n) * sizeof(TW)) + size_t(2 * n) * kRhsChunk * sizeof(TX);
   const size_t bbytes = align16((3 * nn + size_t(n) * nx) * sizeof(TW)) + (size_t(3 * n + nx) + n) * kRhsChunk * sizeof(TX);
   dim3 grid(nblocks), block(n <= 32 ? 64 : 128);
+  if (!forward && bbytes + kPerm > lds_limit) {
+    const size_t wbytes = align16(3 * nn * sizeof(TW)) + (size_t(3 * n + nx) + n) * sizeof(TX);
+    if (wbytes + kPerm > lds_limit) return hipErrorInvalidConfiguration;
+    if (method == kQRP) hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQRP, false, true>), grid, block, wbytes, st, t);
+    else hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kLU, false, true>), grid, block, wbytes, st, t);
+    return hipGetLastError();
+  }
   if (forward) {
     if (method == kLU) hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kLU, true>), grid, block, fbytes, st, t);
     else hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQR, true>), grid, block, fbytes, st, t);
@@ -290,11 +303,11 @@ hipError_t launch_sweep_generic_batched(bool forward, int method, BatchTable<Sol
 }
 
 template hipError_t launch_sweep_generic_batched<double, double>(bool, int, BatchTable<SolveArgs<double, double>> const&,
-                                                                 int, int, int, hipStream_t);
+                                                                 int, int, int, size_t, hipStream_t);
 template hipError_t launch_sweep_generic_batched<float, float>(bool, int, BatchTable<SolveArgs<float, float>> const&,
-                                                               int, int, int, hipStream_t);
+                                                               int, int, int, size_t, hipStream_t);
 template hipError_t launch_sweep_generic_batched<float, double>(bool, int, BatchTable<SolveArgs<float, double>> const&,
-                                                                int, int, int, hipStream_t);
+                                                                int, int, int, size_t, hipStream_t);
 
 // dst[(i%mrow) + (i/mrow)*ldd] += sum_{k=first}^{first+count-1} part[k*m + i]
 template <typename TP, typename TD>

@@ -1,7 +1,9 @@
 """Shapes whose LDS arrays come out at exactly the limit of a workgroup
 (163840 bytes), one below and one beyond: the last solve's block and columns
-(Nc = 128 with 16 columns; Nc = 640 the columns alone) and a whole pair panel
-(n = 32, nx = 224 in FP64).  A drawn solution x, b = A x: |x' - x| <= 50 eps cond relative to the largest entry."""
+(Nc = 128 with 16 columns; Nc = 640 the columns alone), a whole pair panel
+(n = 32, nx = 224 in FP64) and the back substitution of QR / QRP pairs in a
+batch (n = 64, nx = 51: D, E, U, B and 16 columns).  A drawn solution x,
+b = A x: |x' - x| <= 50 eps cond relative to the largest entry."""
 import numpy as np
 import pytest
 
@@ -94,3 +96,21 @@ def test_pair_panel(nx, fits):
     b[:B.shape[0]] = B[:, 0]
     bt.solve(DeviceArray.from_host(b), Xd, max_iter=0, graph=False)
     assert close(s, Xd.to_host()[:x.shape[0]], x[:, 0])
+
+
+@pytest.mark.parametrize("method", [1, 2])
+@pytest.mark.parametrize("n,nx", [(64, 50), (64, 51), (64, 90), (48, 163), (48, 164), (33, 200)])
+def test_batched_qr_back_substitution(n, nx, method):
+    print(f"case back substitution n={n} nx={nx} method={method}", flush=True)
+    N, nr = 6, 2
+    s = systems.gaussian_system(N, n, nx - nr, 0, nr, nx, shift=3.0 * np.sqrt(n), seed=nx)
+    x, B = drawn(s, 1)
+    bt = Batch(mixed=False)
+    bt.plan([(N, n, nx - nr, 0, nr, nx, method), (3, 5, 1, 1, 1, 1, method)])
+    bt.generate(seed=1, shift=4.0)
+    bt.load_system(0, s)
+    Xd = DeviceArray(bt.size("x"))
+    b = np.zeros(bt.size("x"))
+    b[:B.shape[0]] = B[:, 0]
+    rc = bt.solve(DeviceArray.from_host(b), Xd, max_iter=0, graph=False)
+    assert rc in (0, 2) and close(s, Xd.to_host()[:x.shape[0]], x[:, 0])
