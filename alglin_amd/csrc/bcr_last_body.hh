@@ -59,7 +59,10 @@ struct LastLuLds {
   int piv[2][2];
 };
 
-// NANZERO: a column of NaNs counts as a zero pivot (the batched LU's answer).
+// A NaN is not a candidate (a column of NaN and zeros has a zero pivot); with
+// nothing but NaNs left the row at c stays and no zero pivot is reported.
+// NANZERO: a NaN ranks as a zero, and a column of NaNs counts as a zero pivot
+// (the batched LU's answer).
 template <int RPL, int NWV, bool NANZERO>
 __device__ __forceinline__ void lu_last_regs_body(double* Hm, int Nc, int32_t* ipiv, int32_t* st, int w, int lane,
                                                   LastLuLds<RPL>& sm) {
@@ -102,7 +105,7 @@ __device__ __forceinline__ void lu_last_regs_body(double* Hm, int Nc, int32_t* i
           unsigned h, l;
           wave::abs_key(x[k], h, l);
           if (x[k] != x[k]) h = l = 0;   // a NaN is never preferred
-          const bool cand = pos[k] >= c && lane + 64 * k < Nc;
+          const bool cand = pos[k] >= c && lane + 64 * k < Nc && (NANZERO || x[k] == x[k]);
           const bool better = cand && (!cb || h > hb || (h == hb && (l > lbits || (l == lbits && pos[k] < pb))));
           if (better) {
             cb = true;
@@ -111,6 +114,15 @@ __device__ __forceinline__ void lu_last_regs_body(double* Hm, int Nc, int32_t* i
             pb = pos[k];
             kb = k;
           }
+        }
+        if (!NANZERO && __ballot(cb) == 0) {   // only NaNs
+#pragma unroll
+          for (int k = 0; k < RPL; ++k)
+            if (pos[k] == c) {
+              cb = true;
+              pb = c;
+              kb = k;
+            }
         }
         double xs = x[0];
 #pragma unroll
