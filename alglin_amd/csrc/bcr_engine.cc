@@ -473,7 +473,7 @@ void Engine<TA, TW>::factorize_async() {
     hipError_t e = hipSuccess;
     if (!launch_small_factor(sa, st_, &e)) throw HipError("factorize: no small-system kernel");
     hip_check(e, "small factor");
-    stats_.fast_path = 1;
+    if (Ls < N) stats_.fast_path = 1;   // (else the last block only, N = 1 say)
     if (small_last) return;
   }
   // F_eff = F + sum_j Fpart[j]  (cc:823-829 / 1146-1154)
