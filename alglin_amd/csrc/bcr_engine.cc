@@ -440,7 +440,7 @@ void Engine<TA, TW>::factorize_async() {
   // the levels from Ls on in one workgroup (bcr_small.hip), the last block
   // with them; separate launches while every phase is timed
   const bool small = pure && method_ == kLU && pair_variant_ == 0 && !timing_ && n <= 16 && nx <= 8 && nr <= 8;
-  const int Ls = small ? small_factor_level(N, n, sizeof(TW), sizeof(TA) == sizeof(TW)) : N;
+  const int Ls = small ? small_factor_level(N, n, nx, nr, sizeof(TW), sizeof(TA) == sizeof(TW)) : N;
   const bool small_asm = small && int64_t(N - 1) * nr * nx <= kSmallSum;
   const bool small_last = small_asm && last_method_ == kLastLU && !last2_ && d_.Nc() <= 64;
   sa.L0 = Ls;

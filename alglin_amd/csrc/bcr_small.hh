@@ -28,7 +28,7 @@ template <typename TA, typename TW>
 hipError_t launch_prep_single(SingleArgs<TA, TW> const& a, hipStream_t st);
 
 // first level (stride) that one workgroup takes over; N when none is worth it
-int small_factor_level(int N, int n, size_t elem, bool first_ok);
+int small_factor_level(int N, int n, int nx, int nr, size_t elem, bool first_ok);
 int small_solve_level(int N, int n);
 constexpr int kSmallSum = 1 << 16;   // values one workgroup sums
 

@@ -170,8 +170,12 @@ int nmax_of(int n) { return n <= 4 ? 4 : n <= 8 ? 8 : 16; }
 // costs about what a launch of its own does.
 constexpr int kRounds = 2;
 
-int small_factor_level(int N, int n, size_t elem, bool first_ok) {
-  const int nm = nmax_of(n);
+// The round is that of the configuration the launch takes, which grows with the
+// border too (counted by n alone, n = 4 with nx = nr = 8 took eight rounds:
+// N = 1000 factor and solve 379 us, so 253).
+int small_factor_level(int N, int n, int nx, int nr, size_t elem, bool first_ok) {
+  int nm = 16;
+  pair_lu_fast_pick(n, nx, nr, [&](auto NM, auto, auto) { nm = decltype(NM)::value; });
   return first_level(N, kRounds * factor_waves(nm, elem) * (kWave / (2 * nm)), first_ok ? 1 : 2);
 }
 
