@@ -566,7 +566,7 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
   ls.U = svdU_.p; ls.V = svdV_.p; ls.S = svdS_.p; ls.rank = svd_rank_.p;
   // the levels from Ls on in one workgroup (bcr_small.hip), with the xb sum
   // and the last solve between its two sweeps where they fit one too
-  const bool small = used_P_ == 1 && method_ == kLU && sweep_fast_ && !timing_ && n <= 16 && nrhs <= 4;
+  const bool small = used_P_ == 1 && method_ == kLU && !timing_ && n <= 16 && nrhs <= 4;
   const int Ls = small ? small_solve_level(N, n) : N;
   SmallSolveArgs<TW, TX> ss{};
   ss.s = a;
@@ -587,12 +587,11 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
     a.pairs = l.off >= 0 ? pairtab_.p + l.off : nullptr;
     timed(kForward, [&] {
       hipError_t e = hipSuccess;
-      if (method_ == kLU && sweep_fast_ &&
-          ((sweep_mfma(n, nrhs, a.npairs) && launch_sweep_lu_mfma(true, a, st_, &e)) || launch_sweep_lu_fast(true, a, st_, &e) || launch_sweep_lu_stream(true, a, st_, &e)))
-        hip_check(e, "forward_fast");
-      else if (method_ != kLU && sweep_fast_ && launch_forward_qr(a, st_, &e))
-        hip_check(e, "forward_qr");
-      else hip_check(launch_forward(method_, a, st_), "forward");
+      const bool ran = method_ != kLU ? launch_forward_qr(a, st_, &e)
+                                      : (sweep_mfma(n, nrhs, a.npairs) && launch_sweep_lu_mfma(true, a, st_, &e)) ||
+                                            launch_sweep_lu_fast(true, a, st_, &e) || launch_sweep_lu_stream(true, a, st_, &e);
+      if (!ran) throw HipError("solve: no forward sweep kernel");
+      hip_check(e, "forward");
     });
   }
   if (small_last) run_small(kSmallFwd | kSmallXb | kSmallLast | kSmallBwd);
@@ -618,12 +617,11 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
       // the back substitution of a QR pair is the LU one (R where U sits);
       // QRP adds the pair's column exchanges (the streamed sweep's exch)
       a.exch = method_ == kQRP ? 1 : 0;
-      if ((method_ == kLU || method_ == kQR) && sweep_fast_ &&
-          ((sweep_mfma(n, nrhs, a.npairs) && launch_sweep_lu_mfma(false, a, st_, &e)) || launch_sweep_lu_fast(false, a, st_, &e) || launch_sweep_lu_stream(false, a, st_, &e)))
-        hip_check(e, "backward_fast");
-      else if (method_ == kQRP && sweep_fast_ && launch_sweep_lu_stream(false, a, st_, &e))
-        hip_check(e, "backward_stream");
-      else hip_check(launch_backward(method_, a, st_), "backward");
+      const bool ran = (method_ != kQRP && ((sweep_mfma(n, nrhs, a.npairs) && launch_sweep_lu_mfma(false, a, st_, &e)) ||
+                                            launch_sweep_lu_fast(false, a, st_, &e))) ||
+                       launch_sweep_lu_stream(false, a, st_, &e);
+      if (!ran) throw HipError("solve: no backward sweep kernel");
+      hip_check(e, "backward");
       a.exch = 0;
     });
   }

@@ -100,11 +100,9 @@ class Engine {
   int last_method() const { return last_method_; }
   // second last-block solver (SVD path) used when the first fails
   void set_last2(bool on) { last2_ = on; }
-  // LU solves with n <= 32 use the wave-synchronous sweep kernels unless off
-  void set_sweep_fast(bool on) { sweep_fast_ = on; }
   // LU pair kernel choice: 0 default (see level_factor), 3 the
   // register-tiled kernel for every n, 4 column-split waves, 5 the
-  // matrix-core pair (FP32 factors)
+  // matrix-core pair
   void set_pair_variant(int v) { pair_variant_ = v; }
   int method() const { return method_; }
 
@@ -151,7 +149,9 @@ class Engine {
   size_t pending_count() const { return Cpend_.count; }
   FactorStats const& stats() const { return stats_; }
 
-  // per-phase timing with HIP events on the engine stream (see alglin_amd.h)
+  // per-phase timing with HIP events on the engine stream (see alglin_amd.h);
+  // while on, systems with n <= 16 take a launch per level instead of the
+  // fused ones
   enum Phase { kPair = 0, kForward = 1, kBackward = 2, kLast = 3, kReduce = 4, kResidual = 5 };
   void set_timing(bool on) { timing_ = on; }
   void timing(double out[8], bool reset);
@@ -183,7 +183,6 @@ class Engine {
   int method_ = kLU;
   int last_method_ = kLastLU;
   bool last2_ = false;
-  bool sweep_fast_ = true;
   int pair_variant_ = 0;
   hipStream_t st_ = nullptr;
   bool own_stream_ = true;

@@ -88,18 +88,8 @@ __device__ __forceinline__ double rl_after(double v, int who, int cc) {
 
 // columns K.. 15 of one 16-column block of the row sets, those not after
 // column cc of the block getting a zero pivot-row entry; the pivot row is in
-// row set 0 or 1 (a third row set holds border rows only)
-// f(integral_constant<int, I>) for I = B .. E-1, unrolled at compile time
-template <int B, int E, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (B < E) {
-    f(std::integral_constant<int, B>{});
-    static_for<B + 1, E>(f);
-  }
-}
-
-// Columns before KM may lie at or before cc and are masked; the later ones
-// always lie after it.
+// row set 0 or 1 (a third row set holds border rows only).  Columns before KM
+// may lie at or before cc and are masked; the later ones always lie after it.
 template <int K, int KM, int RS, int SP, typename TW>
 __device__ __forceinline__ void update_after(V16<TW>& v0, V16<TW>& v1, V16<TW>& v2, bool sp, int who, int cc, TW lv0,
                                              TW lv1, TW lv2) {
@@ -205,9 +195,6 @@ struct PanelLds {
   alignas(16) TW u[16 * ULD];
   alignas(16) TW lk[16 * 16];
 };
-
-// the LDS accesses of a wave are in order; this keeps the compiler's so
-__device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 template <int B, int NB, int RS, typename TW>
 __device__ __forceinline__ void trailing_update(V16<TW> (&V)[RS][NB], PanelLds<TW, NB>& sm, int pos0, int pos1, int n,
@@ -475,11 +462,9 @@ __device__ __forceinline__ void pair_lu_t_body(FactorArgs<TS, TW> const& a, int 
 template <typename TW, int NB, int RS>
 struct PanelWavesLds {
   static constexpr int TILES = (2 * 16 * NB + kNrB + 15) / 16, RLD = 16 * TILES + 2, ULD = 18;
-  // (two blocks: wave 1 is the only reader of block 0, and needs no second set)
-  static constexpr int SETS = NB == 2 ? 1 : 2;
-  alignas(16) TW x[SETS][16 * RLD];     // multipliers by row (as in PanelLds::x)
+  alignas(16) TW x[2][16 * RLD];        // multipliers by row (as in PanelLds::x)
   alignas(16) TW u[NB - 1][16 * ULD];   // waves 1 ..: the pivot rows of their blocks
-  alignas(16) TW lk[SETS][16 * 16];
+  alignas(16) TW lk[2][16 * 16];
   uint8_t pos[2][128];
 };
 
@@ -488,6 +473,7 @@ struct PanelWavesLds {
 // (every tile tried for a single system too: n = 53, 9001 rows 4255 -> 4284 us).
 template <typename TS, typename TW, int NB, int RS, bool BATCH>
 __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int p) {
+  static_assert(NB >= 3, "one wave takes two blocks (times above)");
   using Lds = PanelWavesLds<TW, NB, RS>;
   constexpr int TILES = Lds::TILES, RLD = Lds::RLD, ULD = Lds::ULD;
   __shared__ Lds sm;
@@ -533,8 +519,8 @@ __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int
 
     for (int b = 0; b < w; ++b) {
       __syncthreads();
-      TW const* const x = sm.x[b & (Lds::SETS - 1)];
-      TW const* const lk = sm.lk[b & (Lds::SETS - 1)];
+      TW const* const x = sm.x[b & 1];
+      TW const* const lk = sm.lk[b & 1];
       // the block's pivot rows of this wave's columns, solved with its unit
       // lower triangle, a column per lane
       TW* const u = sm.u[w - 1];
@@ -579,7 +565,7 @@ __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int
 
     // to the row layout through the place its multipliers will take (its last
     // readers have passed the barrier before)
-    TW* const x = sm.x[w & (Lds::SETS - 1)];
+    TW* const x = sm.x[w & 1];
 #pragma unroll
     for (int t = 0; t < TILES; ++t)
 #pragma unroll
@@ -612,7 +598,7 @@ __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int
   sm.pos[w & 1][lane] = uint8_t(rows.pos0);
   sm.pos[w & 1][lane + 64] = uint8_t(rows.pos1);
   if (w < NB - 1) {
-    TW* const x = sm.x[w & (Lds::SETS - 1)];
+    TW* const x = sm.x[w & 1];
     lds_order();
 #pragma unroll
     for (int s = 0; s < RS; ++s) {
@@ -624,7 +610,7 @@ __device__ __forceinline__ void pair_lu_tw_body(FactorArgs<TS, TW> const& a, int
       }
       if (s < 2 && q >= 0 && q < 16) {
 #pragma unroll
-        for (int k = 0; k < 16; ++k) sm.lk[w & (Lds::SETS - 1)][k * 16 + q] = V[s][k];
+        for (int k = 0; k < 16; ++k) sm.lk[w & 1][k * 16 + q] = V[s][k];
       }
     }
   }
@@ -1198,6 +1184,9 @@ void launch_pair_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, h
     hipLaunchKernelGGL((pair_lu_tw_batched<TS, TW, NB, RS>), pairs, dim3(64 * NB), 0, st, t);
   else
     hipLaunchKernelGGL((pair_lu_t_batched<TS, TW, NB, RS, kNrB>), pairs, dim3(64), 0, st, t);
+  // (four waves may wait here for room behind the other stream's workgroups;
+  // the calls are level with two: batches of 1024 uneven systems FP64 43.9 /
+  // 43.5 ms, FP32 32.8 / 32.5, half of them nearly singular 42.3 / 42.6)
   if (nblocks <= kFewPairs) hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWavesFew>), pairs, dim3(64 * kRhsWavesFew), 0, st, t);
   else hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWaves>), pairs, dim3(64 * kRhsWaves), 0, st, t);
 }

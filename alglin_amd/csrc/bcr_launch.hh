@@ -45,14 +45,11 @@ bool pair_lu_mfma_fits(int n, int nr, int nx);
 template <typename TS, typename TW>
 bool launch_pair_lu_mfma(FactorArgs<TS, TW> const& a, hipStream_t st, hipError_t* err);
 
-template <typename TW, typename TX>
-hipError_t launch_forward(int method, SolveArgs<TW, TX> const& a, hipStream_t st);
-template <typename TW, typename TX>
-hipError_t launch_backward(int method, SolveArgs<TW, TX> const& a, hipStream_t st);
-// streamed LU sweeps, one wavefront per pair (n <= 64)
 // forward sweep of a QR or QRP pair, n <= 64
 template <typename TW, typename TX>
 bool launch_forward_qr(SolveArgs<TW, TX> const& a, hipStream_t st, hipError_t* err);
+// streamed LU sweeps, one wavefront per pair (n <= 64); backward also QR and
+// QRP pairs
 template <typename TW, typename TX>
 bool launch_sweep_lu_stream(bool forward, SolveArgs<TW, TX> const& a, hipStream_t st, hipError_t* err);
 // matrix-core LU sweeps, several right-hand sides (n <= 64, nr <= 16)

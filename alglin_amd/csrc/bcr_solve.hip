@@ -1,11 +1,11 @@
-// Solve-phase kernels of the bordered cyclic reduction.
+// Sweeps of QR and QRP pairs in a batch, and the boundary sums.
 //
-//   forward_kernel   one level of the forward sweep (cc:1615-1719): replays the
+//   forward_body     one level of the forward sweep (cc:1615-1719): replays the
 //                    pair transform on (x_jp, x_j) and writes the border partial
 //                    -C_j' x_j to Xpart[j]
-//   backward_kernel  one level of the back substitution (cc:1805-1949):
-//                    x_j = U^{-1}(x_j - D_j x_jp - E_j x_jpp - B_j xb), QRP swaps
-//   reduce_add       dst += sum_j part[j] (deterministic two-pass tree)
+//   backward_body    one level of the back substitution (cc:1805-1949):
+//                    x_j = R^{-1}(x_j - D_j x_jp - E_j x_jpp - B_j xb), QRP swaps
+//   launch_reduce    dst += sum_j part[j] (deterministic two-pass tree)
 //
 // One workgroup per pair; the pair's factor blocks are staged into LDS with
 // coalesced loads (all in flight at once), the short sequential recurrences
@@ -16,7 +16,7 @@
 namespace bcr {
 
 
-template <typename TW, typename TX, int METHOD>
+template <typename TW, typename TX>
 __device__ __forceinline__ void forward_body(SolveArgs<TW, TX> a, int bid) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int p = bid;
@@ -27,12 +27,9 @@ __device__ __forceinline__ void forward_body(SolveArgs<TW, TX> a, int bid) {
   const int tid = threadIdx.x, nth = blockDim.x;
   TW* Tp = reinterpret_cast<TW*>(smem_raw);                                     // 2n*n + n
   TX* X = reinterpret_cast<TX*>(smem_raw + align16(tsize(n) * sizeof(TW)));   // 2n*kRhsChunk
-  __shared__ int s_perm[64];
 
   const TW* Tj = a.Tm + size_t(j) * tsize(n);
-  const int tcount = (METHOD == kLU) ? n2 * n : int(tsize(n));
-  for (int i = tid; i < tcount; i += nth) Tp[i] = Tj[i];
-  for (int i = tid; i < n; i += nth) s_perm[i] = a.perm[size_t(j) * n + i];
+  for (int i = tid; i < int(tsize(n)); i += nth) Tp[i] = Tj[i];
 
   for (int q0 = 0; q0 < a.nrhs; q0 += kRhsChunk) {
     const int nq = min(kRhsChunk, a.nrhs - q0);
@@ -42,48 +39,31 @@ __device__ __forceinline__ void forward_body(SolveArgs<TW, TX> a, int bid) {
       X[r + q * n2] = a.x[row + size_t(q0 + q) * a.ldx];
     }
     __syncthreads();
-    if (METHOD == kLU) {
-      // row interchanges first (laswp on rows 1..n, cc:939), then L^{-1}
-      for (int q = tid; q < nq; q += nth)
-        for (int c = 0; c < n; ++c) {
-          const int pv = s_perm[c] - 1;
-          if (pv != c) { TX t = X[c + q * n2]; X[c + q * n2] = X[pv + q * n2]; X[pv + q * n2] = t; }
-        }
-      __syncthreads();
+    // Q^T = H_{n-1} ... H_0 (ormqr 'L','T', cc:962-971): one wave per
+    // right-hand side, its rows lane and lane + 64 (2n <= 128) in
+    // registers; per reflector a wave dot product (a butterfly: every
+    // lane ends with the same sum) and an axpy, no barrier
+    const int lane = tid & 63, wv = tid >> 6, nw = nth >> 6;
+    for (int q = wv; q < nq; q += nw) {
+      TX* xq = X + q * n2;
+      TX x0 = lane < n2 ? xq[lane] : TX(0);
+      TX x1 = lane + 64 < n2 ? xq[lane + 64] : TX(0);
       for (int c = 0; c < n; ++c) {
-        for (int i = tid; i < (n2 - c - 1) * nq; i += nth) {
-          const int r = c + 1 + i % (n2 - c - 1), q = i / (n2 - c - 1);
-          X[r + q * n2] -= TX(Tp[r + c * n2]) * X[c + q * n2];
-        }
-        __syncthreads();
-      }
-    } else {
-      // Q^T = H_{n-1} ... H_0 (ormqr 'L','T', cc:962-971): one wave per
-      // right-hand side, its rows lane and lane + 64 (2n <= 128) in
-      // registers; per reflector a wave dot product (a butterfly: every
-      // lane ends with the same sum) and an axpy, no barrier
-      const int lane = tid & 63, wv = tid >> 6, nw = nth >> 6;
-      for (int q = wv; q < nq; q += nw) {
-        TX* xq = X + q * n2;
-        TX x0 = lane < n2 ? xq[lane] : TX(0);
-        TX x1 = lane + 64 < n2 ? xq[lane + 64] : TX(0);
-        for (int c = 0; c < n; ++c) {
-          const TX tau = TX(Tp[size_t(n2) * n + c]);
-          // v = (1 at row c, the stored reflector below it); row c < 64
-          const TX v0 = lane == c ? TX(1) : (lane > c && lane < n2 ? TX(Tp[lane + c * n2]) : TX(0));
-          const TX v1 = lane + 64 < n2 ? TX(Tp[lane + 64 + c * n2]) : TX(0);
-          TX d = fma(v0, x0, v1 * x1);
+        const TX tau = TX(Tp[size_t(n2) * n + c]);
+        // v = (1 at row c, the stored reflector below it); row c < 64
+        const TX v0 = lane == c ? TX(1) : (lane > c && lane < n2 ? TX(Tp[lane + c * n2]) : TX(0));
+        const TX v1 = lane + 64 < n2 ? TX(Tp[lane + 64 + c * n2]) : TX(0);
+        TX d = fma(v0, x0, v1 * x1);
 #pragma unroll
-          for (int off = 32; off >= 1; off >>= 1) d += __shfl_xor(d, off);
-          const TX w = d * tau;
-          x0 = fma(-v0, w, x0);
-          x1 = fma(-v1, w, x1);
-        }
-        if (lane < n2) xq[lane] = x0;
-        if (lane + 64 < n2) xq[lane + 64] = x1;
+        for (int off = 32; off >= 1; off >>= 1) d += __shfl_xor(d, off);
+        const TX w = d * tau;
+        x0 = fma(-v0, w, x0);
+        x1 = fma(-v1, w, x1);
       }
-      __syncthreads();
+      if (lane < n2) xq[lane] = x0;
+      if (lane + 64 < n2) xq[lane + 64] = x1;
     }
+    __syncthreads();
     // TOP (x_jp) <- W[n:2n], BOTTOM (x_j) <- W[0:n]   (cc:1041-1042)
     for (int i = tid; i < n2 * nq; i += nth) {
       const int r = i % n2, q = i / n2;
@@ -101,12 +81,6 @@ __device__ __forceinline__ void forward_body(SolveArgs<TW, TX> a, int bid) {
     __syncthreads();
   }
 }
-
-template <typename TW, typename TX, int METHOD>
-__global__ void __launch_bounds__(128) forward_kernel(SolveArgs<TW, TX> a) {
-  forward_body<TW, TX, METHOD>(a, blockIdx.x);
-}
-
 
 // WIDE: one column at a time and B_j read where it lies, for borders (nx) whose
 // B_j and 16 columns of x_b do not fit the LDS beside D_j, E_j and U
@@ -192,12 +166,6 @@ __device__ __forceinline__ void backward_body(SolveArgs<TW, TX> a, int bid) {
   }
 }
 
-template <typename TW, typename TX, int METHOD>
-__global__ void __launch_bounds__(128) backward_kernel(SolveArgs<TW, TX> a) {
-  backward_body<TW, TX, METHOD, false>(a, blockIdx.x);
-}
-
-
 // part: [count][m] (column j of the partial sums), dst[i] += sum_j part[j][i],
 // dst index i maps to dst[(i % mrow) + (i / mrow) * ldd].
 template <typename TP, typename TD>
@@ -248,31 +216,11 @@ __global__ void __launch_bounds__(64) reduce_final_kernel(const TP* __restrict__
   if (threadIdx.x == 0) dst[(i % mrow) + size_t(i / mrow) * ldd] += TD(s);
 }
 
-template <typename TW, typename TX>
-hipError_t launch_forward(int method, SolveArgs<TW, TX> const& a, hipStream_t st) {
-  const size_t bytes = align16(tsize(a.n) * sizeof(TW)) + size_t(2 * a.n) * kRhsChunk * sizeof(TX);
-  dim3 grid(a.npairs), block(a.n <= 32 ? 64 : 128);
-  if (method == kLU) hipLaunchKernelGGL((forward_kernel<TW, TX, kLU>), grid, block, bytes, st, a);
-  else hipLaunchKernelGGL((forward_kernel<TW, TX, kQR>), grid, block, bytes, st, a);
-  return hipGetLastError();
-}
-
-template <typename TW, typename TX>
-hipError_t launch_backward(int method, SolveArgs<TW, TX> const& a, hipStream_t st) {
-  const size_t nn = size_t(a.n) * a.n;
-  const size_t bytes = align16((3 * nn + size_t(a.n) * a.nx) * sizeof(TW)) +
-                       (size_t(3 * a.n + a.nx) + a.n) * kRhsChunk * sizeof(TX);
-  dim3 grid(a.npairs), block(a.n <= 32 ? 64 : 128);
-  if (method == kQRP) hipLaunchKernelGGL((backward_kernel<TW, TX, kQRP>), grid, block, bytes, st, a);
-  else hipLaunchKernelGGL((backward_kernel<TW, TX, kLU>), grid, block, bytes, st, a);
-  return hipGetLastError();
-}
-
 template <typename TW, typename TX, int METHOD, bool FWD, bool WIDE = false>
 __global__ void __launch_bounds__(128) sweep_generic_batched(BatchTable<SolveArgs<TW, TX>> t) {
   const int e = t.entry[blockIdx.x];
   if (skipped(t.args[e].skip)) return;
-  if (FWD) forward_body<TW, TX, METHOD>(t.args[e], int(blockIdx.x) - t.first[e]);
+  if (FWD) forward_body<TW, TX>(t.args[e], int(blockIdx.x) - t.first[e]);
   else backward_body<TW, TX, METHOD, WIDE>(t.args[e], int(blockIdx.x) - t.first[e]);
 }
 
@@ -289,16 +237,12 @@ hipError_t launch_sweep_generic_batched(bool forward, int method, BatchTable<Sol
     const size_t wbytes = align16(3 * nn * sizeof(TW)) + (size_t(3 * n + nx) + n) * sizeof(TX);
     if (wbytes + kPerm > lds_limit) return hipErrorInvalidConfiguration;
     if (method == kQRP) hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQRP, false, true>), grid, block, wbytes, st, t);
-    else hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kLU, false, true>), grid, block, wbytes, st, t);
+    else hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQR, false, true>), grid, block, wbytes, st, t);
     return hipGetLastError();
   }
-  if (forward) {
-    if (method == kLU) hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kLU, true>), grid, block, fbytes, st, t);
-    else hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQR, true>), grid, block, fbytes, st, t);
-  } else {
-    if (method == kQRP) hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQRP, false>), grid, block, bbytes, st, t);
-    else hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kLU, false>), grid, block, bbytes, st, t);
-  }
+  if (forward) hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQR, true>), grid, block, fbytes, st, t);
+  else if (method == kQRP) hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQRP, false>), grid, block, bbytes, st, t);
+  else hipLaunchKernelGGL((sweep_generic_batched<TW, TX, kQR, false>), grid, block, bbytes, st, t);
   return hipGetLastError();
 }
 
@@ -321,12 +265,6 @@ hipError_t launch_reduce(const TP* part, int first, int count, int m, TP* tmp, i
   return hipGetLastError();
 }
 
-template hipError_t launch_forward<double, double>(int, SolveArgs<double, double> const&, hipStream_t);
-template hipError_t launch_forward<float, float>(int, SolveArgs<float, float> const&, hipStream_t);
-template hipError_t launch_forward<float, double>(int, SolveArgs<float, double> const&, hipStream_t);
-template hipError_t launch_backward<double, double>(int, SolveArgs<double, double> const&, hipStream_t);
-template hipError_t launch_backward<float, float>(int, SolveArgs<float, float> const&, hipStream_t);
-template hipError_t launch_backward<float, double>(int, SolveArgs<float, double> const&, hipStream_t);
 template hipError_t launch_reduce<double, double>(const double*, int, int, int, double*, int, double*, int, int64_t,
                                                   hipStream_t);
 template hipError_t launch_reduce<float, float>(const float*, int, int, int, float*, int, float*, int, int64_t,

@@ -16,24 +16,15 @@
 //            (half 0 of the group forms D_j x_jp + B_j xb, half 1 E_j x_jpp)
 #pragma once
 #include "bcr_launch.hh"
+#include "bcr_wave.hh"
 
 namespace bcr {
 namespace {
 
-__device__ __forceinline__ double rlane(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(int(b & 0xffffffff), l);
-  const int hi = __builtin_amdgcn_readlane(int(b >> 32), l);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-__device__ __forceinline__ float rlane(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
 // value of lane base+idx of the group; for G == 64 idx must be wave-uniform
 template <int G, typename T>
 __device__ __forceinline__ T gbcast(T v, int base, int idx) {
-  if constexpr (G == 64) return rlane(v, idx);
+  if constexpr (G == 64) return wave::rl(v, idx);
   else return __shfl(v, base + idx, 64);
 }
 
@@ -216,7 +207,7 @@ __device__ __forceinline__ void backward_lu_fast_body(SolveArgs<TW, TX> const& a
         for (int q = 0; q < QB; ++q) {
           TX v;
           if constexpr (G == 64) {
-            const TX v0 = rlane(vin[q], c), v1 = rlane(vin[q], NMAX + c);
+            const TX v0 = wave::rl(vin[q], c), v1 = wave::rl(vin[q], NMAX + c);
             v = h == 0 ? v0 : v1;
           } else {
             v = __shfl(vin[q], base + h * NMAX + c, 64);

@@ -30,16 +30,18 @@ __global__ void __launch_bounds__(256) sweep_lu_fast_batched(BatchTable<SolveArg
   else backward_lu_fast_body<TW, TX, NMAX, QB>(t.args[e], sweep_wave(int(blockIdx.x) - t.first[e]));
 }
 
+// four columns at a time only for n <= 8: beyond, several columns go through
+// the matrix cores (all but some 10^6 of them, which its grid does not hold)
 template <typename TW, typename TX, int NMAX>
 hipError_t launch_sweep_nmax(bool forward, SolveArgs<TW, TX> const& a, hipStream_t st) {
-  constexpr int PG = 64 / (2 * NMAX);
+  constexpr int PG = 64 / (2 * NMAX), QB = NMAX <= 8 ? 4 : 1;
   const int blocks = (a.npairs + 4 * PG - 1) / (4 * PG);
   if (forward) {
     if (a.nrhs == 1) hipLaunchKernelGGL((forward_lu_fast_kernel<TW, TX, NMAX, 1>), dim3(blocks), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((forward_lu_fast_kernel<TW, TX, NMAX, 4>), dim3(blocks), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((forward_lu_fast_kernel<TW, TX, NMAX, QB>), dim3(blocks), dim3(256), 0, st, a);
   } else {
     if (a.nrhs == 1) hipLaunchKernelGGL((backward_lu_fast_kernel<TW, TX, NMAX, 1>), dim3(blocks), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((backward_lu_fast_kernel<TW, TX, NMAX, 4>), dim3(blocks), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((backward_lu_fast_kernel<TW, TX, NMAX, QB>), dim3(blocks), dim3(256), 0, st, a);
   }
   return hipGetLastError();
 }

@@ -126,9 +126,6 @@ __device__ __forceinline__ void solve_upper(D4& acc, D4 const& d, int lim, int g
   }
 }
 
-// the LDS accesses of a wave are in order; this keeps the compiler's so
-__device__ __forceinline__ void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
-
 // waves per SIMD asked of the compiler (it would otherwise load ahead into
 // every register)
 constexpr int mfma_waves(int nb) { return nb <= 2 ? 3 : 2; }

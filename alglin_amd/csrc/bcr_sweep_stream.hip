@@ -18,13 +18,6 @@
 namespace bcr {
 namespace {
 
-__device__ __forceinline__ double rlane(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(int(b & 0xffffffff), l);
-  const int hi = __builtin_amdgcn_readlane(int(b >> 32), l);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-}
-
 __device__ __forceinline__ double wsum(double v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
@@ -94,7 +87,7 @@ __device__ __forceinline__ void forward_lu_stream_body(SolveArgs<TW, TX> a, int 
         if (c < n) {
 #pragma unroll
           for (int b = 0; b < QB; ++b) {
-            const TX xc = TX(rlane(double(x0[b]), c));
+            const TX xc = TX(wave::rl(double(x0[b]), c));
             if (r0 > c) x0[b] -= TX(t0[i]) * xc;
             x1[b] -= TX(t1[i]) * xc;
           }
@@ -247,7 +240,7 @@ __device__ __forceinline__ void backward_lu_stream_body(SolveArgs<TW, TX> a, int
   #pragma unroll
         for (int i = 0; i < kChunk; ++i) {
           const int c = c0 + i;
-          if (c < n) s -= TX(d[i]) * TX(rlane(double(vjp), c)) + TX(e[i]) * TX(rlane(double(vjpp), c));
+          if (c < n) s -= TX(d[i]) * TX(wave::rl(double(vjp), c)) + TX(e[i]) * TX(wave::rl(double(vjpp), c));
         }
       }
       // B_j xb: the two columns above, then eight columns' loads in flight
@@ -281,7 +274,7 @@ __device__ __forceinline__ void backward_lu_stream_body(SolveArgs<TW, TX> a, int
         for (int i = 0; i < kChunk; ++i) {
           const int c = c1 - i;
           if (c >= 0) {
-            const TX xc = TX(rlane(double(s * dinv), c));
+            const TX xc = TX(wave::rl(double(s * dinv), c));
             if (lane < c) s -= TX(u[i]) * xc;
             else if (lane == c) s = xc;
           }
@@ -316,7 +309,7 @@ __device__ __forceinline__ void backward_lu_stream_body(SolveArgs<TW, TX> a, int
           if (c < n) {
   #pragma unroll
             for (int b = 0; b < QB; ++b)
-              s[b] -= TX(d[i]) * TX(rlane(double(vjp[b]), c)) + TX(e[i]) * TX(rlane(double(vjpp[b]), c));
+              s[b] -= TX(d[i]) * TX(wave::rl(double(vjp[b]), c)) + TX(e[i]) * TX(wave::rl(double(vjpp[b]), c));
           }
         }
       }
@@ -353,7 +346,7 @@ __device__ __forceinline__ void backward_lu_stream_body(SolveArgs<TW, TX> a, int
           if (c >= 0) {
   #pragma unroll
             for (int b = 0; b < QB; ++b) {
-              const TX xc = TX(rlane(double(s[b] * dinv), c));
+              const TX xc = TX(wave::rl(double(s[b] * dinv), c));
               if (lane < c) s[b] -= TX(u[i]) * xc;
               else if (lane == c) s[b] = xc;
             }
@@ -397,7 +390,7 @@ __device__ __forceinline__ void backward_lu_stream2_body(SolveArgs<TW, TX> a, in
   const unsigned od = dj * unsigned(nn) + unsigned(rc), ob = dj * unsigned(n * nx) + unsigned(rc);
   const unsigned ot = dj * unsigned(tsize(n)) + unsigned(rc);
   auto bc = [&](TX v, int c) -> TX {
-    const TX v0 = TX(rlane(double(v), c)), v1 = TX(rlane(double(v), 32 + c));
+    const TX v0 = TX(wave::rl(double(v), c)), v1 = TX(wave::rl(double(v), 32 + c));
     return h ? v1 : v0;
   };
   const TX dinv = row ? TX(1) / TX(gload(Tw, ot + unsigned(rc) * n2)) : TX(1);
