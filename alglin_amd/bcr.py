@@ -341,6 +341,9 @@ class BorderedCR:
                     status=int(out[3]), backward_error=float(out[4]))
 
     def set_timing(self, on=True):
+        """Per-phase GPU times from now on (timing()).  While on, LU systems with
+        n <= 16 take a launch per level instead of the fused ones: same factors,
+        but the phases' sum exceeds the untimed call's time."""
         self._check(lib().alglin_bcr_set_timing(self._h, int(on)), "set_timing")
 
     def timing(self, reset=True) -> dict:

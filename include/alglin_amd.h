@@ -166,7 +166,12 @@ int alglin_bcr_set_fallback(alglin_bcr_t h, int on);
 int alglin_bcr_refine_report(alglin_bcr_t h, double out[5]);
 
 /* ---- per-phase GPU timing (HIP events on the handle's stream) --------------- */
-/* on=1 records an event pair around every launch group from now on */
+/* on=1 records an event pair around every launch group from now on.  The
+   phases can be told apart only where they are launches of their own: while
+   timing is on, LU systems with n <= 16 take a launch per level instead of the
+   fused ones (small levels, boundary sums and last block in one launch each
+   way), with the same factors, so the phases' sum exceeds the untimed call's
+   time. */
 int alglin_bcr_set_timing(alglin_bcr_t h, int on);
 /* accumulated milliseconds since the last reset and launch counts:
    out[0] pair eliminations  out[1] forward sweeps  out[2] backward sweeps
