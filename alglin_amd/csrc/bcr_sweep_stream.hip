@@ -115,7 +115,9 @@ __device__ __forceinline__ void forward_lu_stream_body(SolveArgs<TW, TX> a, int 
 // (ONE: 2n <= 64), the reflectors streamed kChunk columns at a time, v^T x as a
 // wave sum.  The chain of the n sums bounds a small level (n = 32 FP64: a
 // workgroup with T in LDS and ds_bpermute sums 30 us, this 8); the first
-// level of 10000 pairs 253 -> 52 us (164 MB of factors).
+// level of 10000 pairs 253 -> 52 us (164 MB of factors).  With few rows and many
+// columns the memory round trips of a pass of QB columns are all there is, so its
+// loads are in flight together (n = 1, N = 300, 64 columns: 60 -> 35 us a level).
 template <typename TW, typename TX, bool ONE, int QB>
 __device__ __forceinline__ void forward_qr_stream_body(SolveArgs<TW, TX> const& a, int bid) {
   const int lane = threadIdx.x & 63;
@@ -148,11 +150,12 @@ __device__ __forceinline__ void forward_qr_stream_body(SolveArgs<TW, TX> const& 
 #pragma unroll
     for (int b = 0; b < QB; ++b) {
       const TX* x = a.x + size_t(q0 + b < nrhs ? q0 + b : nrhs - 1) * a.ldx;
-      x0[b] = v0 ? x[in0] : TX(0);
-      x1[b] = v1 ? x[in1] : TX(0);
+      const TX y0 = x[in0], y1 = ONE ? TX(0) : x[in1];   // (valid rows: all loads in flight)
+      x0[b] = keep_if(y0, v0);
+      x1[b] = ONE ? TX(0) : keep_if(y1, v1);
     }
     for (int c0 = 0; c0 < n; c0 += kChunk) {
-      if (c0 > 0 || q0 > 0) load_chunk(c0);
+      if (c0 > 0 || (q0 > 0 && n > kChunk)) load_chunk(c0);
 #pragma unroll
       for (int i = 0; i < kChunk; ++i) {
         const int c = c0 + i;
@@ -176,10 +179,14 @@ __device__ __forceinline__ void forward_qr_stream_body(SolveArgs<TW, TX> const& 
         TX* x = a.x + size_t(q) * a.ldx;
         if (v0) x[out0] = x0[b];
         if (v1) x[out1] = x1[b];
-        for (int i = 0; i < nr; ++i) {
-          const TX s = wave::sum(lane < n ? TX(Cj[i + size_t(lane) * nr]) * x0[b] : TX(0));
-          if (lane == 0) a.Xpart[size_t(j) * nr * nrhs + i + size_t(q) * nr] = -s;
-        }
+      }
+    }
+    for (int i = 0; i < nr; ++i) {
+      const TX c = keep_if(TX(gload(Cj, unsigned(i) + unsigned(lane < n ? lane : 0) * unsigned(nr))), lane < n);
+#pragma unroll
+      for (int b = 0; b < QB; ++b) {
+        const TX s = wave::sum(c * (lane < n ? x0[b] : TX(0)));
+        if (lane == 0 && q0 + b < nrhs) a.Xpart[size_t(j) * nr * nrhs + i + size_t(q0 + b) * nr] = -s;
       }
     }
   }
