@@ -567,7 +567,7 @@ void Engine<TA, TW>::solve_async(TX* x, int nrhs, int64_t ldx) {
   // the levels from Ls on in one workgroup (bcr_small.hip), with the xb sum
   // and the last solve between its two sweeps where they fit one too
   const bool small = used_P_ == 1 && method_ == kLU && !timing_ && n <= 16 && nrhs <= 4;
-  const int Ls = small ? small_solve_level(N, n) : N;
+  const int Ls = small ? small_solve_level(N, n, nr, nrhs, sizeof(TX)) : N;
   SmallSolveArgs<TW, TX> ss{};
   ss.s = a;
   ss.L0 = Ls;

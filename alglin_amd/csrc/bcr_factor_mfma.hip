@@ -16,9 +16,10 @@
 //     steps that update the block's columns from the group's first on).  In
 //     FP64 the trailing blocks take a block's 16 steps at once on the matrix
 //     cores (trailing_update); in FP32 each step updates them (a lane read
-//     and two FMAs per column: the way through LDS costs as much).  VALU
-//     issue bounds it: N = 100000, n = 32 FP64, first level 909 -> 750 us
-//     with the blocked update (loads and stores alone are 0.4 ms).  Rows do
+//     and two FMAs per column: the way through LDS costs as much).  The
+//     steps' chain at two waves per SIMD bounds it, VALU issue next (57 %
+//     busy): N = 100000, n = 32 FP64, first level 909 -> 750 us with the
+//     blocked update, 711 now (loads and stores alone are 0.4 ms).  Rows do
 //     not move; each row is stored at its final position (T, C_j U^-1, perm),
 //     and the positions themselves go to the unused tail of T (one byte per
 //     row).  pair_lu_tw: the same by a wave per block, FP64 beyond n = 48 and
@@ -45,7 +46,7 @@
 //     for loads behind stores waits for those: 1.62 -> 1.27 ms at N = 100000,
 //     n = 32 FP64, first level), the operands live in registers instead of
 //     LDS (more pairs per CU), and stores are whole runs (1.41 ms with
-//     operands in LDS and stores by column; now 0.97 ms, 3.2 TB/s).
+//     operands in LDS and stores by column; now 0.98 ms, 3.9 TB/s with T).
 //     The right-hand part of a QR pair (pair_qr_rhs) is the same kernel with
 //     other products: 16 reflectors at a time as I - V T V^T (dlarft), V in
 //     LDS, x + V (-T^T (V^T x)) with the tile's rows in registers throughout.

@@ -29,7 +29,7 @@ hipError_t launch_prep_single(SingleArgs<TA, TW> const& a, hipStream_t st);
 
 // first level (stride) that one workgroup takes over; N when none is worth it
 int small_factor_level(int N, int n, int nx, int nr, size_t elem, bool first_ok);
-int small_solve_level(int N, int n);
+int small_solve_level(int N, int n, int nr, int nrhs, size_t elem);
 constexpr int kSmallSum = 1 << 16;   // values one workgroup sums
 
 // levels a.L0 .. of an LU factorization in one workgroup: n <= 16, nx, nr <= 8;

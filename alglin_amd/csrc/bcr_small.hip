@@ -166,8 +166,8 @@ int nmax_of(int n) { return n <= 4 ? 4 : n <= 8 ? 8 : 16; }
 
 }  // namespace
 
-// Rounds of one workgroup that a level may take: a further round of pairs
-// costs about what a launch of its own does.
+// Rounds of one workgroup that a level of the factorization may take: a further
+// round of pairs costs about what a launch of its own does.
 constexpr int kRounds = 2;
 
 // The round is that of the configuration the launch takes, which grows with the
@@ -179,9 +179,15 @@ int small_factor_level(int N, int n, int nx, int nr, size_t elem, bool first_ok)
   return first_level(N, kRounds * factor_waves(nm, elem) * (kWave / (2 * nm)), first_ok ? 1 : 2);
 }
 
-int small_solve_level(int N, int n) {
-  const int nm = nmax_of(n);
-  return first_level(N, kRounds * solve_waves(nm) * (kWave / (2 * nm)), 1);
+// A level of the sweeps: one round, its waves already fill the CU; half of one
+// where the border sums of a pair are many, two where a pair has little work in
+// FP32.  FP64, N = 1000, against two rounds and against a launch per level: n = 8,
+// 1 column 90, 97, 126 us; nr = 16, 4 columns 256, 333, 284; n = 16, 1 column 133,
+// 142, 164; n = 2, nr = 16, 4 columns 199, 257, 218.  FP32, n = 2, nr = 2, 1 column,
+// N = 1000, factor and solve: two rounds 117, one 122.
+int small_solve_level(int N, int n, int nr, int nrhs, size_t elem) {
+  const int nm = nmax_of(n), round = solve_waves(nm) * (kWave / (2 * nm)), sums = nr * nrhs;
+  return first_level(N, sums >= 32 ? round / 2 : nm == 4 && elem == 4 && sums <= 4 ? 2 * round : round, 1);
 }
 
 template <typename TA, typename TW>
