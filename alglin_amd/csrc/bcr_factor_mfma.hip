@@ -1185,9 +1185,10 @@ void launch_pair_batched(BatchTable<FactorArgs<TS, TW>> const& t, int nblocks, h
     hipLaunchKernelGGL((pair_lu_tw_batched<TS, TW, NB, RS>), pairs, dim3(64 * NB), 0, st, t);
   else
     hipLaunchKernelGGL((pair_lu_t_batched<TS, TW, NB, RS, kNrB>), pairs, dim3(64), 0, st, t);
-  // (four waves may wait here for room behind the other stream's workgroups;
-  // the calls are level with two: batches of 1024 uneven systems FP64 43.9 /
-  // 43.5 ms, FP32 32.8 / 32.5, half of them nearly singular 42.3 / 42.6)
+  // (four waves may wait here for room behind the other stream's workgroups,
+  // but large batches are level with two: 1024 uneven systems FP64 44.0 / 43.8 ms,
+  // FP32 32.6 / 32.8, half of them nearly singular 42.5 / 42.5; and one to eight
+  // systems of n > 32 take 5-7 % less: 8 of n = 49 .. 64 1.65 / 1.77 ms)
   if (nblocks <= kFewPairs) hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWavesFew>), pairs, dim3(64 * kRhsWavesFew), 0, st, t);
   else hipLaunchKernelGGL((pair_rhs_mfma_batched<TS, TW, NB, NRT, kRhsWaves>), pairs, dim3(64 * kRhsWaves), 0, st, t);
 }
