@@ -8,7 +8,10 @@ counted by n alone it took 1.6 times as long.
 Solve: a level takes one round of the workgroup, and less with many border sums
 per pair: four columns with a border of 16 against one column with a border of 2
 take 3.3 times as long at n = 8, 3.9 at n = 2 and 4; with two rounds for either
-3.9 and 4.6 to 4.8, slower than a launch per level."""
+3.9 and 4.6 to 4.8, slower than a launch per level.
+
+Another load on the machine can spoil a timing, so the best of three counts; the
+ratios above are far enough apart for that."""
 import time
 
 import numpy as np
@@ -35,9 +38,12 @@ def median_time(n, N, r):
 
 @pytest.mark.parametrize("N", [600, 1000])
 def test_level_rule_counts_the_border(N):
-    a, b = median_time(4, N, 8), median_time(5, N, 8)
-    print(f"case N={N}: n = 4 {1e6 * a:.0f} us, n = 5 {1e6 * b:.0f} us", flush=True)
-    assert a <= 1.15 * b
+    ratio = []
+    while len(ratio) < 3 and not (ratio and min(ratio) <= 1.15):
+        a, b = median_time(4, N, 8), median_time(5, N, 8)
+        print(f"case N={N}: n = 4 {1e6 * a:.0f} us, n = 5 {1e6 * b:.0f} us", flush=True)
+        ratio.append(a / b)
+    assert min(ratio) <= 1.15
 
 
 def solve_time(n, N, r, m):
@@ -61,6 +67,9 @@ def solve_time(n, N, r, m):
 
 @pytest.mark.parametrize("n,N,times", [(8, 1000, 3.6), (8, 4000, 3.6), (4, 1000, 4.35), (2, 1000, 4.35)])
 def test_solve_level_rule_counts_the_work(n, N, times):
-    a, b = solve_time(n, N, 2, 1), solve_time(n, N, 16, 4)
-    print(f"case n={n} N={N}: 1 column {1e6 * a:.0f} us, border of 16 and 4 columns {1e6 * b:.0f} us", flush=True)
-    assert b <= times * a
+    ratio = []
+    while len(ratio) < 3 and not (ratio and min(ratio) <= times):
+        a, b = solve_time(n, N, 2, 1), solve_time(n, N, 16, 4)
+        print(f"case n={n} N={N}: 1 column {1e6 * a:.0f} us, border of 16 and 4 columns {1e6 * b:.0f} us", flush=True)
+        ratio.append(b / a)
+    assert min(ratio) <= times
