@@ -17,9 +17,9 @@
 //     FP64 the trailing blocks take a block's 16 steps at once on the matrix
 //     cores (trailing_update); in FP32 each step updates them (a lane read
 //     and two FMAs per column: the way through LDS costs as much).  The
-//     steps' chain at two waves per SIMD bounds it, VALU issue next (57 %
+//     steps' chain at two waves per SIMD bounds it, VALU issue next (55 %
 //     busy): N = 100000, n = 32 FP64, first level 909 -> 750 us with the
-//     blocked update, 711 now (loads and stores alone are 0.4 ms).  Rows do
+//     blocked update, 713 now (loads and stores alone are 0.4 ms).  Rows do
 //     not move; each row is stored at its final position (T, C_j U^-1, perm),
 //     and the positions themselves go to the unused tail of T (one byte per
 //     row).  pair_lu_tw: the same by a wave per block, FP64 beyond n = 48 and
