@@ -182,10 +182,10 @@ __device__ __forceinline__ void forward_qr_stream_body(SolveArgs<TW, TX> const& 
       }
     }
     for (int i = 0; i < nr; ++i) {
-      const TX c = keep_if(TX(gload(Cj, unsigned(i) + unsigned(lane < n ? lane : 0) * unsigned(nr))), lane < n);
+      const TX c = TX(gload(Cj, unsigned(i) + unsigned(lane < n ? lane : 0) * unsigned(nr)));
 #pragma unroll
       for (int b = 0; b < QB; ++b) {
-        const TX s = wave::sum(c * (lane < n ? x0[b] : TX(0)));
+        const TX s = wave::sum(lane < n ? c * x0[b] : TX(0));   // (the product rounded before the sum)
         if (lane == 0 && q0 + b < nrhs) a.Xpart[size_t(j) * nr * nrhs + i + size_t(q0 + b) * nr] = -s;
       }
     }
