@@ -51,6 +51,9 @@ def test_many_columns_of_a_small_block():
             t.append(time.perf_counter() - t0)
         return np.median(t[5:])
 
-    a, b = median(4), median(64)
-    print(f"case 4 columns {1e6 * a:.0f} us, 64 columns {1e6 * b:.0f} us", flush=True)
-    assert b <= 5 * a
+    ratio = []
+    while len(ratio) < 3 and not (ratio and min(ratio) <= 5):   # another load can spoil a timing
+        a, b = median(4), median(64)
+        print(f"case 4 columns {1e6 * a:.0f} us, 64 columns {1e6 * b:.0f} us", flush=True)
+        ratio.append(b / a)
+    assert min(ratio) <= 5
